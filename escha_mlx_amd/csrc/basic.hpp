@@ -260,12 +260,17 @@ __global__ __launch_bounds__(64) void k_route_topk(const float* __restrict__ log
 // Shared memory holds per-expert counts; E <= 4096.
 // The body runs in one block of 1024 threads (k_build_groups, or block 0 of
 // k_moe_prep).
-// Fast form when E * ceil(m / 64) <= kGroupMaskWords: a bit per (expert,
-// row) in LDS.  A row's rank within its expert is the popcount of its
-// expert's bits below it, an expert's count the popcount of all of them, so
-// every slot is written once (no clearing pass, no ordering between writers)
-// and the only serial step is the prefix over the experts' padded counts.
+// Few rows (E * ceil(m / 64) <= kGroupMaskWords): a bit per (expert, row) in
+// LDS; a row's rank within its expert is the popcount of its expert's bits
+// below it, so every slot is written once and the only serial step is the
+// prefix over the experts' padded counts.  Many rows: each of the 16 waves
+// owns a contiguous segment and counts per expert (16 E counters, in the
+// mask's LDS: E <= kGroupHistE), the prefix gives each (wave, expert) its first
+// slot, and the waves place their segments with no barrier between them
+// (16,384 rows of 256 experts; ranking each row by a scan of its chunk's earlier
+// rows took 264 us there).  Many rows of more experts: the mask form in chunks.
 constexpr int kGroupMaskWords = 4096;
+constexpr int kGroupHistE = kGroupMaskWords * 8 / (16 * 4);  // 512
 
 // exclusive prefix over the block (1024 threads) of one int per thread; the
 // block's total in *total
@@ -291,9 +296,8 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* s_wsum, int* tot
 __device__ void build_groups_mask(const int* __restrict__ row_expert, int m, int E, int R,
                                   int n_groups, int* __restrict__ rows_idx,
                                   int* __restrict__ group_expert, int* s_start,
+                                  unsigned long long* s_mask, int* s_wsum,
                                   int* __restrict__ n_active) {
-  __shared__ unsigned long long s_mask[kGroupMaskWords];  // [E][nw]
-  __shared__ int s_wsum[16];
   const int tid = threadIdx.x, nt = blockDim.x;
   const int nw = (m + 63) >> 6;
   for (int i = tid; i < E * nw; i += nt) s_mask[i] = 0ull;
@@ -340,74 +344,137 @@ __device__ void build_groups_mask(const int* __restrict__ row_expert, int m, int
   }
 }
 
+// The segment form (E <= kGroupHistE): s_hist[wave][E] holds the wave's rows
+// per expert, then the slot of its next row of that expert.
+__device__ void build_groups_hist(const int* __restrict__ row_expert, int m, int E, int R,
+                                  int n_groups, int* __restrict__ rows_idx,
+                                  int* __restrict__ group_expert, int* s_hist, int* s_wsum,
+                                  int* __restrict__ n_active) {
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  for (int i = tid; i < 16 * E; i += nt) s_hist[i] = 0;
+  __syncthreads();
+  const int seg = ((m + 15) / 16 + 63) / 64 * 64;
+  const int r0 = wave * seg, r1 = min(m, r0 + seg);
+  int* hist = s_hist + wave * E;
+  for (int r = r0 + lane; r < r1; r += 64) atomicAdd(&hist[row_expert[r]], 1);
+  __syncthreads();
+  // expert tid: its padded count, first slot, groups and padding slots (= m),
+  // and each wave's first slot
+  int cnt = 0;
+  if (tid < E)
+    for (int w = 0; w < 16; ++w) cnt += s_hist[w * E + tid];
+  const int pad = (cnt + R - 1) / R * R;
+  int total;
+  const int start = block_exclusive_scan(pad, s_wsum, &total);
+  if (tid < E) {
+    int slot = start;
+    for (int w = 0; w < 16; ++w) {
+      const int k = s_hist[w * E + tid];
+      s_hist[w * E + tid] = slot;
+      slot += k;
+    }
+    for (int g = start / R; g < (start + pad) / R; ++g) group_expert[g] = tid;
+    for (int i = cnt; i < pad; ++i) rows_idx[start + i] = m;
+  }
+  if (n_active && tid == 0) *n_active = total / R;
+  for (int i = total + tid; i < n_groups * R; i += nt) rows_idx[i] = m;
+  for (int g = total / R + tid; g < n_groups; g += nt) group_expert[g] = -1;
+  __syncthreads();
+  // 64 rows at a time: a row's rank among them is the number of lower lanes
+  // with the same expert, found bit by bit
+  int e_next = r0 + lane < r1 ? row_expert[r0 + lane] : 0;
+  for (int r = r0; r < r1; r += 64) {
+    const int e = e_next;
+    const bool ok = r + lane < r1;
+    if (r + 64 + lane < r1) e_next = row_expert[r + 64 + lane];
+    unsigned long long same = __ballot(ok);
+#pragma unroll
+    for (int b = 0; b < 9; ++b) {
+      const unsigned long long bit = __ballot((e >> b) & 1);
+      same &= (e >> b) & 1 ? bit : ~bit;
+    }
+    const int rank = __popcll(same & ((1ull << lane) - 1ull)), n = __popcll(same);
+    if (ok) {
+      const int slot = hist[e];
+      rows_idx[slot + rank] = r + lane;
+      if (rank == n - 1) hist[e] = slot + n;
+    }
+    // the slots just written are read by the next 64 rows
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+}
+
 // n_active (when not null): the number of groups that hold rows.
 __device__ void build_groups_block(const int* __restrict__ row_expert, int m, int E, int R,
                                    int n_groups, int* __restrict__ rows_idx,
                                    int* __restrict__ group_expert,
                                    int* __restrict__ n_active = nullptr) {
-  __shared__ int s_start[4096];  // first padded slot of each expert
+  // first padded slot of each expert (chunked form: plus its rows placed so far)
+  __shared__ int s_start[4096];
+  __shared__ unsigned long long s_mask[kGroupMaskWords];  // [E][nw]
+  __shared__ int s_wsum[16];
   if ((long)E * ((m + 63) >> 6) <= kGroupMaskWords) {
-    build_groups_mask(row_expert, m, E, R, n_groups, rows_idx, group_expert, s_start, n_active);
+    build_groups_mask(row_expert, m, E, R, n_groups, rows_idx, group_expert, s_start, s_mask,
+                      s_wsum, n_active);
     return;
   }
-  __shared__ int s_cnt[4096];    // rows per expert, then rows placed so far
-  __shared__ int s_e[1024];      // one chunk of row_expert
+  if (E <= kGroupHistE) {
+    build_groups_hist(row_expert, m, E, R, n_groups, rows_idx, group_expert,
+                      reinterpret_cast<int*>(s_mask), s_wsum, n_active);
+    return;
+  }
   const int tid = threadIdx.x, nt = blockDim.x;
-  for (int e = tid; e < E; e += nt) s_cnt[e] = 0;
-  for (int i = tid; i < n_groups * R; i += nt) rows_idx[i] = m;
-  for (int g = tid; g < n_groups; g += nt) group_expert[g] = -1;
+  const int nw = kGroupMaskWords / E;  // mask words per expert, 64 rows each
+  for (int e = tid; e < E; e += nt) s_start[e] = 0;
+  for (int i = tid; i < E * nw; i += nt) s_mask[i] = 0ull;
   __syncthreads();
-  for (int r = tid; r < m; r += nt) atomicAdd(&s_cnt[row_expert[r]], 1);
+  for (int r = tid; r < m; r += nt) atomicAdd(&s_start[row_expert[r]], 1);
   __syncthreads();
-  // exclusive prefix of the padded counts: each thread sums 4 experts, then a
-  // block-wide scan of the 1024 partial sums (Hillis-Steele in LDS)
-  {
-    int loc[4], sum = 0;
+  // experts 4 tid .. 4 tid + 3: padded counts, first slots, their groups and
+  // their padding slots (= m)
+  int cnt[4], sum = 0;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = 4 * tid + j;
-      loc[j] = e < E ? (s_cnt[e] + R - 1) / R * R : 0;
-      sum += loc[j];
-    }
-    s_e[tid] = sum;
-    __syncthreads();
-    for (int off = 1; off < 1024; off <<= 1) {
-      const int v = tid >= off ? s_e[tid - off] : 0;
-      __syncthreads();
-      s_e[tid] += v;
-      __syncthreads();
-    }
-    int acc = s_e[tid] - sum;  // exclusive
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int e = 4 * tid + j;
-      if (e < E) s_start[e] = acc;
-      acc += loc[j];
-    }
+  for (int j = 0; j < 4; ++j) {
+    cnt[j] = 4 * tid + j < E ? s_start[4 * tid + j] : 0;
+    sum += (cnt[j] + R - 1) / R * R;
   }
-  __syncthreads();
-  // group_expert: every padded group of expert e
-  for (int e = tid; e < E; e += nt) {
-    const int ng = (s_cnt[e] + R - 1) / R;
-    for (int g = 0; g < ng; ++g) group_expert[s_start[e] / R + g] = e;
-    if (n_active && e == E - 1) *n_active = s_start[e] / R + ng;
-    s_cnt[e] = 0;
+  int total;
+  int start = block_exclusive_scan(sum, s_wsum, &total);
+  for (int j = 0; j < 4; ++j) {
+    const int e = 4 * tid + j, pad = (cnt[j] + R - 1) / R * R;
+    if (e < E) {
+      s_start[e] = start;
+      for (int g = start / R; g < (start + pad) / R; ++g) group_expert[g] = e;
+      for (int i = cnt[j]; i < pad; ++i) rows_idx[start + i] = m;
+    }
+    start += pad;
   }
-  __syncthreads();
-  // stable placement, one chunk of nt rows at a time: a row's rank is the
-  // number of earlier rows of its expert (earlier chunks counted in s_cnt)
-  for (int c0 = 0; c0 < m; c0 += nt) {
-    const int r = c0 + tid;
-    const int e = r < m ? row_expert[r] : -1;
-    s_e[tid] = e;
+  if (n_active && tid == 0) *n_active = total / R;
+  for (int i = total + tid; i < n_groups * R; i += nt) rows_idx[i] = m;
+  for (int g = total / R + tid; g < n_groups; g += nt) group_expert[g] = -1;
+  // stable placement, one chunk of rows at a time
+  for (int c0 = 0; c0 < m; c0 += 64 * nw) {
+    const int n = min(64 * nw, m - c0);
+    for (int r = tid; r < n; r += nt)
+      atomicOr(&s_mask[row_expert[c0 + r] * nw + (r >> 6)], 1ull << (r & 63));
     __syncthreads();
-    if (r < m) {
-      int rank = s_cnt[e];
-      for (int q = 0; q < tid; ++q) rank += (s_e[q] == e);
-      rows_idx[s_start[e] + rank] = r;
+    for (int r = tid; r < n; r += nt) {
+      const int e = row_expert[c0 + r], w0 = r >> 6;
+      const unsigned long long* me = s_mask + e * nw;
+      int rank = __popcll(me[w0] & ((1ull << (r & 63)) - 1ull));
+      for (int w = 0; w < w0; ++w) rank += __popcll(me[w]);
+      rows_idx[s_start[e] + rank] = c0 + r;
     }
     __syncthreads();
-    if (r < m) atomicAdd(&s_cnt[e], 1);
+    for (int e = tid; e < E; e += nt) {
+      int k = 0;
+      for (int w = 0; w < nw; ++w) {
+        k += __popcll(s_mask[e * nw + w]);
+        s_mask[e * nw + w] = 0ull;
+      }
+      s_start[e] += k;
+    }
     __syncthreads();
   }
 }

@@ -20,6 +20,7 @@
 #include "probe.hpp"
 #include "layers.hpp"
 #include "proj.hpp"
+#include "grouped.hpp"
 
 namespace {
 
@@ -483,6 +484,20 @@ int mma2_row_blocks(int M, int TN) {
     }
   }
   return best;
+}
+
+// k_combine, 8 columns per thread where the rows allow 16-byte accesses.
+int combine_rows(const uint16_t* d16, const float* scores, int T, int top_k, int H, uint16_t* y,
+                 hipStream_t s) {
+  const bool wide = H % 8 == 0 && (reinterpret_cast<uintptr_t>(d16) |
+                                   reinterpret_cast<uintptr_t>(y)) % 16 == 0;
+  const int cols = wide ? 8 : 1;
+  const dim3 grid((H / cols + 255) / 256, T);
+  if (wide)
+    hipLaunchKernelGGL(esc::k_combine<8>, grid, dim3(256), 0, s, d16, scores, top_k, H, y);
+  else
+    hipLaunchKernelGGL(esc::k_combine<1>, grid, dim3(256), 0, s, d16, scores, top_k, H, y);
+  return launched("k_combine");
 }
 
 // k_gemm_mma2 launch (TN % 16 == 0); OUT: output transform fused, y written.
@@ -986,9 +1001,7 @@ int esc_moe_combine(const uint16_t* d16, const float* scores, int T, int top_k, 
   ESC_REQUIRE(d16 && scores && y, "null pointer");
   ESC_REQUIRE(T >= 0 && top_k >= 1 && H > 0, "bad T=%d / top_k=%d / H=%d", T, top_k, H);
   if (T == 0) return ESC_OK;
-  hipLaunchKernelGGL(esc::k_combine, dim3((H + 255) / 256, T), dim3(256), 0, S(stream), d16,
-                     scores, top_k, H, y);
-  return launched("k_combine");
+  return combine_rows(d16, scores, T, top_k, H, y, S(stream));
 }
 
 // ---- dense int8 / f16 GEMV (q8.hpp): shared expert, gates, vocabulary head
@@ -1173,9 +1186,43 @@ int moe_input(const uint16_t* x, const int32_t* ids, int top_k, const float* rin
   return launched("k_moe_input");
 }
 
+// Row blocks of 16 per group of the grouped matrix-core GEMM (k_moe_mma), 0:
+// the split-K chain.  Measured on MI355X (256 experts, hidden 2048, intermediate
+// 512, top-8; whole call, the split-K chain by hash / by table in brackets): 4
+// rows per expert 184 us (165 / -), 8 rows 186 (246 / 211), 16 rows 208 (394 /
+// 349), 64 rows 357 (1200 / -).  So from 8 rows per expert, at the row-block
+// size with the least work: a group costs 0.43 + 0.071 NRB (208, 263, 292 and
+// 337 us with one group of 2, 4, 6 and 8 row blocks per expert), and an expert
+// with Poisson(M / E) rows takes sum over j of P(rows > 16 NRB j) groups.
+constexpr int kMoeMmaRowsPerExpert = 8;
+int moe_mma_nrb(int M, int E, int H, int I) {
+  if (E > 4096 || M / E < kMoeMmaRowsPerExpert) return 0;
+  // 32-bit byte offsets into the transformed rows
+  if ((size_t)M * std::max(H, I) * 2 > 0xFFFFFFF0u) return 0;
+  const double lam = (double)M / E, dev = std::sqrt(2.0 * lam);
+  int best = 8;
+  double best_cost = 1e30;
+  for (int nrb = 8; nrb >= 2; nrb -= 2) {
+    const int br = 16 * nrb;
+    // the j whose P is 1 to within rounding, then the others (normal tail)
+    int j = std::max(0, (int)((lam - 6 * std::sqrt(lam)) / br));
+    double groups = j;
+    for (double p = 1.0; p > 1e-4; ++j) {
+      p = 0.5 * std::erfc((j * br + 0.5 - lam) / dev);
+      groups += p;
+    }
+    const double cost = groups * (0.43 + 0.071 * nrb);
+    if (cost < best_cost * 0.999) {
+      best_cost = cost;
+      best = nrb;
+    }
+  }
+  return best;
+}
+
 struct MoePlan {
-  int M, S1, S2, R, n_groups;
-  size_t off_xh, off_p1, off_xh2, off_p2, off_rows, off_gexp, off_nact, total;
+  int M, S1, S2, R, n_groups, nrb;
+  size_t off_xh, off_p1, off_xh2, off_p2, off_rows, off_gexp, off_nact, off_d16, total;
 };
 // base: bytes at the start of the workspace left to the caller (the
 // no-allocation variant keeps its counters there).
@@ -1201,7 +1248,22 @@ MoePlan moe_plan(int T, int top_k, int E, int H, int I, int K_gu, int K_dn, size
   p.off_rows = al(p.off_p2 + (size_t)p.S2 * p.M * H * 4);
   p.off_gexp = al(p.off_rows + (size_t)p.n_groups * p.R * 4);
   p.off_nact = al(p.off_gexp + (size_t)p.n_groups * 4);
+  p.off_d16 = 0;
   p.total = al(p.off_nact + 4);
+  p.nrb = moe_mma_nrb(p.M, E, H, I);
+  if (p.nrb) {
+    // the grouped GEMM's buffers in the same bytes (fewer: f16 rows in place of
+    // the float32 partials), so what a workspace of this size holds, and which
+    // shapes a fixed scratch takes, does not depend on the path
+    p.R = 16 * p.nrb;
+    p.n_groups = (int)(((long)p.M + (long)E * (p.R - 1) + p.R - 1) / p.R);
+    p.off_xh2 = al(p.off_xh + (size_t)p.M * H * 2);
+    p.off_d16 = al(p.off_xh2 + (size_t)p.M * I * 2);
+    p.off_rows = al(p.off_d16 + (size_t)p.M * H * 2);
+    p.off_gexp = al(p.off_rows + (size_t)p.n_groups * p.R * 4);
+    p.off_nact = al(p.off_gexp + (size_t)p.n_groups * 4);
+    p.total = std::max(p.total, al(p.off_nact + 4));
+  }
   return p;
 }
 
@@ -1250,6 +1312,41 @@ int group_rows(int K, int lut, int R, const uint16_t* xh, const uint32_t* code, 
   }
   return K == 2 ? GroupRowsF<2, false>::run(R, xh, code, rows, gexp, n_groups, M, TK, TN, S, part, s)
                 : GroupRowsF<3, false>::run(R, xh, code, rows, gexp, n_groups, M, TK, TN, S, part, s);
+}
+
+template <int K, bool GU>
+int moe_mma_k(int nrb, const esc::MoeMmaArgs& a, hipStream_t s) {
+  const dim3 grid((unsigned)(8 * ((a.n_groups + 7) / 8) * a.ncb)), blk(256);
+  switch (nrb) {
+    case 2: hipLaunchKernelGGL((esc::k_moe_mma<K, 2, GU>), grid, blk, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((esc::k_moe_mma<K, 4, GU>), grid, blk, 0, s, a); break;
+    case 6: hipLaunchKernelGGL((esc::k_moe_mma<K, 6, GU>), grid, blk, 0, s, a); break;
+    case 8: hipLaunchKernelGGL((esc::k_moe_mma<K, 8, GU>), grid, blk, 0, s, a); break;
+    default: return fail(ESC_EINVAL, "internal: %d row blocks", nrb);
+  }
+  return launched("k_moe_mma");
+}
+
+template <bool GU>
+int moe_mma(int K, int nrb, const esc::MoeMmaArgs& a, hipStream_t s) {
+  return K == 2 ? moe_mma_k<2, GU>(nrb, a, s) : moe_mma_k<3, GU>(nrb, a, s);
+}
+
+// k_moe_prep: the input transform of every routed row and the grouping.
+int moe_prep(const uint16_t* x, const int32_t* ids, int T, int top_k, const float* rin, int H,
+             float rs, uint16_t* xh, const MoePlan& p, int E, int* rows, int* gexp, int* nact,
+             hipStream_t s) {
+  // four slots per wave once that leaves eight waves per SIMD
+  const bool four = (long)T * top_k * (H / 128) / 4 >= 32L * device_cus();
+  const long waves = (long)(H / 128) * T * (four ? (top_k + 3) / 4 : top_k);
+  const dim3 grid((unsigned)(1 + (waves + 15) / 16)), blk(1024);
+  if (four)
+    hipLaunchKernelGGL(esc::k_moe_prep<4>, grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh, p.M, E,
+                       p.R, p.n_groups, rows, gexp, nact);
+  else
+    hipLaunchKernelGGL(esc::k_moe_prep<1>, grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh, p.M, E,
+                       p.R, p.n_groups, rows, gexp, nact);
+  return launched("k_moe_prep");
 }
 
 // One-launch path (fused.hpp).  Latency mode: small items over the whole GPU
@@ -1628,10 +1725,17 @@ int moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scores, 
   int* nact = reinterpret_cast<int*>(w + p.off_nact);
   if (p.R) {
     // input transform and expert grouping in one launch
-    const int waves = H / 128 * p.M;
-    hipLaunchKernelGGL(esc::k_moe_prep, dim3(1 + (waves + 15) / 16), dim3(1024), 0, s, x, ids,
-                       top_k, gu_rin, H, rs, xh, p.M, E, p.R, p.n_groups, rows, gexp, nact);
-    if (int rc = launched("k_moe_prep")) return rc;
+    if (int rc = moe_prep(x, ids, T, top_k, gu_rin, H, rs, xh, p, E, rows, gexp, nact, s)) return rc;
+    if (p.nrb) {
+      uint16_t* d16 = reinterpret_cast<uint16_t*>(w + p.off_d16);
+      esc::MoeMmaArgs a{xh, gu_code, rows, gexp, gu_rout, dn_rin, xh2, p.M, H / 16, 2 * I / 16,
+                        p.n_groups, I / 128, rs};
+      if (int rc = moe_mma<true>(K_gu, p.nrb, a, s)) return rc;
+      a = {xh2, dn_code, rows, gexp, dn_rout, nullptr, d16, p.M, I / 16, H / 16, p.n_groups,
+           (H + 255) / 256, rs};
+      if (int rc = moe_mma<false>(K_dn, p.nrb, a, s)) return rc;
+      return combine_rows(d16, scores, T, top_k, H, y, s);
+    }
     if (int rc = group_rows(K_gu, use_lut, p.R, xh, gu_code, rows, gexp, nact, p.n_groups, p.M,
                             H / 16, 2 * I / 16, p.S1, p1, s))
       return rc;

@@ -302,57 +302,44 @@ __global__ __launch_bounds__(kMmaThreads, 2) void k_gemm_mfma(const uint16_t* __
 // The kernel is decode-bound: the host picks NRB for the shape.
 // D register r of lane l: output column of tile-lane 4(l/16) + r, row l%16 of
 // the row block.
-// OUT: the output transform is fused into the epilogue (y f16 = (bias +)
-// f16((H128(row) * rs) * rout), the formula of k_output_transform): per 16-row
-// block the two waves of each 128-column block exchange their 64 columns
-// through LDS and each transforms 8 rows; mid is not written.
-template <int K, int NRB, bool OUT = false>
-__global__ __launch_bounds__(256, 2) void k_gemm_mma2(
-    const uint16_t* __restrict__ xh, const uint32_t* __restrict__ code, int M, int TK, int TN,
-    float* __restrict__ mid, const float* __restrict__ rout = nullptr,
-    const uint16_t* __restrict__ bias = nullptr, float rs = 0.f, uint16_t* __restrict__ y = nullptr) {
+template <int K, int NRB>
+struct Mma2 {
   using G = Geo<K>;
-  constexpr int TPS = 16 / G::LPT, GPW = 4 / TPS, NA = GPW * G::NCOL;
+  static constexpr int TPS = 16 / G::LPT, GPW = 4 / TPS, NA = GPW * G::NCOL;
   static_assert(NA == 4, "four 16-column groups per wave");
   static_assert(NRB % 2 == 0 && NRB >= 2 && NRB <= 8, "whole x chunks per thread, 2 waves/SIMD");
-  constexpr int BR = 16 * NRB;            // rows per block
-  constexpr int XCH = BR * 8 / 256;       // 16-byte x chunks per thread per stage
-  __shared__ uint4 s_x[2][BR * 8];        // [stage][row][chunk ^ (row & 7)]
+  static constexpr int BR = 16 * NRB;            // rows per block
+  static constexpr int XCH = BR * 8 / 256;       // 16-byte x chunks per thread per stage
+};
 
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int IC = TK * 16, OC = TN * 16;
-  const int ncb = TN / 16;
-  int rb, cb;
-  if (ncb % 8 == 0) {
-    const int per = ncb / 8, qq = blockIdx.x / 8, x = blockIdx.x % 8;
-    rb = qq / per;
-    cb = 8 * (qq % per) + x;
-  } else {
-    rb = blockIdx.x / ncb;
-    cb = blockIdx.x % ncb;
-  }
-  const int row0 = rb * BR;
-  const int tile0 = cb * 16 + 4 * wave;
-  const int gk = lane >> 4, c = lane & 15, tc = c / G::LPT, q = lane % G::LPT;
+// Byte offset of the workgroup's x chunk j of thread tid from the start of
+// its row: chunk e = tid + 256j of a stage is row e/8, logical chunk
+// (e%8)^(row&7) = kt (lc/2) half (lc%2), 128 bytes per row per stage.
+__device__ __forceinline__ int mma2_x_row(int tid, int j) { return (tid + 256 * j) >> 3; }
+__device__ __forceinline__ uint32_t mma2_x_chunk(int tid, int j) {
+  const int e = tid + 256 * j;
+  return 16u * ((e & 7) ^ ((e >> 3) & 7));
+}
+
+// The main loop over steps [s0, s1) (s1 > s0): acc[a][r] += the wave's 64
+// columns x row block r.  cbase: the lane's code words of the wave's first
+// tile at kt gk (lane / 16); xoff: byte offsets of the thread's x chunks.
+template <int K, int NRB>
+__device__ __forceinline__ void mma2_loop(const uint32_t* __restrict__ cbase, size_t kstride,
+                                          __amdgpu_buffer_rsrc_t xrs, const uint32_t* xoff, int s0,
+                                          int s1, uint4 (*s_x)[16 * NRB * 8],
+                                          f32x4_t (*acc)[NRB]) {
+  using G = Geo<K>;
+  using D = Mma2<K, NRB>;
+  constexpr int TPS = D::TPS, GPW = D::GPW, NA = D::NA, XCH = D::XCH;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int gk = lane >> 4, c = lane & 15;
   const int src = (lane & ~(G::LPT - 1)) | ((lane + G::LPT - 1) & (G::LPT - 1));
-
-  // code: tile group tg of the wave, lane's kt = 4s + gk
-  const size_t kstride = (size_t)TN * (8 * K);
-  const uint32_t* cbase = code + (size_t)(tile0 + tc) * (8 * K) + q * G::WPL + gk * kstride;
   auto load_code = [&](LaneWords<K>* cw, int s) {
 #pragma unroll
     for (int tg = 0; tg < GPW; ++tg)
       cw[tg] = load_lane_words<K>(cbase + (size_t)tg * TPS * (8 * K) + (size_t)(4 * s) * kstride);
   };
-  // x: chunk e = tid + 256j of a stage is row e/8, logical chunk (e%8)^(row&7)
-  // = kt (lc/2) half (lc%2), 128 bytes per row per stage
-  uint32_t xoff[XCH];
-#pragma unroll
-  for (int j = 0; j < XCH; ++j) {
-    const int e = tid + 256 * j, r = e >> 3, lc = (e & 7) ^ (r & 7);
-    xoff[j] = 2u * ((uint32_t)min(row0 + r, M - 1) * IC) + 16u * lc;
-  }
-  const __amdgpu_buffer_rsrc_t xrs = buf_rsrc(xh, (size_t)M * IC * 2);
   auto load_x = [&](uint4* xr, int s) {
 #pragma unroll
     for (int j = 0; j < XCH; ++j) {
@@ -364,8 +351,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mma2(
 #pragma unroll
     for (int j = 0; j < XCH; ++j) s_x[buf][tid + 256 * j] = xr[j];
   };
-
-  f32x4_t acc[NA][NRB];
 #pragma unroll
   for (int a = 0; a < NA; ++a)
 #pragma unroll
@@ -374,7 +359,6 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mma2(
   // software pipeline: the MFMAs of step s and the decode of step s+1 sit in
   // one straight-line body (the matrix pipe and the VALU overlap); loads past
   // the last step re-read it (in bounds, never used)
-  const int NS = TK / 4;
   auto decode_step = [&](const LaneWords<K>* w, u32x4_t (*Ad)[2]) {
 #pragma unroll
     for (int tg = 0; tg < GPW; ++tg) {
@@ -388,17 +372,17 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mma2(
   LaneWords<K> cw[GPW];
   uint4 xr[XCH];
   u32x4_t A[NA][2];
-  load_code(cw, 0);
-  load_x(xr, 0);
+  load_code(cw, s0);
+  load_x(xr, s0);
   store_x(xr, 0);
   decode_step(cw, A);
-  load_code(cw, min(1, NS - 1));
+  load_code(cw, min(s0 + 1, s1 - 1));
   lds_barrier();
-  for (int s = 0; s < NS; ++s) {
-    const int buf = s & 1;
-    load_x(xr, min(s + 1, NS - 1));
+  for (int s = s0; s < s1; ++s) {
+    const int buf = (s - s0) & 1;
+    load_x(xr, min(s + 1, s1 - 1));
     LaneWords<K> cn[GPW];
-    load_code(cn, min(s + 2, NS - 1));
+    load_code(cn, min(s + 2, s1 - 1));
     u32x4_t An[NA][2];
 #pragma unroll
     for (int P = 0; P < 2; ++P)
@@ -420,6 +404,67 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mma2(
     for (int tg = 0; tg < GPW; ++tg) cw[tg] = cn[tg];
     lds_barrier();
   }
+}
+
+// A wave's 64 columns of one 16-row block into LDS (sp: the rows' first
+// column of the wave; pitch floats between rows).
+template <int K, int NRB>
+__device__ __forceinline__ void mma2_to_lds(const f32x4_t (*acc)[NRB], int r, float* sp,
+                                            int pitch) {
+  using G = Geo<K>;
+  using D = Mma2<K, NRB>;
+  const int lane = threadIdx.x & 63, gk = lane >> 4, c = lane & 15;
+#pragma unroll
+  for (int tg = 0; tg < D::GPW; ++tg)
+#pragma unroll
+    for (int ci = 0; ci < G::NCOL; ++ci)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        const int i = 4 * gk + rr, tc = i / G::LPT, q = i % G::LPT;
+        sp[c * pitch + 16 * (D::TPS * tg + tc) + G::col(q, ci)] = acc[tg * G::NCOL + ci][r][rr];
+      }
+}
+
+// OUT: the output transform is fused into the epilogue (y f16 = (bias +)
+// f16((H128(row) * rs) * rout), the formula of k_output_transform): per 16-row
+// block the two waves of each 128-column block exchange their 64 columns
+// through LDS and each transforms 8 rows; mid is not written.
+template <int K, int NRB, bool OUT = false>
+__global__ __launch_bounds__(256, 2) void k_gemm_mma2(
+    const uint16_t* __restrict__ xh, const uint32_t* __restrict__ code, int M, int TK, int TN,
+    float* __restrict__ mid, const float* __restrict__ rout = nullptr,
+    const uint16_t* __restrict__ bias = nullptr, float rs = 0.f, uint16_t* __restrict__ y = nullptr) {
+  using G = Geo<K>;
+  using D = Mma2<K, NRB>;
+  constexpr int TPS = D::TPS, GPW = D::GPW, NA = D::NA, BR = D::BR, XCH = D::XCH;
+  __shared__ uint4 s_x[2][BR * 8];        // [stage][row][chunk ^ (row & 7)]
+
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+  const int IC = TK * 16, OC = TN * 16;
+  const int ncb = TN / 16;
+  int rb, cb;
+  if (ncb % 8 == 0) {
+    const int per = ncb / 8, qq = blockIdx.x / 8, x = blockIdx.x % 8;
+    rb = qq / per;
+    cb = 8 * (qq % per) + x;
+  } else {
+    rb = blockIdx.x / ncb;
+    cb = blockIdx.x % ncb;
+  }
+  const int row0 = rb * BR;
+  const int tile0 = cb * 16 + 4 * wave;
+  const int gk = lane >> 4, c = lane & 15, tc = c / G::LPT, q = lane % G::LPT;
+
+  // code: tile group tg of the wave, lane's kt = 4s + gk
+  const size_t kstride = (size_t)TN * (8 * K);
+  const uint32_t* cbase = code + (size_t)(tile0 + tc) * (8 * K) + q * G::WPL + gk * kstride;
+  uint32_t xoff[XCH];
+#pragma unroll
+  for (int j = 0; j < XCH; ++j)
+    xoff[j] = 2u * ((uint32_t)min(row0 + mma2_x_row(tid, j), M - 1) * IC) + mma2_x_chunk(tid, j);
+  const __amdgpu_buffer_rsrc_t xrs = buf_rsrc(xh, (size_t)M * IC * 2);
+  f32x4_t acc[NA][NRB];
+  mma2_loop<K, NRB>(cbase, kstride, xrs, xoff, 0, TK / 4, s_x, acc);
 
   if constexpr (!OUT) {
 #pragma unroll
@@ -446,16 +491,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mma2(
 #pragma unroll
     for (int r = 0; r < NRB; ++r) {
       // this wave's 64 columns of rows 16r..16r+15 into the pair's LDS block
-#pragma unroll
-      for (int tg = 0; tg < GPW; ++tg)
-#pragma unroll
-        for (int ci = 0; ci < G::NCOL; ++ci)
-#pragma unroll
-          for (int rr = 0; rr < 4; ++rr) {
-            const int i = 4 * gk + rr, tc = i / G::LPT, q = i % G::LPT;
-            sp[c * kPitch + 64 * hw + 16 * (TPS * tg + tc) + G::col(q, ci)] =
-                acc[tg * G::NCOL + ci][r][rr];
-          }
+      mma2_to_lds<K, NRB>(acc, r, sp + 64 * hw, kPitch);
       __syncthreads();
 #pragma unroll 2
       for (int j = 0; j < 8; ++j) {

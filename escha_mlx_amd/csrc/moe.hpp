@@ -8,23 +8,31 @@
 
 namespace esc {
 
-// xh[row] = f16(H128(f32(x[row / k]) * rin[ids[row]]) * RS), 128-block blk
-// of one row, by one wave.
+// xh[row] = f16(H128(f32(x[tok]) * rin[ids[row]]) * RS), 128-block blk of the
+// rows row = tok * top_k + s of up to NS slots s from s0 of one token, by one
+// wave: the token's inputs are read once, every slot's scales are requested
+// before any is used (slots past the last re-read it and store nothing).
+template <int NS>
 __device__ __forceinline__ void moe_input_wave(const uint16_t* __restrict__ x,
                                                const int* __restrict__ ids, int top_k,
                                                const float* __restrict__ rin, int H, float rs,
-                                               uint16_t* __restrict__ xh, int blk, int row) {
+                                               uint16_t* __restrict__ xh, int blk, int tok,
+                                               int s0) {
   const int lane = threadIdx.x & 63;
-  const int tok = row / top_k, e = ids[row];
-  const int c = blk * 128 + 2 * lane;
-  const uint16_t* xr = x + (size_t)tok * H + c;
-  const float* r = rin + (size_t)e * H + c;
-  float v0 = (float)__builtin_bit_cast(half_t, xr[0]) * r[0];
-  float v1 = (float)__builtin_bit_cast(half_t, xr[1]) * r[1];
-  h128_wave(v0, v1);
-  uint16_t* o = xh + (size_t)row * H + c;
-  o[0] = __builtin_bit_cast(uint16_t, to_f16(v0 * rs));
-  o[1] = __builtin_bit_cast(uint16_t, to_f16(v1 * rs));
+  const int c = blk * 128 + 2 * lane, row0 = tok * top_k + s0, n = top_k - s0;
+  const float2 xv = row_pair<kRowsF16>(x, (size_t)tok * H + c);
+  float2 r[NS];
+#pragma unroll
+  for (int j = 0; j < NS; ++j)
+    r[j] = ld_global_f2(rin + (size_t)ids[row0 + min(j, n - 1)] * H + c);
+#pragma unroll
+  for (int j = 0; j < NS; ++j) {
+    float v0 = xv.x * r[j].x, v1 = xv.y * r[j].y;
+    h128_wave(v0, v1);
+    if (j < n)
+      *reinterpret_cast<uint32_t*>(xh + (size_t)(row0 + j) * H + c) =
+          pack2(to_f16(v0 * rs), to_f16(v1 * rs));
+  }
 }
 
 // grid (H/128, T*k), block 64.
@@ -32,13 +40,17 @@ __global__ __launch_bounds__(64) void k_moe_input(const uint16_t* __restrict__ x
                                                   const int* __restrict__ ids, int top_k,
                                                   const float* __restrict__ rin, int H, float rs,
                                                   uint16_t* __restrict__ xh) {
-  moe_input_wave(x, ids, top_k, rin, H, rs, xh, blockIdx.x, blockIdx.y);
+  const int row = blockIdx.y, tok = row / top_k;
+  moe_input_wave<1>(x, ids, top_k, rin, H, rs, xh, blockIdx.x, tok, row - tok * top_k);
 }
 
 // The chain's two independent first steps in one launch: block 0 groups the
 // routed rows by expert (build_groups_block); every other block runs 16 of
-// the (128-block, row) input transforms, one per wave.  grid
-// 1 + ceil(H/128 * m / 16), block 1024.
+// the input transforms of (128-block, token, NS slots), one per wave.  NS = 4
+// (a token's inputs and ids read once per four slots, 4-byte accesses) where
+// the rows fill the GPU all the same; NS = 1 below that.  grid
+// 1 + ceil(H/128 * T * ceil(top_k/NS) / 16), block 1024.
+template <int NS>
 __global__ __launch_bounds__(1024) void k_moe_prep(const uint16_t* __restrict__ x,
                                                    const int* __restrict__ ids, int top_k,
                                                    const float* __restrict__ rin, int H, float rs,
@@ -50,8 +62,11 @@ __global__ __launch_bounds__(1024) void k_moe_prep(const uint16_t* __restrict__ 
     build_groups_block(ids, m, E, R, n_groups, rows_idx, group_expert, n_active);
     return;
   }
-  const int nhb = H / 128, w = (blockIdx.x - 1) * 16 + (threadIdx.x >> 6);
-  if (w < nhb * m) moe_input_wave(x, ids, top_k, rin, H, rs, xh, w % nhb, w / nhb);
+  const int nhb = H / 128, ns = (top_k + NS - 1) / NS;
+  const int w = __builtin_amdgcn_readfirstlane((blockIdx.x - 1) * 16 + (threadIdx.x >> 6));
+  const int p = w / nhb, tok = p / ns;  // (token, slots), blk fastest
+  if (tok < m / top_k)
+    moe_input_wave<NS>(x, ids, top_k, rin, H, rs, xh, w % nhb, tok, (p - tok * ns) * NS);
 }
 
 // The grouped split-K GEMM of k_gemv_fast_rows with the table decode, as a
@@ -349,19 +364,46 @@ __global__ __launch_bounds__(256) void k_swiglu(const uint16_t* __restrict__ gu,
 }
 
 // Weighted slot-order combine of already-transformed down outputs:
-// y[t] = f16(sum_s f32(d16[t*k+s]) * f32(f16(score[t*k+s]))).  grid (ceil(H/256), T), block 256.
+// y[t] = f16(sum_s f32(d16[t*k+s]) * f32(f16(score[t*k+s]))).  V columns per
+// thread (V = 8: 16-byte accesses, H a multiple of 8 and 16-byte aligned rows;
+// V = 1 otherwise), the rows of 8 slots requested together (slots past the
+// last re-read it and add +0: the sum starts at +0 and is never -0).  Reads
+// d16 once: 2048 tokens x 8 slots x 2048 columns (67 MB) is HBM-bound.
+// grid (ceil(H/V/256), T), block 256.
+template <int V>
 __global__ __launch_bounds__(256) void k_combine(const uint16_t* __restrict__ d16,
                                                  const float* __restrict__ scores, int top_k,
                                                  int H, uint16_t* __restrict__ y) {
-  const int c = blockIdx.x * 256 + threadIdx.x, tok = blockIdx.y;
+  const int c = (blockIdx.x * 256 + threadIdx.x) * V, tok = blockIdx.y;
   if (c >= H) return;
-  float a = 0.f;
-  for (int s = 0; s < top_k; ++s) {
-    const int row = tok * top_k + s;
-    const float w = (float)(half_t)scores[row];
-    a = a + (float)__builtin_bit_cast(half_t, d16[(size_t)row * H + c]) * w;
+  struct alignas(2 * V) Vec {
+    uint16_t h[V];
+  };
+  float a[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) a[i] = 0.f;
+  for (int s0 = 0; s0 < top_k; s0 += 8) {
+    const int n = min(8, top_k - s0);
+    Vec v[8];
+    float w[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int row = tok * top_k + s0 + min(j, n - 1);
+      w[j] = (float)(half_t)scores[row];
+      v[j] = *reinterpret_cast<const Vec*>(d16 + (size_t)row * H + c);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < V; ++i) {
+        const float t = (float)__builtin_bit_cast(half_t, v[j].h[i]) * w[j];
+        a[i] = a[i] + (j < n ? t : 0.f);
+      }
   }
-  y[(size_t)tok * H + c] = __builtin_bit_cast(uint16_t, (half_t)a);
+  Vec o;
+#pragma unroll
+  for (int i = 0; i < V; ++i) o.h[i] = __builtin_bit_cast(uint16_t, (half_t)a[i]);
+  *reinterpret_cast<Vec*>(y + (size_t)tok * H + c) = o;
 }
 
 }  // namespace esc

@@ -1,0 +1,65 @@
+"""GPU parity of the many-row expert path: the grouped matrix-core GEMM with its
+transforms and SwiGLU in the epilogues, at each of its row-block sizes, and the
+grouping of many rows."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ref_np as R
+
+from .conftest import has_gpu
+from .test_gpu_parity import _moe_case, _oracle_moe, dcode, ops
+
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(not has_gpu(), reason="needs a ROCm GPU")]
+
+DEV = "cuda"
+
+
+def _args(c, K_gu, K_dn):
+    dv = lambda n: torch.from_numpy(c[n]).to(DEV)
+    return [dcode(c["gu_code"]), dv("gu_rin"), dv("gu_rout"), K_gu, dcode(c["dn_code"]),
+            dv("dn_rin"), dv("dn_rout"), K_dn]
+
+
+# rows per expert 20, 33, 66, 96 on average: 32-, 64-, 96- and 128-row groups;
+# H of three 128-column blocks (half a workgroup unused in the down leg)
+@pytest.mark.parametrize("E,T,k,H,I,K_gu,K_dn", [(4, 40, 2, 256, 128, 2, 3), (3, 50, 2, 384, 128, 3, 2),
+                                                 (8, 66, 8, 256, 256, 2, 2), (2, 96, 2, 384, 128, 3, 3)],
+                         ids=["rows32", "rows64_h384", "rows96", "rows128_h384"])
+@pytest.mark.parametrize("skew", [False, True], ids=["spread", "skewed"])
+def test_grouped_gemm_path_vs_oracle(E, T, k, H, I, K_gu, K_dn, skew):
+    """f16 roundings at the oracle's points, float32 sums in another order: the
+    bar of the other expert paths (5e-3 of the largest output).  Skewed: every
+    token's first slot goes to expert 1, so some groups are full and others
+    hold one row or none."""
+    c = _moe_case(E, H, I, K_gu, K_dn, T, k, 70 + E + T)
+    logits = c["logits"].copy()
+    if skew:
+        logits[:, 1] += 20.0
+    ids, sc = ops().route_topk(torch.from_numpy(logits).to(DEV), k)
+    x = torch.from_numpy(c["x"]).to(DEV)
+    args = _args(c, K_gu, K_dn)
+    ws = torch.zeros(ops().moe_expert_path_workspace(T, k, E, H, I), dtype=torch.uint8, device=DEV)
+    y = ops().moe_expert_path(x, ids, sc, *args, ws=ws)
+    ids_np, sc_np = ids.cpu().numpy(), sc.cpu().numpy()
+    want = _oracle_moe(c, ids_np, sc_np, E, H, I, K_gu, K_dn, np.unique(ids_np)).astype(np.float32)
+    got = y.cpu().numpy().astype(np.float32)
+    assert np.abs(got - want).max() / np.abs(want).max() < 5e-3
+    assert torch.equal(ops().moe_expert_path(x, ids, sc, *args, lut=True, ws=ws), y)
+
+
+@pytest.mark.parametrize("m,E", [(1025, 256), (16384, 256), (5000, 512), (3000, 513), (1300, 2048)])
+def test_build_groups_many_rows(m, E):
+    """Both many-row forms (wave segments up to 512 experts, mask chunks above)
+    against the oracle's model: a skewed expert, an empty one, a ragged end."""
+    from escha_mlx_amd import moe
+    rng = np.random.default_rng(m + E)
+    re = rng.integers(0, E - 1, size=m).astype(np.int32)
+    re[rng.random(m) < 0.3] = E // 2
+    ng = moe.n_groups_bound(m, E, 16)
+    rows_idx, group_expert = moe.build_groups(torch.from_numpy(re).to(DEV), E, 16, ng)
+    ri, ge = R.build_groups(re, E, 16, ng)
+    assert np.array_equal(rows_idx.cpu().numpy(), ri)
+    assert np.array_equal(group_expert.cpu().numpy(), ge)
