@@ -345,7 +345,8 @@ __device__ void build_groups_mask(const int* __restrict__ row_expert, int m, int
 }
 
 // The segment form (E <= kGroupHistE): s_hist[wave][E] holds the wave's rows
-// per expert, then the slot of its next row of that expert.
+// per expert (s_cnt: the wave's own), then the slot of its next row of that
+// expert.
 __device__ void build_groups_hist(const int* __restrict__ row_expert, int m, int E, int R,
                                   int n_groups, int* __restrict__ rows_idx,
                                   int* __restrict__ group_expert, int* s_hist, int* s_wsum,
@@ -356,8 +357,8 @@ __device__ void build_groups_hist(const int* __restrict__ row_expert, int m, int
   __syncthreads();
   const int seg = ((m + 15) / 16 + 63) / 64 * 64;
   const int r0 = wave * seg, r1 = min(m, r0 + seg);
-  int* hist = s_hist + wave * E;
-  for (int r = r0 + lane; r < r1; r += 64) atomicAdd(&hist[row_expert[r]], 1);
+  int* s_cnt = s_hist + wave * E;
+  for (int r = r0 + lane; r < r1; r += 64) atomicAdd(&s_cnt[row_expert[r]], 1);
   __syncthreads();
   // expert tid: its padded count, first slot, groups and padding slots (= m),
   // and each wave's first slot
@@ -396,13 +397,38 @@ __device__ void build_groups_hist(const int* __restrict__ row_expert, int m, int
     }
     const int rank = __popcll(same & ((1ull << lane) - 1ull)), n = __popcll(same);
     if (ok) {
-      const int slot = hist[e];
+      const int slot = s_cnt[e];
       rows_idx[slot + rank] = r + lane;
-      if (rank == n - 1) hist[e] = slot + n;
+      if (rank == n - 1) s_cnt[e] = slot + n;
     }
     // the slots just written are read by the next 64 rows
     __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
+}
+
+// Places rows row0 .. row0 + n - 1 (row_expert: of row0; n <= 64 nw) from their
+// experts' next slots s_cnt; the masks are zero before and after.
+__device__ void build_groups_chunk(const int* __restrict__ row_expert, int row0, int n, int E,
+                                   int nw, int* __restrict__ rows_idx, int* s_cnt,
+                                   unsigned long long* s_mask) {
+  const int tid = threadIdx.x, nt = blockDim.x;
+  for (int r = tid; r < n; r += nt)
+    atomicOr(&s_mask[row_expert[r] * nw + (r >> 6)], 1ull << (r & 63));
+  __syncthreads();
+  for (int r = tid; r < n; r += nt) {
+    const int e = row_expert[r], w0 = r >> 6;
+    const unsigned long long* me = s_mask + e * nw;
+    int rank = __popcll(me[w0] & ((1ull << (r & 63)) - 1ull));
+    for (int w = 0; w < w0; ++w) rank += __popcll(me[w]);
+    rows_idx[s_cnt[e] + rank] = row0 + r;
+  }
+  __syncthreads();
+  for (int r = tid; r < n; r += nt) {
+    const int e = row_expert[r];
+    atomicAdd(&s_cnt[e], 1);
+  }
+  for (int i = tid; i < E * nw; i += nt) s_mask[i] = 0ull;
+  __syncthreads();
 }
 
 // n_active (when not null): the number of groups that hold rows.
@@ -410,7 +436,7 @@ __device__ void build_groups_block(const int* __restrict__ row_expert, int m, in
                                    int n_groups, int* __restrict__ rows_idx,
                                    int* __restrict__ group_expert,
                                    int* __restrict__ n_active = nullptr) {
-  // first padded slot of each expert (chunked form: plus its rows placed so far)
+  // first padded slot of each expert
   __shared__ int s_start[4096];
   __shared__ unsigned long long s_mask[kGroupMaskWords];  // [E][nw]
   __shared__ int s_wsum[16];
@@ -426,17 +452,18 @@ __device__ void build_groups_block(const int* __restrict__ row_expert, int m, in
   }
   const int tid = threadIdx.x, nt = blockDim.x;
   const int nw = kGroupMaskWords / E;  // mask words per expert, 64 rows each
-  for (int e = tid; e < E; e += nt) s_start[e] = 0;
+  int* s_cnt = s_start;  // rows per expert, then each expert's next slot
+  for (int e = tid; e < E; e += nt) s_cnt[e] = 0;
   for (int i = tid; i < E * nw; i += nt) s_mask[i] = 0ull;
   __syncthreads();
-  for (int r = tid; r < m; r += nt) atomicAdd(&s_start[row_expert[r]], 1);
+  for (int r = tid; r < m; r += nt) atomicAdd(&s_cnt[row_expert[r]], 1);
   __syncthreads();
   // experts 4 tid .. 4 tid + 3: padded counts, first slots, their groups and
   // their padding slots (= m)
   int cnt[4], sum = 0;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    cnt[j] = 4 * tid + j < E ? s_start[4 * tid + j] : 0;
+    cnt[j] = 4 * tid + j < E ? s_cnt[4 * tid + j] : 0;
     sum += (cnt[j] + R - 1) / R * R;
   }
   int total;
@@ -444,7 +471,7 @@ __device__ void build_groups_block(const int* __restrict__ row_expert, int m, in
   for (int j = 0; j < 4; ++j) {
     const int e = 4 * tid + j, pad = (cnt[j] + R - 1) / R * R;
     if (e < E) {
-      s_start[e] = start;
+      s_cnt[e] = start;
       for (int g = start / R; g < (start + pad) / R; ++g) group_expert[g] = e;
       for (int i = cnt[j]; i < pad; ++i) rows_idx[start + i] = m;
     }
@@ -454,29 +481,9 @@ __device__ void build_groups_block(const int* __restrict__ row_expert, int m, in
   for (int i = total + tid; i < n_groups * R; i += nt) rows_idx[i] = m;
   for (int g = total / R + tid; g < n_groups; g += nt) group_expert[g] = -1;
   // stable placement, one chunk of rows at a time
-  for (int c0 = 0; c0 < m; c0 += 64 * nw) {
-    const int n = min(64 * nw, m - c0);
-    for (int r = tid; r < n; r += nt)
-      atomicOr(&s_mask[row_expert[c0 + r] * nw + (r >> 6)], 1ull << (r & 63));
-    __syncthreads();
-    for (int r = tid; r < n; r += nt) {
-      const int e = row_expert[c0 + r], w0 = r >> 6;
-      const unsigned long long* me = s_mask + e * nw;
-      int rank = __popcll(me[w0] & ((1ull << (r & 63)) - 1ull));
-      for (int w = 0; w < w0; ++w) rank += __popcll(me[w]);
-      rows_idx[s_start[e] + rank] = c0 + r;
-    }
-    __syncthreads();
-    for (int e = tid; e < E; e += nt) {
-      int k = 0;
-      for (int w = 0; w < nw; ++w) {
-        k += __popcll(s_mask[e * nw + w]);
-        s_mask[e * nw + w] = 0ull;
-      }
-      s_start[e] += k;
-    }
-    __syncthreads();
-  }
+  __syncthreads();
+  for (int c0 = 0; c0 < m; c0 += 64 * nw)
+    build_groups_chunk(row_expert + c0, c0, min(64 * nw, m - c0), E, nw, rows_idx, s_cnt, s_mask);
 }
 
 __global__ __launch_bounds__(1024) void k_build_groups(const int* __restrict__ row_expert, int m,
