@@ -251,6 +251,96 @@ struct FastRowsF {
   }
 };
 
+// Compute units of the current device (queried once per device).
+int device_cus() {
+  static int cus[64] = {};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+  if (!cus[dev]) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      n = 256;
+    cus[dev] = n;
+  }
+  return cus[dev];
+}
+
+// Row blocks of 16 per k_gemm_mma2 workgroup (NRB in {2,4,6,8}) and splits S of
+// the K steps (4 kt each).  A step of one workgroup takes about 0.66 + 0.055 NRB
+// us of its CU (K = 3; decode, then MFMAs), a lone workgroup on a CU 1.24 times
+// that, and no step less than 1.05 + 0.02 NRB us (the code's latency over the two
+// steps it is requested ahead).  A launch takes what the busiest CU holds; splits add
+// their float32 partials, written and read back at about 4.5 TB/s, and the
+// reduction launch.  Measured on MI355X (whole linear, unsplit against the plan's
+// choice; a sweep of 19 (NRB, S) pairs finds nothing more than 5 % faster):
+// K = 3 17408 -> 5120, 16 / 40 / 256 / 2048 rows 284 / 287 / 291 / 526 us against
+// 37 / 42 / 88 / 446; K = 2 5120 -> 5120, 16 / 256 / 2048 rows 90 / 96 / 165
+// against 25 / 44 / 155; K = 2 2048 -> 4096, 16 / 600 rows 42 / 53 against 25 /
+// 37.  A split keeps at least kMmaMinSteps steps.
+constexpr int kMmaMinSteps = 10;
+constexpr size_t kMmaPartMax = size_t(128) << 20;
+struct MmaPlan {
+  int nrb, S;
+  size_t part_bytes;
+};
+size_t mma2_part_bytes(int M, int TN, int S) {
+  return (size_t)S * ((M + 15) / 16) * ((TN + 15) / 16) * 16384;
+}
+MmaPlan mma_plan(int M, int TK, int TN, bool split) {
+  const int cus = device_cus(), NS = TK / 4, ncb = (TN + 15) / 16;
+  MmaPlan best{8, 1, 0};
+  double best_cost = 1e30;
+  for (int S = 1; S == 1 || (split && S * kMmaMinSteps <= NS); ++S) {
+    const size_t part = S > 1 ? mma2_part_bytes(M, TN, S) : 0;
+    if (part > kMmaPartMax) break;
+    const double extra = S > 1 ? 2.0 * part / 4.5e6 + 5.0 : 0.0;
+    for (int nrb = 8; nrb >= 2; nrb -= 2) {
+      const long wgs = (long)((M + 16 * nrb - 1) / (16 * nrb)) * ncb * S;
+      const long n = (wgs + cus - 1) / cus;
+      const double step = std::max((n + (n & 1 ? 0.24 : 0.0)) * (0.66 + 0.055 * nrb),
+                                   1.05 + 0.02 * nrb);
+      const double cost = step * ((NS + S - 1) / S) + extra;
+      // a split has to pay: 5 % over one launch
+      if (cost < best_cost * (S > 1 && best.S == 1 ? 0.95 : 0.999)) {
+        best_cost = cost;
+        best = {nrb, S, part};
+      }
+    }
+  }
+  return best;
+}
+
+template <int MODE>
+int gemm_mma2_launch(int K, int nrb, int S, const esc::MmaArgs& a, hipStream_t s) {
+  const dim3 grid(((a.M + 16 * nrb - 1) / (16 * nrb)) * ((a.TN + 15) / 16), S);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a); };
+  if (K == 2) {
+    if (nrb == 2) go(esc::k_gemm_mma2<2, 2, MODE>);
+    else if (nrb == 4) go(esc::k_gemm_mma2<2, 4, MODE>);
+    else if (nrb == 6) go(esc::k_gemm_mma2<2, 6, MODE>);
+    else go(esc::k_gemm_mma2<2, 8, MODE>);
+  } else {
+    if (nrb == 2) go(esc::k_gemm_mma2<3, 2, MODE>);
+    else if (nrb == 4) go(esc::k_gemm_mma2<3, 4, MODE>);
+    else if (nrb == 6) go(esc::k_gemm_mma2<3, 6, MODE>);
+    else go(esc::k_gemm_mma2<3, 8, MODE>);
+  }
+  return launched("k_gemm_mma2");
+}
+
+// The many-row GEMM with its output transform: one launch, or the splits'
+// partials into a.mid (plan.part_bytes) and their reduction.
+int gemm_mma2_out(int K, const MmaPlan& plan, const esc::MmaArgs& a, hipStream_t s) {
+  if (plan.S == 1) return gemm_mma2_launch<esc::kMmaOut>(K, plan.nrb, 1, a, s);
+  if (int rc = gemm_mma2_launch<esc::kMmaPart>(K, plan.nrb, plan.S, a, s)) return rc;
+  const dim3 grid((a.TN + 15) / 16, (a.M + 15) / 16);
+  if (K == 2)
+    hipLaunchKernelGGL(esc::k_mma2_reduce<2>, grid, dim3(256), 0, s, a, plan.S);
+  else
+    hipLaunchKernelGGL(esc::k_mma2_reduce<3>, grid, dim3(256), 0, s, a, plan.S);
+  return launched("k_mma2_reduce");
+}
+
 // ---- one-launch linear for M < 16 (linear.hpp)
 constexpr int kLinearSmallRows = 16;
 constexpr int kLinearSmallRowsLut = 8;
@@ -286,6 +376,8 @@ size_t rows1_part_bytes(int TK, int TN) { return (size_t)(TN / 16) * rows1_maxc(
 struct LinearPlan {
   int R, S, KS, groups, row_groups;
   size_t off_part, off_cnt, off_xh, off_mid, total;
+  MmaPlan mma;        // 16 rows and more
+  size_t min_total;   // enough without splits
 };
 
 // Fewest splits that reach the workgroup target: more splits mean more
@@ -339,9 +431,12 @@ LinearPlan linear_plan(int M, int K, int IC, int OC, bool lut) {
     if (M == 1 && TN % 16 == 0)
       p.total = std::max(p.total, p.off_part + al(rows1_part_bytes(TK, TN)));
   } else {
+    // the splits' partials, or the M x OC floats that a workspace always had
+    p.mma = mma_plan(M, TK, TN, true);
     p.off_xh = 0;
     p.off_mid = al((size_t)M * IC * 2);
-    p.total = p.off_mid + al((size_t)M * OC * 4);
+    p.min_total = p.off_mid + al((size_t)M * OC * 4);
+    p.total = p.off_mid + al(std::max((size_t)M * OC * 4, p.mma.part_bytes));
   }
   return p;
 }
@@ -389,20 +484,6 @@ int linear_pair_k(int K0, int K1, const esc::LinearSmallArgs& a0, const esc::Lin
   if (K0 == 2) return K1 == 2 ? linear_pair_launch<2, 2, LUT>(a0, a1, s)
                               : linear_pair_launch<2, 3, LUT>(a0, a1, s);
   return K1 == 2 ? linear_pair_launch<3, 2, LUT>(a0, a1, s) : linear_pair_launch<3, 3, LUT>(a0, a1, s);
-}
-
-// Compute units of the current device (queried once per device).
-int device_cus() {
-  static int cus[64] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-  if (!cus[dev]) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      n = 256;
-    cus[dev] = n;
-  }
-  return cus[dev];
 }
 
 // k_proj_rows1 over a.np projections whose x .. TK, TN are filled: each
@@ -466,26 +547,6 @@ int launch_rows1(esc::ProjArgs& a, int K, bool lut, hipStream_t s, bool merged =
   return lut ? launch_rows1_k<3, kTablePairs3>(a, (int)grid, s) : launch_rows1_k<3, 0>(a, (int)grid, s);
 }
 
-// Row blocks of 16 per k_gemm_mma2 workgroup (NRB in {2,4,6,8}).  The kernel
-// is decode-bound, so a tile's time grows slowly with its rows (measured on
-// MI355X: 0.76 + 0.03 NRB, relative to NRB = 8), and a launch takes as many
-// tile-times as the busiest CU holds tiles: pick the NRB that minimises
-// ceil(tiles / CUs) * tile time.
-int mma2_row_blocks(int M, int TN) {
-  const int cus = device_cus();
-  int best = 8;
-  double best_cost = 1e30;
-  for (int nrb = 8; nrb >= 2; nrb -= 2) {
-    const long tiles = (long)((M + 16 * nrb - 1) / (16 * nrb)) * (TN / 16);
-    const double cost = (double)((tiles + cus - 1) / cus) * (0.76 + 0.03 * nrb);
-    if (cost < best_cost * 0.999) {
-      best_cost = cost;
-      best = nrb;
-    }
-  }
-  return best;
-}
-
 // k_combine, 8 columns per thread where the rows allow 16-byte accesses.
 int combine_rows(const uint16_t* d16, const float* scores, int T, int top_k, int H, uint16_t* y,
                  hipStream_t s) {
@@ -498,30 +559,6 @@ int combine_rows(const uint16_t* d16, const float* scores, int T, int top_k, int
   else
     hipLaunchKernelGGL(esc::k_combine<1>, grid, dim3(256), 0, s, d16, scores, top_k, H, y);
   return launched("k_combine");
-}
-
-// k_gemm_mma2 launch (TN % 16 == 0); OUT: output transform fused, y written.
-template <bool OUT>
-int gemm_mma2(int K, const uint16_t* xh, const uint32_t* code, int M, int TK, int TN, float* mid,
-              const float* rout, const uint16_t* bias, float rs, uint16_t* y, hipStream_t s) {
-  const int nrb = mma2_row_blocks(M, TN);
-  const int blocks = ((M + 16 * nrb - 1) / (16 * nrb)) * (TN / 16);
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, s, xh, code, M, TK, TN, mid, rout, bias,
-                       rs, y);
-  };
-  if (K == 2) {
-    if (nrb == 2) go(esc::k_gemm_mma2<2, 2, OUT>);
-    else if (nrb == 4) go(esc::k_gemm_mma2<2, 4, OUT>);
-    else if (nrb == 6) go(esc::k_gemm_mma2<2, 6, OUT>);
-    else go(esc::k_gemm_mma2<2, 8, OUT>);
-  } else {
-    if (nrb == 2) go(esc::k_gemm_mma2<3, 2, OUT>);
-    else if (nrb == 4) go(esc::k_gemm_mma2<3, 4, OUT>);
-    else if (nrb == 6) go(esc::k_gemm_mma2<3, 6, OUT>);
-    else go(esc::k_gemm_mma2<3, 8, OUT>);
-  }
-  return launched("k_gemm_mma2");
 }
 
 }  // namespace
@@ -641,24 +678,38 @@ size_t esc_linear_workspace(int M, int K, int IC, int OC) {
 int esc_linear(const uint16_t* x, const float* rin, const uint32_t* code, const float* rout,
                const uint16_t* bias, int M, int K, int IC, int OC, int use_lut, float rs,
                uint16_t* y, void* ws, size_t ws_bytes, void* stream) {
+  return esc_linear_typed(x, ESC_ROWS_F16, rin, code, rout, bias, M, K, IC, OC, use_lut, rs, y, ws,
+                          ws_bytes, stream);
+}
+
+int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t* code,
+                     const float* rout, const uint16_t* bias, int M, int K, int IC, int OC,
+                     int use_lut, float rs, void* y, void* ws, size_t ws_bytes, void* stream) {
   if (int rc = check_proj(K, IC, OC)) return rc;
   ESC_REQUIRE(x && rin && code && rout && y, "null pointer");
   ESC_REQUIRE(M >= 0, "negative row count");
+  ESC_REQUIRE(dtype == ESC_ROWS_F16 || ((dtype == ESC_ROWS_BF16 || dtype == ESC_ROWS_F32) &&
+                                        (M >= kLinearSmallRows || M == 0)),
+              "row element type %d with %d rows", dtype, M);
   if (M == 0) return ESC_OK;
   use_lut = linear_uses_lut(M, IC, OC, use_lut != 0);
   const LinearPlan lp = linear_plan(M, K, IC, OC, use_lut != 0);
-  if (!ws || ws_bytes < lp.total)
-    return fail(ESC_ENOSPACE, "workspace %zu bytes < required %zu", ws_bytes, lp.total);
+  const size_t need = M < kLinearSmallRows ? lp.total : lp.min_total;
+  if (!ws || ws_bytes < need)
+    return fail(ESC_ENOSPACE, "workspace %zu bytes < required %zu", ws_bytes, need);
   const int TK = IC / 16, TN = OC / 16;
   hipStream_t s = S(stream);
   char* w = static_cast<char*>(ws);
+  const uint16_t* x16 = static_cast<const uint16_t*>(x);
+  uint16_t* y16 = static_cast<uint16_t*>(y);
   if (rows1_single(M, IC, OC, use_lut != 0)) {
     // one row: the persistent kernel, its counters at off_cnt and its
     // partials at off_part (linear_plan sizes both)
     esc::ProjArgs a{};
     a.np = 1;
     a.rs = rs;
-    a.pr[0] = esc::ProjOne{x, rin, code, rout, bias, y, reinterpret_cast<float*>(w + lp.off_part),
+    a.pr[0] = esc::ProjOne{x16, rin, code, rout, bias, y16,
+                           reinterpret_cast<float*>(w + lp.off_part),
                            reinterpret_cast<int*>(w + lp.off_cnt), TK, TN};
     return launch_rows1(a, K, use_lut != 0, s);
   }
@@ -666,15 +717,19 @@ int esc_linear(const uint16_t* x, const float* rin, const uint32_t* code, const 
     // the split-K kernel, by hash (linear_uses_lut)
     float* part = reinterpret_cast<float*>(w + lp.off_part);
     int* cnt = reinterpret_cast<int*>(w + lp.off_cnt);
-    const esc::LinearSmallArgs a = small_args(x, rin, code, rout, bias, M, TK, TN, lp, rs, part, cnt, y);
+    const esc::LinearSmallArgs a =
+        small_args(x16, rin, code, rout, bias, M, TK, TN, lp, rs, part, cnt, y16);
     return K == 2 ? LinearSmallF<2, false>::run(a, s) : LinearSmallF<3, false>::run(a, s);
   }
   // many rows: input transform, then the matrix-core GEMM with the output
-  // transform in its epilogue (or GEMM + output transform for OC % 256 != 0)
+  // transform in its epilogue, or in its splits' reduction.  A workspace with
+  // no room for the partials takes the one launch.
   uint16_t* xh = reinterpret_cast<uint16_t*>(w + lp.off_xh);
-  if (int rc = esc_input_transform(x, rin, nullptr, M, IC, rs, xh, stream)) return rc;
-  return esc_gemm_mfma_out(xh, code, rout, bias, M, K, IC, OC, rs, y, w + lp.off_mid,
-                           lp.total - lp.off_mid, stream);
+  if (int rc = esc_input_transform_typed(x, dtype, rin, nullptr, M, IC, rs, xh, stream)) return rc;
+  const MmaPlan plan = ws_bytes < lp.total ? mma_plan(M, TK, TN, false) : lp.mma;
+  const esc::MmaArgs a{xh, code, M, TK, TN, reinterpret_cast<float*>(w + lp.off_mid),
+                       rout, bias, rs, y, dtype};
+  return gemm_mma2_out(K, plan, a, s);
 }
 
 size_t esc_gemm_mfma_out_workspace(int M, int K, int IC, int OC) {
@@ -691,15 +746,13 @@ int esc_gemm_mfma_out(const uint16_t* xh, const uint32_t* code, const float* rou
   if (M == 0) return ESC_OK;
   const int TK = IC / 16, TN = OC / 16;
   hipStream_t s = S(stream);
-  // OC a multiple of 256: the output transform in the GEMM's epilogue
-  if (TN % 16 == 0) return gemm_mma2<true>(K, xh, code, M, TK, TN, nullptr, rout, bias, rs, y, s);
   const size_t need = esc_gemm_mfma_out_workspace(M, K, IC, OC);
-  if (!ws || ws_bytes < need)
+  if (need && (!ws || ws_bytes < need))
     return fail(ESC_ENOSPACE, "workspace %zu bytes < required %zu", ws_bytes, need);
-  float* mid = static_cast<float*>(ws);
-  if (int rc = esc_gemm_mfma(xh, code, M, K, IC, OC, 0, mid, stream)) return rc;
-  return esc_output_transform(mid, rout, nullptr, bias, M, OC, rs, y, stream);
+  const esc::MmaArgs a{xh, code, M, TK, TN, nullptr, rout, bias, rs, y, ESC_ROWS_F16};
+  return gemm_mma2_out(K, mma_plan(M, TK, TN, false), a, s);
 }
+
 
 size_t esc_linear_pair_workspace(int M, int K0, int K1, int IC, int OC0, int OC1) {
   const size_t a = esc_linear_workspace(M, K0, IC, OC0), b = esc_linear_workspace(M, K1, IC, OC1);
@@ -952,16 +1005,8 @@ int esc_gemm_mfma(const uint16_t* xh, const uint32_t* code, int M, int K, int IC
   if (M == 0) return ESC_OK;
   const int TK = IC / 16, TN = OC / 16;
   hipStream_t s = S(stream);
-  if (TN % 16 == 0)
-    return gemm_mma2<false>(K, xh, code, M, TK, TN, mid, nullptr, nullptr, 0.f, nullptr, s);
-  const int blocks = ((M + esc::kMmaRows - 1) / esc::kMmaRows) * (TN / 8);
-  if (K == 2)
-    hipLaunchKernelGGL(esc::k_gemm_mfma<2>, dim3(blocks), dim3(esc::kMmaThreads), 0, s, xh, code,
-                       M, TK, TN, mid);
-  else
-    hipLaunchKernelGGL(esc::k_gemm_mfma<3>, dim3(blocks), dim3(esc::kMmaThreads), 0, s, xh, code,
-                       M, TK, TN, mid);
-  return launched("k_gemm_mfma");
+  const esc::MmaArgs a{xh, code, M, TK, TN, mid, nullptr, nullptr, 0.f, nullptr, ESC_ROWS_F16};
+  return gemm_mma2_launch<esc::kMmaMid>(K, mma_plan(M, TK, TN, false).nrb, 1, a, s);
 }
 
 int esc_build_groups(const int32_t* row_expert, int m, int E, int R, int n_groups,

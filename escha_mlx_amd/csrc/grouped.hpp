@@ -48,17 +48,18 @@ __global__ __launch_bounds__(256, 2) void k_moe_mma(MoeMmaArgs a) {
   using G = Geo<K>;
   using D = Mma2<K, NRB>;
   constexpr int BR = D::BR, XCH = D::XCH;
-  constexpr int kPitch = 128 + 4;  // floats per staged row
   __shared__ uint4 s_x[2][BR * 8];
-  static_assert(sizeof(s_x) >= 2 * 16 * kPitch * sizeof(float) || NRB < 6, "");
-  __shared__ float s_o[NRB < 6 ? 2 * 16 * kPitch : 1];
+  // the epilogue's exchange areas, over x's stages where they fit
+  constexpr int kAreas = GU ? kMma2Xch + 4 * 3 * 64 : 2 * kMma2Xch;  // float4
+  constexpr bool kOwn = sizeof(s_x) < kAreas * sizeof(float4);
+  __shared__ float4 s_o[kOwn ? kAreas : 1];
   const int per = 8 * a.ncb, q8 = blockIdx.x / per, rem = blockIdx.x % per;
   const int g = 8 * q8 + rem % 8, cb = rem / 8;
   if (g >= a.n_groups) return;
   const int e = a.group_expert[g];
   if (e < 0) return;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int pair = wave >> 1, hw = wave & 1;
+  const int pair = wave >> 1, hw = wave & 1;  // 128-column half, 64-column quarter
   const int M = a.M, TK = a.TK, TN = a.TN;
   const int IC = TK * 16, OC = TN * 16;
   const int gk = lane >> 4, c = lane & 15, tc = c / G::LPT, q = lane % G::LPT;
@@ -80,53 +81,114 @@ __global__ __launch_bounds__(256, 2) void k_moe_mma(MoeMmaArgs a) {
   f32x4_t acc[D::NA][NRB];
   mma2_loop<K, NRB>(cbase, kstride, xrs, xoff, 0, TK / 4, s_x, acc);
 
-  float* so = NRB < 6 ? s_o : reinterpret_cast<float*>(&s_x[0][0]);
-  float* sp = so + pair * 16 * kPitch;
+  float4* so = kOwn ? s_o : reinterpret_cast<float4*>(&s_x[0][0]);
   const float rs = a.rs;
+  const int chunk = mma2_chunk<K>();
   if constexpr (GU) {
-    const int I = OC / 2, col = 128 * cb + 2 * lane;
-    const float2 rg = ld_global_f2(a.rout + (size_t)e * OC + col);
-    const float2 ru = ld_global_f2(a.rout + (size_t)e * OC + I + col);
-    const float2 ri = ld_global_f2(a.dn_rin + (size_t)e * I + col);
+    const int I = OC / 2;
+    // gate (pair 0) and up (pair 1) output scales of the lane's 16 columns
+    // col + 64b + j; then the lane's 8 columns of h, ch + j
+    const int col = 128 * cb + 32 * hw + 8 * chunk;
+    float ro[16], ri[8];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      ro[j] = as_global(a.rout + (size_t)e * OC + pair * I)[col + 64 * (j >> 3) + (j & 7)];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ri[j] = as_global(a.dn_rin + (size_t)e * I)[col + 64 * pair + j];
+    uint4* s_gu = reinterpret_cast<uint4*>(so + kMma2Xch);  // gate / up halves, f16
+    float4* s_a = so + kMma2Xch + 256;                      // the two cross-wave stages of h
+    float4* s_b = s_a + 256;
 #pragma unroll
     for (int r = 0; r < NRB; ++r) {
-      mma2_to_lds<K, NRB>(acc, r, sp + 64 * hw, kPitch);
-      __syncthreads();
-#pragma unroll 2
+      const int row = rows[16 * r + c];
+      float v[16], o[16];
+      mma2_h64<K, NRB>(acc, r, v);
+      mma2_h128_last(v, so, o);
+      half_t h[16];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) h[j] = to_f16((o[j] * rs) * ro[j]);
+      // gate waves keep columns 64b + .. of b = 0 and get their up values, up
+      // waves b = 1 and their gate values: wave (pair, hw) then has the h
+      // columns col + 64 pair + j
+      uint32_t mine[4], send[4];
+#pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int rl = 4 * wave + j, row = rows[16 * r + rl];
-        if (row >= M) continue;  // wave-uniform: padding follows the group's rows
-        const float* sg = so + rl * kPitch + 2 * lane;
-        const float* su = sg + 16 * kPitch;
-        float g0 = sg[0], g1 = sg[1], u0 = su[0], u1 = su[1];
-        h128_wave(g0, g1);
-        h128_wave(u0, u1);
-        const half_t h0 = swiglu1(to_f16((g0 * rs) * rg.x), to_f16((u0 * rs) * ru.x));
-        const half_t h1 = swiglu1(to_f16((g1 * rs) * rg.y), to_f16((u1 * rs) * ru.y));
-        float v0 = (float)h0 * ri.x, v1 = (float)h1 * ri.y;
-        h128_wave(v0, v1);
-        *reinterpret_cast<uint32_t*>(a.out + (size_t)row * I + col) =
-            pack2(to_f16(v0 * rs), to_f16(v1 * rs));
+        const uint32_t p0 = pack2(h[2 * j], h[2 * j + 1]), p1 = pack2(h[8 + 2 * j], h[9 + 2 * j]);
+        mine[j] = pick(pair, p1, p0);
+        send[j] = pick(pair, p0, p1);
       }
-      __syncthreads();
+      s_gu[wave * 64 + lane] = make_uint4(send[0], send[1], send[2], send[3]);
+      lds_barrier();
+      const uint4 got4 = s_gu[(wave ^ 2) * 64 + lane];
+      const uint32_t got[4] = {got4.x, got4.y, got4.z, got4.w};
+      float f[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t gw = pick(pair, got[j >> 1], mine[j >> 1]);
+        const uint32_t uw = pick(pair, mine[j >> 1], got[j >> 1]);
+        const half_t hv = swiglu1(__builtin_bit_cast(half_t, (uint16_t)(gw >> (16 * (j & 1)))),
+                                  __builtin_bit_cast(half_t, (uint16_t)(uw >> (16 * (j & 1)))));
+        f[j] = (float)hv * ri[j];
+      }
+      // H128 of h: column bits 0..2 in registers, 3 and 4 in the lanes (bit 3
+      // is lane bit 4 for K = 2, lane bit 5 for K = 3), 5 and 6 across the waves
+      bfly_reg<1>(f);
+      bfly_reg<2>(f);
+      bfly_reg<4>(f);
+      bfly_lane<4, K == 2>(f);  // register bit 2: column bit 3
+      bfly_lane<4, K != 2>(f);  // register bit 2: column bit 4
+      // column bit 5: the other wave of the pair; this wave keeps bit 4 = hw
+      float4* x5 = s_a + wave * 64 + lane;
+      float t[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t[j] = pick(hw, f[j], f[4 + j]);
+      *x5 = make_float4(t[0], t[1], t[2], t[3]);
+      lds_barrier();
+      const float4 p5 = s_a[(wave ^ 1) * 64 + lane];
+      const float q5[4] = {p5.x, p5.y, p5.z, p5.w};
+      float lo[4], hi[4];  // column bit 5 = 0, 1
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float m = pick(hw, f[4 + j], f[j]);
+        const float x0 = pick(hw, q5[j], m), x1 = pick(hw, m, q5[j]);
+        lo[j] = x0 + x1;
+        hi[j] = x0 - x1;
+      }
+      // column bit 6: the other pair; this wave keeps bit 5 = pair
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t[j] = pick(pair, lo[j], hi[j]);
+      s_b[wave * 64 + lane] = make_float4(t[0], t[1], t[2], t[3]);
+      lds_barrier();
+      const float4 p6 = s_b[(wave ^ 2) * 64 + lane];
+      const float q6[4] = {p6.x, p6.y, p6.z, p6.w};
+      half_t y0[4], y1[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float m = pick(pair, hi[j], lo[j]);
+        const float x0 = pick(pair, q6[j], m), x1 = pick(pair, m, q6[j]);
+        y0[j] = to_f16((x0 + x1) * rs);
+        y1[j] = to_f16((x0 - x1) * rs);
+      }
+      // columns 64b + 32 pair + 16 hw + 8 (bit 3) + 4 (bit 2) + j, the column
+      // bits 2 and 3 in the lanes
+      if (row < M) {
+        const int b2 = K == 2 ? gk & 1 : gk >> 1, b3 = K == 2 ? gk >> 1 : gk & 1;
+        uint16_t* d = a.out + (size_t)row * I + 128 * cb + 32 * pair + 16 * hw + 8 * b3 + 4 * b2;
+        *reinterpret_cast<uint2*>(d) = make_uint2(pack2(y0[0], y0[1]), pack2(y0[2], y0[3]));
+        *reinterpret_cast<uint2*>(d + 64) = make_uint2(pack2(y1[0], y1[1]), pack2(y1[2], y1[3]));
+      }
     }
   } else {
-    const int col = 256 * cb + 128 * pair + 2 * lane;
-    const float2 ro = ld_global_f2(a.rout + (size_t)e * OC + (live ? col : 0));
+    const int col = live ? 256 * cb + 128 * pair + 32 * hw + 8 * chunk : 0;
+    float ro[16];
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      ro[j] = as_global(a.rout + (size_t)e * OC)[col + 64 * (j >> 3) + (j & 7)];
 #pragma unroll
     for (int r = 0; r < NRB; ++r) {
-      mma2_to_lds<K, NRB>(acc, r, sp + 64 * hw, kPitch);
-      __syncthreads();
-#pragma unroll 2
-      for (int j = 0; j < 8; ++j) {
-        const int rl = 8 * hw + j, row = rows[16 * r + rl];
-        if (row >= M || !live) continue;
-        float v0 = sp[rl * kPitch + 2 * lane], v1 = sp[rl * kPitch + 2 * lane + 1];
-        h128_wave(v0, v1);
-        *reinterpret_cast<uint32_t*>(a.out + (size_t)row * OC + col) =
-            pack2(to_f16((v0 * rs) * ro.x), to_f16((v1 * rs) * ro.y));
-      }
-      __syncthreads();
+      const int row = rows[16 * r + c];
+      mma2_out<K, NRB>(acc, r, so + (r & 1) * kMma2Xch, rs, ro, nullptr, col, row < M && live,
+                       a.out, kRowsF16, (size_t)row * OC + col);
     }
   }
 }

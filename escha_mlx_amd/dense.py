@@ -155,13 +155,13 @@ class EschaLinear(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         w = self._w
         shape = x.shape
-        # f16 rows take the fused transforms; bf16 / f32 rows are transformed
-        # from their float32 values first (dense.py:287-292), then the same
-        # kernels run from xh
+        # bf16 / f32 rows are transformed from their float32 values
+        # (dense.py:287-292); below 16 rows in a launch of its own, then the
+        # f16 rows' kernels run from xh
         rows = ops.as_rows(x.reshape(-1, shape[-1]))
         m = rows.shape[0]
-        if (rows.dtype == torch.float16 and not self._exact and self._block_r_pin is None
-                and self._fused_had and (m < ops.LINEAR_SMALL_ROWS or self._mat)):
+        if (not self._exact and self._block_r_pin is None and self._fused_had
+                and (self._mat if m >= ops.LINEAR_SMALL_ROWS else rows.dtype == torch.float16)):
             # the whole linear in esc_linear (one launch below 16 rows)
             y = ops.linear(rows, w.code, w.rin, w.rout, w.K, w.IC, w.OC, bias=self.bias,
                            lut=self._lut, ws=self._linear_ws(m, rows.device))

@@ -248,21 +248,25 @@ def linear(x: torch.Tensor, code_u32: torch.Tensor, rin: torch.Tensor, rout: tor
            rs: float = RS, ws: torch.Tensor | None = None) -> torch.Tensor:
     """The whole coded linear (input transform, GEMV/GEMM, output transform,
     optional f16 bias) -> y f16 [m, OC]; one launch below 16 rows
-    (dense.py:337-362).  ws must be zero-filled before its first use (the
-    one-launch path keeps self-resetting counters there)."""
+    (dense.py:337-362).  From 16 rows x may also be bf16 or f32: transformed
+    from its exact float32 values, y (the f16 result) in x's type.  ws must be
+    zero-filled before its first use (the one-launch path keeps self-resetting
+    counters there)."""
     _dev(x, code_u32, rin, rout, bias)
     m = x.shape[0]
-    if x.dtype != torch.float16 or tuple(x.shape) != (m, IC):
+    typed = m >= LINEAR_SMALL_ROWS and x.dtype in ROWS_DTYPES
+    if not (typed or x.dtype == torch.float16) or tuple(x.shape) != (m, IC):
         raise ValueError(f"x must be f16 [m, {IC}]")
-    y = torch.empty((m, OC), dtype=torch.float16, device=x.device)
+    y = torch.empty((m, OC), dtype=x.dtype, device=x.device)
     if m == 0:
         return y
     if ws is None:  # counters (one-launch path) must start at zero; the rest is scratch
         need = linear_workspace(m, K, IC, OC)
         alloc = torch.zeros if m < LINEAR_SMALL_ROWS else torch.empty
         ws = alloc(max(need, 4), dtype=torch.uint8, device=x.device)
-    _lib.call("esc_linear", _ptr(x), _ptr(rin), _ptr(_as_u32(code_u32)), _ptr(rout), _ptr(bias), m,
-              K, IC, OC, _lut_flag(lut), rs, _ptr(y), _ptr(ws), ws.numel(), _stream())
+    _lib.call("esc_linear_typed", _ptr(x), ROWS_DTYPES[x.dtype], _ptr(rin), _ptr(_as_u32(code_u32)),
+              _ptr(rout), _ptr(bias), m, K, IC, OC, _lut_flag(lut), rs, _ptr(y), _ptr(ws),
+              ws.numel(), _stream())
     return y
 
 

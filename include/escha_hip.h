@@ -115,10 +115,9 @@ int esc_dense_gemm_rows_out(const uint16_t* xh, const uint32_t* code, const floa
                             void* stream);
 
 /* mid f32 [M][OC] = xh f16 [M][IC] @ decode(code [TK][TN][8K]) on the matrix
- * cores: for OC a multiple of 256, v_mfma_f32_16x16x32_f16 with the weights
- * decoded straight into A operands (16*NRB rows x 256 columns per workgroup,
- * NRB chosen per shape); otherwise v_mfma_f32_32x32x16_f16 on weights decoded
- * into LDS (256 rows x 128 columns per workgroup).
+ * cores: v_mfma_f32_16x16x32_f16 with the weights decoded straight into A
+ * operands (16*NRB rows x 256 columns per workgroup, NRB chosen per shape; the
+ * last workgroup half used where OC is an odd multiple of 128).
  * Decoded weights are bit-exact; the float32 sum is reassociated
  * (deterministic; tolerance contract).  use_lut is accepted for the call
  * surface: table and hash decode give identical weights.
@@ -128,11 +127,11 @@ int esc_gemm_mfma(const uint16_t* xh, const uint32_t* code, int M, int K, int IC
 
 /* The many-row GEMM and its output transform in one step: y f16 [M][OC] =
  * (bias +) f16((H128(xh @ decode(code)) * rs) * rout), xh f16 [M][IC] already
- * input-transformed.  For OC a multiple of 256 the transform runs in the
- * epilogue of esc_gemm_mfma's kernel (no f32 mid; ws unused, the workspace
- * size is 0); otherwise esc_gemm_mfma into ws (esc_gemm_mfma_out_workspace
- * bytes, M * OC f32), then esc_output_transform.  Bit-identical to those two
- * calls; deterministic, reassociated float32 sum (tolerance contract).
+ * input-transformed.  The transform runs in the epilogue of esc_gemm_mfma's
+ * kernel (no f32 mid).  ws: esc_gemm_mfma_out_workspace bytes (0 for OC a
+ * multiple of 256, M * OC f32 otherwise; not written).  Bit-identical to
+ * esc_gemm_mfma, then esc_output_transform; deterministic, reassociated float32
+ * sum (tolerance contract).
  * Replaces EschaLinear's many-row path, self._output_rows(self._gemv(xh))
  * (escha_mlx/dense.py:356): msl.dense_gemm_mat then msl.dense_scaled_had_out
  * (escha_mlx/msl.py:1762-1782, 1486-1489). */
@@ -153,7 +152,12 @@ int esc_gemm_mfma_out(const uint16_t* xh, const uint32_t* code, const float* rou
  * groups when one would leave the GPU short of workgroups) sharing each
  * decoded weight on the matrix core.  The last split of each column group
  * sums the partials in fixed order and output-transforms.
- * M >= 16: input transform, then esc_gemm_mfma_out.  ws: esc_linear_workspace bytes, zero-filled before its
+ * M >= 16: input transform, then the matrix-core GEMM with the output transform
+ * in its epilogue (esc_gemm_mfma_out), or, where the tiles leave compute units
+ * idle, its K steps split over workgroups whose float32 partials a second launch
+ * sums in split order and output-transforms.  A ws of at least M * (2 IC + 4 OC)
+ * bytes (each rounded up to 256) that has no room for the partials takes one
+ * launch.  ws: esc_linear_workspace bytes, zero-filled before its
  * first use (its counters are left zero after every call); calls sharing one
  * ws must not overlap, and a ws moved to another shape is zero-filled again
  * (each shape's plan puts its counters where another's partials may lie).  Tolerance contract (reassociated float32 sum);
@@ -163,6 +167,15 @@ size_t esc_linear_workspace(int M, int K, int IC, int OC);
 int esc_linear(const uint16_t* x, const float* rin, const uint32_t* code, const float* rout,
                const uint16_t* bias, int M, int K, int IC, int OC, int use_lut, float rs,
                uint16_t* y, void* ws, size_t ws_bytes, void* stream);
+
+/* esc_linear for rows of another element type (ESC_ROWS_*): the rows are
+ * transformed from their exact float32 values, y has the rows' element type
+ * (the f16 result converted).  bf16 and f32 rows: M >= 16.
+ * Replaces EschaLinear.__call__ on non-f16 rows (escha_mlx/dense.py:287-292,
+ * 337-362). */
+int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t* code,
+                     const float* rout, const uint16_t* bias, int M, int K, int IC, int OC,
+                     int use_lut, float rs, void* y, void* ws, size_t ws_bytes, void* stream);
 
 /* Two coded linears over the same rows x f16 [M][IC] in one dispatch:
  * y0 = esc_linear(x; rin0, code0, rout0, bias0, K0, OC0) and likewise y1

@@ -179,3 +179,42 @@ def test_linear_many_rows_is_transform_then_gemm_out():
     y = ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias)
     want = ops().gemm_mfma_out(ops().scaled_had(x, rin_d, None), code, rout_d, K, ic, oc, bias=bias)
     assert torch.equal(y, want)
+
+
+# ---- esc_linear from 16 rows with its K steps split over workgroups: 1280
+# inputs are the fewest that split (20 steps), 1408 split unevenly; half a
+# workgroup of columns (384), one row past a row block, several row blocks
+SPLIT_SHAPES = [(2, 1280, 256, 16), (3, 1408, 384, 17), (2, 2688, 640, 33), (3, 2048, 512, 130)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("K,ic,oc,m", SPLIT_SHAPES)
+def test_linear_split_steps(K, ic, oc, m, dtype):
+    """Against the float64 product of the transformed rows (2e-3 of each row's
+    largest value: f16 output; bf16 output rounds once more, 2^-9); repeatable;
+    a workspace with no room for the partials takes the single launch, which is
+    esc_gemm_mfma_out's bits."""
+    rng = np.random.default_rng(5 * K + m)
+    u32, code = _code(rng, ic, oc, K)
+    rin = rng.choice([-1.0, 1.0], ic).astype(np.float32)
+    rout = _rout(rng, oc)
+    bias = (rng.standard_normal(oc) * 0.05).astype(np.float16)
+    x = torch.from_numpy(rng.standard_normal((m, ic)).astype(np.float32)).to(dtype).to(DEV)
+    rin_d, rout_d, bias_d = (torch.from_numpy(a).to(DEV) for a in (rin, rout, bias))
+    y = ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d)
+    assert y.dtype == dtype
+    xh = R.input_transform(x.float().cpu().numpy(), rin)
+    exact = R.h128(xh.astype(np.float64) @ R.reconstruct(u32, ic, oc, K).astype(np.float64)) \
+        * R.RS * rout + bias.astype(np.float64)
+    got = y.float().cpu().numpy().astype(np.float64)
+    err = (np.abs(got - exact).max(axis=1) / np.abs(exact).max(axis=1)).max()
+    assert err < 2e-3 + (2.0 ** -9 if dtype == torch.bfloat16 else 0.0), err
+    assert torch.equal(ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d), y)
+    al = lambda v: (v + 255) // 256 * 256
+    small = al(2 * m * ic) + al(4 * m * oc)
+    assert ops().linear_workspace(m, K, ic, oc) > small
+    ws = torch.empty(small, dtype=torch.uint8, device=DEV)
+    one = ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d, ws=ws)
+    want = ops().gemm_mfma_out(ops().scaled_had(x, rin_d, None), code, rout_d, K, ic, oc, bias=bias_d)
+    assert torch.equal(one, want.to(dtype))
