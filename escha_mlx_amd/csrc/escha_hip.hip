@@ -1137,6 +1137,42 @@ int rows_w8_mma(const uint16_t* x, const void* w, const float* scale, int M, int
   return ESC_OK;
 }
 
+// The matrix-core GEMMs from kRowsGemmRows rows (kRowsGemmRowsF16 for f16
+// weights, whose GEMV takes 8 rows per launch) and K a multiple of 64.  The time
+// of a launch is that of the busiest CU: n workgroups on it take t0 + t1 n us per
+// step (fitted to a sweep of 7 kernels over 33 shapes, int8, on MI355X).  K = 2048,
+// whole call: 203 x 512 14.1 us (16 rows per launch: 153), 1000 x 4096 38 (852),
+// 2048 x 4096 61 (1743), 64 x 248320 144 (570).
+constexpr int kRowsGemmRows = 17, kRowsGemmRowsF16 = 9;
+template <bool Q8>
+int rows_gemm(const uint16_t* x, const void* w, const float* scale, int M, int K, int O,
+              uint16_t* y, hipStream_t s) {
+  const int cus = device_cus(), NS = K / 64;
+  struct Kern {
+    void (*fn)(const uint16_t*, const void*, const float*, int, int, int, uint16_t*);
+    int rows, cols, steps;
+    double t0, t1;
+  };
+  // k_rows_gemm's four waves share the steps
+  const Kern kerns[] = {{esc::k_rows_gemm<Q8, 2>, 32, 64, (NS + 3) / 4, 0.0, 1.05},
+                        {esc::k_rows_gemm<Q8, 4>, 64, 64, (NS + 3) / 4, 0.0, 1.5},
+                        {esc::k_rows_gemm_lds<Q8, 4>, 64, 256, NS, 0.4, 0.75},
+                        {esc::k_rows_gemm_lds<Q8, 6>, 96, 256, NS, 0.6, 0.8},
+                        {esc::k_rows_gemm_lds<Q8, 8>, 128, 256, NS, 0.8, 1.0}};
+  const Kern* best = nullptr;
+  double best_cost = 0.0;
+  long best_blocks = 0;
+  for (const Kern& k : kerns) {
+    const long blocks = (long)((O + k.cols - 1) / k.cols) * ((M + k.rows - 1) / k.rows);
+    const double cost = (k.t0 + k.t1 * ((blocks + cus - 1) / cus)) * k.steps;
+    if (!best || cost < best_cost) best = &k, best_cost = cost, best_blocks = blocks;
+  }
+  ESC_REQUIRE(best_blocks < (1L << 31), "%d rows x %d channels is too large", M, O);
+  hipLaunchKernelGGL(best->fn, dim3((unsigned)best_blocks), dim3(256), 0, s, x, w, scale, M, K, O,
+                     y);
+  return launched("k_rows_gemm");
+}
+
 template <bool Q8>
 int rows_gemv(const uint16_t* x, const void* w, const float* scale, int M, int K, int O,
               uint16_t* y, hipStream_t s) {
@@ -1144,6 +1180,8 @@ int rows_gemv(const uint16_t* x, const void* w, const float* scale, int M, int K
   const int chunks = K / cw;
   ESC_REQUIRE(K > 0 && K % cw == 0 && chunks >= 8 && chunks <= 64 * kRowsMaxCpl,
               "K=%d: need a multiple of %d in [%d, %d]", K, cw, 8 * cw, 64 * kRowsMaxCpl * cw);
+  if (M >= (Q8 ? kRowsGemmRows : kRowsGemmRowsF16) && K % 64 == 0)
+    return rows_gemm<Q8>(x, w, scale, M, K, O, y, s);
   if constexpr (Q8) {
     if (const int nr = w8_mma_rows(M, K); nr >= 2) return rows_w8_mma(x, w, scale, M, K, O, y, nr, s);
   }

@@ -79,7 +79,7 @@ __global__ __launch_bounds__(256, 2) void k_moe_mma(MoeMmaArgs a) {
   }
   const __amdgpu_buffer_rsrc_t xrs = buf_rsrc(a.xh, (size_t)M * IC * 2);
   f32x4_t acc[D::NA][NRB];
-  mma2_loop<K, NRB>(cbase, kstride, xrs, xoff, 0, TK / 4, s_x, acc);
+  mma2_loop<NRB>(CodedCols<K>{cbase, kstride}, xrs, xoff, 0, TK / 4, s_x, acc);
 
   float4* so = kOwn ? s_o : reinterpret_cast<float4*>(&s_x[0][0]);
   const float rs = a.rs;

@@ -58,25 +58,48 @@ __device__ __forceinline__ uint32_t mma2_x_chunk(int tid, int j) {
   return 16u * ((e & 7) ^ ((e >> 3) & 7));
 }
 
-// The main loop over steps [s0, s1) (s1 > s0): acc[a][r] += the wave's 64
-// columns x row block r.  cbase: the lane's code words of the wave's first
-// tile at kt gk (lane / 16); xoff: byte offsets of the thread's x chunks.
-template <int K, int NRB>
-__device__ __forceinline__ void mma2_loop(const uint32_t* __restrict__ cbase, size_t kstride,
-                                          __amdgpu_buffer_rsrc_t xrs, const uint32_t* xoff, int s0,
-                                          int s1, uint4 (*s_x)[16 * NRB * 8],
-                                          f32x4_t (*acc)[NRB]) {
+// Where the main loop's A operands come from: 64 columns x 64 inputs a step, as
+// four 16-column groups of two operands each (input halves; lane l: column
+// l % 16, inputs 16 (l / 16) + 8 half ..).  Coded weights: cbase is the lane's
+// code words of the wave's first tile at kt gk (lane / 16).
+template <int K>
+struct CodedCols {
   using G = Geo<K>;
-  using D = Mma2<K, NRB>;
-  constexpr int TPS = D::TPS, GPW = D::GPW, NA = D::NA, XCH = D::XCH;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int gk = lane >> 4, c = lane & 15;
-  const int src = (lane & ~(G::LPT - 1)) | ((lane + G::LPT - 1) & (G::LPT - 1));
-  auto load_code = [&](LaneWords<K>* cw, int s) {
+  static constexpr int TPS = 16 / G::LPT, GPW = 4 / TPS;
+  struct Regs {
+    LaneWords<K> w[GPW];
+  };
+  const uint32_t* cbase;
+  size_t kstride;
+  __device__ __forceinline__ void load(Regs& r, int s) const {
 #pragma unroll
     for (int tg = 0; tg < GPW; ++tg)
-      cw[tg] = load_lane_words<K>(cbase + (size_t)tg * TPS * (8 * K) + (size_t)(4 * s) * kstride);
-  };
+      r.w[tg] = load_lane_words<K>(cbase + (size_t)tg * TPS * (8 * K) + (size_t)(4 * s) * kstride);
+  }
+  __device__ __forceinline__ void decode(const Regs& r, u32x4_t (*Ad)[2]) const {
+    const int lane = threadIdx.x & 63;
+    const int src = (lane & ~(G::LPT - 1)) | ((lane + G::LPT - 1) & (G::LPT - 1));
+#pragma unroll
+    for (int tg = 0; tg < GPW; ++tg) {
+      const uint32_t wprev = __shfl(r.w[tg].w[G::WPL - 1], src);
+#pragma unroll
+      for (int ci = 0; ci < G::NCOL; ++ci)
+#pragma unroll
+        for (int P = 0; P < 2; ++P)
+          Ad[tg * G::NCOL + ci][P] = mma_a_operand<K>(r.w[tg], wprev, ci, P);
+    }
+  }
+};
+
+// The main loop over steps [s0, s1) (s1 > s0): acc[a][r] += the wave's 64
+// columns x row block r.  xoff: byte offsets of the thread's x chunks.
+template <int NRB, typename Cols>
+__device__ __forceinline__ void mma2_loop(const Cols& cols, __amdgpu_buffer_rsrc_t xrs,
+                                          const uint32_t* xoff, int s0, int s1,
+                                          uint4 (*s_x)[16 * NRB * 8], f32x4_t (*acc)[NRB]) {
+  constexpr int NA = 4, XCH = NRB / 2;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int gk = lane >> 4, c = lane & 15;
   auto load_x = [&](uint4* xr, int s) {
 #pragma unroll
     for (int j = 0; j < XCH; ++j) {
@@ -96,30 +119,20 @@ __device__ __forceinline__ void mma2_loop(const uint32_t* __restrict__ cbase, si
   // software pipeline: the MFMAs of step s and the decode of step s+1 sit in
   // one straight-line body (the matrix pipe and the VALU overlap); loads past
   // the last step re-read it (in bounds, never used)
-  auto decode_step = [&](const LaneWords<K>* w, u32x4_t (*Ad)[2]) {
-#pragma unroll
-    for (int tg = 0; tg < GPW; ++tg) {
-      const uint32_t wprev = __shfl(w[tg].w[G::WPL - 1], src);
-#pragma unroll
-      for (int ci = 0; ci < G::NCOL; ++ci)
-#pragma unroll
-        for (int P = 0; P < 2; ++P) Ad[tg * G::NCOL + ci][P] = mma_a_operand<K>(w[tg], wprev, ci, P);
-    }
-  };
-  LaneWords<K> cw[GPW];
+  typename Cols::Regs cw;
   uint4 xr[XCH];
   u32x4_t A[NA][2];
-  load_code(cw, s0);
+  cols.load(cw, s0);
   load_x(xr, s0);
   store_x(xr, 0);
-  decode_step(cw, A);
-  load_code(cw, min(s0 + 1, s1 - 1));
+  cols.decode(cw, A);
+  cols.load(cw, min(s0 + 1, s1 - 1));
   lds_barrier();
   for (int s = s0; s < s1; ++s) {
     const int buf = (s - s0) & 1;
     load_x(xr, min(s + 1, s1 - 1));
-    LaneWords<K> cn[GPW];
-    load_code(cn, min(s + 2, s1 - 1));
+    typename Cols::Regs cn;
+    cols.load(cn, min(s + 2, s1 - 1));
     u32x4_t An[NA][2];
 #pragma unroll
     for (int P = 0; P < 2; ++P)
@@ -130,15 +143,14 @@ __device__ __forceinline__ void mma2_loop(const uint32_t* __restrict__ cbase, si
 #pragma unroll
         for (int a = 0; a < NA; ++a) acc[a][r] = mma16(A[a][P], b, acc[a][r]);
       }
-    decode_step(cw, An);
+    cols.decode(cw, An);
     store_x(xr, buf ^ 1);
 #pragma unroll
     for (int a = 0; a < NA; ++a) {
       A[a][0] = An[a][0];
       A[a][1] = An[a][1];
     }
-#pragma unroll
-    for (int tg = 0; tg < GPW; ++tg) cw[tg] = cn[tg];
+    cw = cn;
     lds_barrier();
   }
 }
@@ -372,7 +384,7 @@ __global__ __launch_bounds__(256, 2) void k_gemm_mma2(MmaArgs p) {
     s1 = NS * ((int)blockIdx.y + 1) / (int)gridDim.y;
   }
   f32x4_t acc[NA][NRB];
-  mma2_loop<K, NRB>(cbase, kstride, xrs, xoff, s0, s1, s_x, acc);
+  mma2_loop<NRB>(CodedCols<K>{cbase, kstride}, xrs, xoff, s0, s1, s_x, acc);
 
   if constexpr (MODE == kMmaMid) {
 #pragma unroll

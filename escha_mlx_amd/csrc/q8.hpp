@@ -16,7 +16,7 @@
 #pragma once
 
 #include "basic.hpp"
-#include "fast.hpp"
+#include "mfma.hpp"
 
 namespace esc {
 
@@ -233,6 +233,212 @@ __global__ __launch_bounds__(256) void k_rows_w8_mma(const uint16_t* __restrict_
         if (o < O) y[(size_t)j * ldy + o] = __builtin_bit_cast(uint16_t, to_f16(acc[r]));
       }
     }
+  }
+}
+
+// The A operands of 64 weight rows (channels) x 64 k a step, for k_rows_gemm and
+// (as mma2_loop's columns) k_rows_gemm_lds: lane l reads 16 weights of channels
+// 16a + l % 16 at k 16 (l / 16), converted per the contract (int8) or as they are.
+template <bool Q8>
+struct RowCols {
+  static constexpr int WL = Q8 ? 1 : 2;  // 16-byte loads per lane, channel and step
+  struct Regs {
+    uint4 w[4][WL];
+  };
+  const char* wb;
+  uint32_t wo[4];
+  float sc[4], ms[4];
+  __device__ __forceinline__ void load(Regs& r, int s) const {
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int i = 0; i < WL; ++i)
+        r.w[a][i] = *reinterpret_cast<const uint4*>(wb + (wo[a] + 64u * WL * s + 16u * i));
+  }
+  __device__ __forceinline__ void decode(const Regs& r, u32x4_t (*A)[2]) const {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      if constexpr (Q8) {
+        const uint32_t ww[4] = {r.w[a][0].x, r.w[a][0].y, r.w[a][0].z, r.w[a][0].w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          uint32_t p0, p1;
+          w8_to_f16x4(ww[i], sc[a], ms[a], p0, p1);
+          A[a][i >> 1][2 * (i & 1)] = p0;
+          A[a][i >> 1][2 * (i & 1) + 1] = p1;
+        }
+      } else {
+        A[a][0] = __builtin_bit_cast(u32x4_t, r.w[a][0]);
+        A[a][1] = __builtin_bit_cast(u32x4_t, r.w[a][WL - 1]);
+      }
+    }
+  }
+  // channels o0 + 64 wave + 16a + l % 16, clamped to the last one
+  __device__ __forceinline__ void init(const void* wv, const float* scale, int o0, int K, int O) {
+    const int lane = threadIdx.x & 63;
+    wb = static_cast<const char*>(wv) + (size_t)o0 * K * WL;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+      const int oc = min(16 * a + (lane & 15), O - 1 - o0);
+      wo[a] = (uint32_t)((oc * K + 16 * (lane >> 4)) * WL);
+      sc[a] = 0.f;
+      if constexpr (Q8) sc[a] = scale[o0 + oc];
+      ms[a] = -128.f * sc[a];
+    }
+  }
+};
+
+// Four consecutive channels o .. o + 3 of one row (f16).
+__device__ __forceinline__ void rows_store4(uint16_t* y, int row, int o, int O, const f32x4_t& v) {
+  uint16_t* d = y + (size_t)row * O + o;
+  if (o + 3 < O && O % 4 == 0) {
+    *reinterpret_cast<uint2*>(d) =
+        make_uint2(pack2(to_f16(v[0]), to_f16(v[1])), pack2(to_f16(v[2]), to_f16(v[3])));
+  } else {
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (o + i < O) d[i] = __builtin_bit_cast(uint16_t, to_f16(v[i]));
+  }
+}
+
+// Many rows on the matrix core: y[m][o] = f16(sum_k x[m][k] * wf[o][k]) for int8
+// weights (Q8: wf = f16(f32(w8) * scale[o]), the contract rounding) or f16 ones.
+// A workgroup is 16 NRB rows x 64 channels; its four waves split K (in steps of
+// 64) and run without a barrier: per step a lane reads 16 weights of each of
+// four channels (o0 + 16a + l % 16, k0 + 16 (l / 16)), which become two A operands
+// each, and 2 NRB B operands straight from x (row l % 16 of a row block, the same
+// k; x is small and shared by every column of workgroups, so it is L2 traffic).
+// The waves' sums meet in LDS in wave order, wave a finishing channels o0 + 16a.
+// Splitting K inside the workgroup, not the channels, keeps enough workgroups in
+// flight for the narrow projections (203 rows x 512 channels: 56 workgroups of
+// 8 steps) and needs no x staging.  Bound by the weights' conversion (about 2.5
+// VALU per weight and 16 NRB rows) and the matrix pipe.  Measured on MI355X: 1000
+// rows x 4096 channels, K = 2048: see rows_gemm.  K a multiple of 64, at most
+// 8192; grid ceil(O / 64) * ceil(M / (16 NRB)), column blocks fastest, block 256.
+template <bool Q8, int NRB>
+__global__ __launch_bounds__(256, 2) void k_rows_gemm(const uint16_t* __restrict__ x,
+                                                      const void* __restrict__ wv,
+                                                      const float* __restrict__ scale, int M,
+                                                      int K, int O, uint16_t* __restrict__ y) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int c = lane & 15, g = lane >> 4;
+  const int ncb = (O + 63) / 64;
+  const int o0 = (blockIdx.x % ncb) * 64, row0 = (blockIdx.x / ncb) * 16 * NRB;
+  const int NS = K / 64, s0 = NS * wave / 4, s1 = NS * (wave + 1) / 4;
+  // channels past O and rows past M read the last one and are not stored;
+  // uniform bases and 32-bit byte offsets (at most 128 rows of 16 KiB)
+  const char* xb = reinterpret_cast<const char*>(x + (size_t)row0 * K);
+  uint32_t xo[NRB];
+  RowCols<Q8> cols;
+  cols.init(wv, scale, o0, K, O);
+#pragma unroll
+  for (int r = 0; r < NRB; ++r)
+    xo[r] = (uint32_t)(min(16 * r + c, M - 1 - row0) * K + 16 * g) * 2u;
+  f32x4_t acc[4][NRB];
+#pragma unroll
+  for (int a = 0; a < 4; ++a)
+#pragma unroll
+    for (int r = 0; r < NRB; ++r) acc[a][r] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  if (s0 < s1) {
+    typename RowCols<Q8>::Regs w, wn;
+    cols.load(w, s0);
+    for (int s = s0; s < s1; ++s) {
+      constexpr int RB = NRB < 4 ? NRB : 4;  // row blocks whose B operands are held at once
+      uint4 b[RB][2];
+      auto load_b = [&](int r0) {
+#pragma unroll
+        for (int r = 0; r < RB; ++r) {
+          const uint4* p = reinterpret_cast<const uint4*>(xb + (xo[r0 + r] + 128u * s));
+          b[r][0] = p[0];
+          b[r][1] = p[1];
+        }
+      };
+      load_b(0);
+      cols.load(wn, min(s + 1, s1 - 1));
+      u32x4_t A[4][2];
+      cols.decode(w, A);
+#pragma unroll
+      for (int r0 = 0; r0 < NRB; r0 += RB) {
+        if (r0) load_b(r0);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int r = 0; r < RB; ++r)
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+              acc[a][r0 + r] =
+                  mma16(A[a][h], __builtin_bit_cast(u32x4_t, b[r][h]), acc[a][r0 + r]);
+      }
+      w = wn;
+    }
+  }
+  // rounds of up to four row blocks: every wave hands the channels of the
+  // others over and sums its own
+  constexpr int RR = NRB < 4 ? NRB : 4;
+  __shared__ f32x4_t s_acc[4][4][RR][64];  // [channel group][wave][row block][lane]
+#pragma unroll
+  for (int r0 = 0; r0 < NRB; r0 += RR) {
+    if (r0) __syncthreads();
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int r = 0; r < RR; ++r) s_acc[a][wave][r][lane] = acc[a][r0 + r];
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < RR; ++r) {
+      f32x4_t v = s_acc[wave][0][r][lane];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) {
+        const f32x4_t t = s_acc[wave][w][r][lane];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = v[i] + t[i];
+      }
+      // lane: row c of the block, channels o .. o + 3
+      const int row = row0 + 16 * (r0 + r) + c, o = o0 + 16 * wave + 4 * g;
+      if (row >= M) continue;
+      rows_store4(y, row, o, O, v);
+    }
+  }
+}
+
+// The same product where there are tiles enough to fill the chip: k_gemm_mma2's
+// main loop over int8 / f16 channels, a workgroup's four waves on 64 channels
+// each and x staged through LDS once for all of them (in k_rows_gemm every wave
+// reads its own x: 16 KiB per wave and step at 128 rows, more than the 64 B per
+// clock of a CU's L1).  K a multiple of 64; grid ceil(O / 256) * ceil(M / (16 NRB)),
+// column blocks fastest, block 256.
+template <bool Q8, int NRB>
+__global__ __launch_bounds__(256, 2) void k_rows_gemm_lds(const uint16_t* __restrict__ x,
+                                                          const void* __restrict__ wv,
+                                                          const float* __restrict__ scale, int M,
+                                                          int K, int O,
+                                                          uint16_t* __restrict__ y) {
+  constexpr int XCH = NRB / 2;
+  __shared__ uint4 s_x[2][16 * NRB * 8];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int ncb = (O + 255) / 256;
+  const int cb = blockIdx.x % ncb, row0 = (blockIdx.x / ncb) * 16 * NRB;
+  // a wave past the last channel runs the last one's and stores nothing
+  const int o0 = min(cb * 256 + 64 * wave, O - 1);
+  RowCols<Q8> cols;
+  cols.init(wv, scale, o0, K, O);
+  uint32_t xoff[XCH];
+#pragma unroll
+  for (int j = 0; j < XCH; ++j)
+    xoff[j] = 2u * (uint32_t)(min(mma2_x_row(tid, j), M - 1 - row0) * K) + mma2_x_chunk(tid, j);
+  const __amdgpu_buffer_rsrc_t xrs =
+      buf_rsrc(x + (size_t)row0 * K, (size_t)min(16 * NRB, M - row0) * K * 2);
+  f32x4_t acc[4][NRB];
+  mma2_loop<NRB>(cols, xrs, xoff, 0, K / 64, s_x, acc);
+  if (cb * 256 + 64 * wave >= O) return;
+  const int c = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int r = 0; r < NRB; ++r) {
+    const int row = row0 + 16 * r + c;
+    if (row >= M) continue;
+#pragma unroll
+    for (int a = 0; a < 4; ++a) rows_store4(y, row, o0 + 16 * a + 4 * g, O, acc[a][r]);
   }
 }
 

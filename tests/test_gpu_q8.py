@@ -163,3 +163,30 @@ def test_q8_embed_bit_exact(K):
     bad = emb(torch.tensor([0, N, -1, N - 1], device=DEV)).cpu().numpy()
     assert np.isnan(bad[1]).all() and np.isnan(bad[2]).all()
     assert np.array_equal(bad[[0, 3]].view(np.uint16), R.q8_embed(np.array([0, N - 1]), w8, scale).view(np.uint16))
+
+
+# ---- many rows (k_rows_gemm, k_rows_gemm_lds at 64, 96 and 128 rows): one row
+# past the smaller path, ragged rows and channels, few steps of K
+@pytest.mark.parametrize("m,K,O", [(17, 128, 97), (33, 2048, 512), (130, 192, 64), (203, 576, 66),
+                                   (500, 128, 4001), (260, 192, 20000), (700, 128, 8200)])
+@pytest.mark.parametrize("q8", [True, False], ids=["int8", "f16"])
+def test_many_rows_vs_f64(m, K, O, q8):
+    """Within the other w8a16 paths' 2e-3 of each row's largest float64 value
+    (f16 output, float32 sums), and one-hot rows bit-exact."""
+    rng = np.random.default_rng(m + K + O)
+    x = rng.standard_normal((m, K)).astype(np.float16)
+    x[0] = 0
+    x[0, K - 1] = 1.0  # one-hot: the output row is the weights' last column
+    if q8:
+        w8 = rng.integers(-128, 128, size=(O, K), dtype=np.int8)
+        scale = rng.uniform(0.5, 1.5, O).astype(np.float32) * 1e-2
+        wf = R.q8_dequant(w8, scale)
+        y = ops().w8a16(_dev(x), _dev(w8), _dev(scale))
+    else:
+        wf = (rng.standard_normal((O, K)) * 0.05).astype(np.float16)
+        y = ops().gemv_f16w(_dev(x), _dev(wf))
+    got = y.cpu().numpy()
+    want = x.astype(np.float64) @ wf.astype(np.float64).T
+    assert np.array_equal(got[0].view(np.uint16), wf[:, K - 1].view(np.uint16))
+    err = (np.abs(got - want).max(axis=1) / np.abs(want).max(axis=1)).max()
+    assert err < 2e-3, err
