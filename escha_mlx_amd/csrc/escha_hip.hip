@@ -1137,13 +1137,23 @@ int rows_w8_mma(const uint16_t* x, const void* w, const float* scale, int M, int
   return ESC_OK;
 }
 
-// The matrix-core GEMMs from kRowsGemmRows rows (kRowsGemmRowsF16 for f16
-// weights, whose GEMV takes 8 rows per launch) and K a multiple of 64.  The time
-// of a launch is that of the busiest CU: n workgroups on it take t0 + t1 n us per
-// step (fitted to a sweep of 7 kernels over 33 shapes, int8, on MI355X).  K = 2048,
-// whole call: 203 x 512 14.1 us (16 rows per launch: 153), 1000 x 4096 38 (852),
-// 2048 x 4096 61 (1743), 64 x 248320 144 (570).
-constexpr int kRowsGemmRows = 17, kRowsGemmRowsF16 = 9;
+// Whether the matrix-core GEMMs take a shape (K a multiple of 64).  f16 weights:
+// from 9 rows, where the GEMV needs a second launch.  int8: where k_rows_w8_mma
+// needs a second launch (its rows of x fill a workgroup's LDS), and below that for
+// long rows of few channels, which leave its workgroups (16 channels a wave, all of
+// K) latency-bound: whole call, K = 5120 to 5120 / 16384 channels, 2 rows 21 / 23 us
+// against 16 / 20, 8 rows 44 / 47 against 17 / 21; not for K <= 2048 (4096 channels
+// level, 248320 channels 104 us against 135).
+bool rows_gemm_takes(bool q8, int M, int K, int O) {
+  if (K % 64) return false;
+  if (!q8) return M > 8;
+  return M >= 2 && (M > w8_mma_rows(M, K) || (K >= 4096 && O <= 32768));
+}
+
+// The time of a launch is that of the busiest CU: n workgroups on it take t0 + t1 n
+// us per step (fitted to a sweep of 7 kernels over 33 shapes, int8, on MI355X).
+// K = 2048, whole call: 203 x 512 14.1 us (16 rows per launch: 153), 1000 x 4096 35
+// (852), 2048 x 4096 59 (1743), 64 x 248320 144 (570).
 template <bool Q8>
 int rows_gemm(const uint16_t* x, const void* w, const float* scale, int M, int K, int O,
               uint16_t* y, hipStream_t s) {
@@ -1180,7 +1190,7 @@ int rows_gemv(const uint16_t* x, const void* w, const float* scale, int M, int K
   const int chunks = K / cw;
   ESC_REQUIRE(K > 0 && K % cw == 0 && chunks >= 8 && chunks <= 64 * kRowsMaxCpl,
               "K=%d: need a multiple of %d in [%d, %d]", K, cw, 8 * cw, 64 * kRowsMaxCpl * cw);
-  if (M >= (Q8 ? kRowsGemmRows : kRowsGemmRowsF16) && K % 64 == 0)
+  if (rows_gemm_takes(Q8, M, K, O))
     return rows_gemm<Q8>(x, w, scale, M, K, O, y, s);
   if constexpr (Q8) {
     if (const int nr = w8_mma_rows(M, K); nr >= 2) return rows_w8_mma(x, w, scale, M, K, O, y, nr, s);
