@@ -100,6 +100,13 @@ constexpr int kTransformRows = 16;
 // Element types of the rows an input transform reads (esc_input_transform_typed).
 enum { kRowsF16 = 0, kRowsBF16 = 1, kRowsF32 = 2 };
 
+// One 16-bit row element as float32 (exact); dt is kRowsF16 or kRowsBF16.
+__device__ __forceinline__ float row_value16(uint16_t v, int dt) {
+  const float b = __builtin_bit_cast(float, (uint32_t)v << 16);
+  const float h = (float)__builtin_bit_cast(half_t, v);
+  return dt == kRowsBF16 ? b : h;
+}
+
 // Elements c, c + 1 of a row as float32 (exact for every type).
 template <int DT>
 __device__ __forceinline__ float2 row_pair(const void* rows, size_t i) {

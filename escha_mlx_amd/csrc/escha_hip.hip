@@ -1272,10 +1272,20 @@ namespace {
 constexpr int kMoeGroupRows = 8;
 int moe_group_rows(int M, int E) { return M >= E ? kMoeGroupRows : 0; }
 
-int moe_input(const uint16_t* x, const int32_t* ids, int top_k, const float* rin, int H, float rs,
-              uint16_t* xh, int M, hipStream_t s) {
-  hipLaunchKernelGGL(esc::k_moe_input, dim3(H / 128, M), dim3(64), 0, s, x, ids, top_k, rin, H, rs,
-                     xh);
+// f(std::integral_constant<int, DT>) for the row element type dtype.
+template <typename F>
+void by_rows_type(int dtype, F f) {
+  if (dtype == ESC_ROWS_BF16) f(std::integral_constant<int, esc::kRowsBF16>{});
+  else if (dtype == ESC_ROWS_F32) f(std::integral_constant<int, esc::kRowsF32>{});
+  else f(std::integral_constant<int, esc::kRowsF16>{});
+}
+
+int moe_input(const void* x, int dtype, const int32_t* ids, int top_k, const float* rin, int H,
+              float rs, uint16_t* xh, int M, hipStream_t s) {
+  by_rows_type(dtype, [&](auto dt) {
+    hipLaunchKernelGGL(esc::k_moe_input<decltype(dt)::value>, dim3(H / 128, M), dim3(64), 0, s, x,
+                       ids, top_k, rin, H, rs, xh);
+  });
   return launched("k_moe_input");
 }
 
@@ -1426,19 +1436,22 @@ int moe_mma(int K, int nrb, const esc::MoeMmaArgs& a, hipStream_t s) {
 }
 
 // k_moe_prep: the input transform of every routed row and the grouping.
-int moe_prep(const uint16_t* x, const int32_t* ids, int T, int top_k, const float* rin, int H,
-             float rs, uint16_t* xh, const MoePlan& p, int E, int* rows, int* gexp, int* nact,
-             hipStream_t s) {
+int moe_prep(const void* x, int dtype, const int32_t* ids, int T, int top_k, const float* rin,
+             int H, float rs, uint16_t* xh, const MoePlan& p, int E, int* rows, int* gexp,
+             int* nact, hipStream_t s) {
   // four slots per wave once that leaves eight waves per SIMD
   const bool four = (long)T * top_k * (H / 128) / 4 >= 32L * device_cus();
   const long waves = (long)(H / 128) * T * (four ? (top_k + 3) / 4 : top_k);
   const dim3 grid((unsigned)(1 + (waves + 15) / 16)), blk(1024);
-  if (four)
-    hipLaunchKernelGGL(esc::k_moe_prep<4>, grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh, p.M, E,
-                       p.R, p.n_groups, rows, gexp, nact);
-  else
-    hipLaunchKernelGGL(esc::k_moe_prep<1>, grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh, p.M, E,
-                       p.R, p.n_groups, rows, gexp, nact);
+  by_rows_type(dtype, [&](auto dt) {
+    constexpr int DT = decltype(dt)::value;
+    if (four)
+      hipLaunchKernelGGL((esc::k_moe_prep<4, DT>), grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh,
+                         p.M, E, p.R, p.n_groups, rows, gexp, nact);
+    else
+      hipLaunchKernelGGL((esc::k_moe_prep<1, DT>), grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh,
+                         p.M, E, p.R, p.n_groups, rows, gexp, nact);
+  });
   return launched("k_moe_prep");
 }
 
@@ -1762,8 +1775,8 @@ int esc_moe_set_spin_limit(int polls) {
 namespace {
 // The expert path on a given workspace; int_region > 0 puts every counter in
 // a fixed region at its start (see fused_plan).
-int moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scores, int T, int top_k,
-                    int E, int H, int I, const uint32_t* gu_code, const float* gu_rin,
+int moe_expert_path(const void* x, int dtype, const int32_t* ids, const float* scores, int T,
+                    int top_k, int E, int H, int I, const uint32_t* gu_code, const float* gu_rin,
                     const float* gu_rout, int K_gu, const uint32_t* dn_code, const float* dn_rin,
                     const float* dn_rout, int K_dn, int use_lut, uint16_t* y, void* ws,
                     size_t ws_bytes, size_t int_region, void* stream, bool one_launch = false) {
@@ -1775,7 +1788,8 @@ int moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scores, 
   if (int rc = check_proj(K_dn, I, H)) return rc;
   ESC_REQUIRE(T >= 0, "negative token count");
   if (T == 0) return ESC_OK;
-  if (fused_eligible(T, top_k, H, I)) {
+  // the item kernels read 16-bit rows; float32 rows take the chain
+  if (fused_eligible(T, top_k, H, I) && dtype != ESC_ROWS_F32) {
     // throughput_ok: two launches (gate_up items, down items + combine),
     // measured faster than the single persistent launch for one token-layer
     // on gfx950; otherwise (or when the caller asks for it) the single
@@ -1794,7 +1808,8 @@ int moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scores, 
     // word, outside every shape's counters, so a give-up of one call never
     // lands in the counters of a later call of another shape.
     if (int_region) p.status = reinterpret_cast<int*>(static_cast<char*>(ws) + int_region) - 1;
-    p.l0 = esc::MoeLayer{x, ids, scores, gu_code, gu_rin, gu_rout, dn_code, dn_rin, dn_rout, y};
+    p.xdt = dtype;
+    p.l0 = esc::MoeLayer{static_cast<const uint16_t*>(x), ids, scores, gu_code, gu_rin, gu_rout, dn_code, dn_rin, dn_rout, y};
     p.layers = nullptr;
     if (two) return launch_fused<true>(p, K_gu, K_dn, f.grid, S(stream));
     // only the single persistent launch waits across workgroups
@@ -1818,7 +1833,7 @@ int moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scores, 
   int* nact = reinterpret_cast<int*>(w + p.off_nact);
   if (p.R) {
     // input transform and expert grouping in one launch
-    if (int rc = moe_prep(x, ids, T, top_k, gu_rin, H, rs, xh, p, E, rows, gexp, nact, s)) return rc;
+    if (int rc = moe_prep(x, dtype, ids, T, top_k, gu_rin, H, rs, xh, p, E, rows, gexp, nact, s)) return rc;
     if (p.nrb) {
       uint16_t* d16 = reinterpret_cast<uint16_t*>(w + p.off_d16);
       esc::MoeMmaArgs a{xh, gu_code, rows, gexp, gu_rout, dn_rin, xh2, p.M, H / 16, 2 * I / 16,
@@ -1832,7 +1847,7 @@ int moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scores, 
     if (int rc = group_rows(K_gu, use_lut, p.R, xh, gu_code, rows, gexp, nact, p.n_groups, p.M,
                             H / 16, 2 * I / 16, p.S1, p1, s))
       return rc;
-  } else if (int rc = moe_input(x, ids, top_k, gu_rin, H, rs, xh, p.M, s)) {
+  } else if (int rc = moe_input(x, dtype, ids, top_k, gu_rin, H, rs, xh, p.M, s)) {
     return rc;
   } else if (int rc = by_k_lut<FastF>(K_gu, use_lut, xh, gu_code, ids, p.M, H / 16, 2 * I / 16,
                                       p.S1, p1, s)) {
@@ -1926,8 +1941,22 @@ int esc_moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scor
                         const uint32_t* dn_code, const float* dn_rin, const float* dn_rout,
                         int K_dn, int use_lut, uint16_t* y, void* ws, size_t ws_bytes,
                         void* stream) {
+  return esc_moe_expert_path_typed(x, ESC_ROWS_F16, ids, scores, T, top_k, E, H, I, gu_code, gu_rin,
+                                   gu_rout, K_gu, dn_code, dn_rin, dn_rout, K_dn, use_lut, y, ws,
+                                   ws_bytes, stream);
+}
+
+int esc_moe_expert_path_typed(const void* x, int dtype, const int32_t* ids, const float* scores,
+                              int T, int top_k, int E, int H, int I, const uint32_t* gu_code,
+                              const float* gu_rin, const float* gu_rout, int K_gu,
+                              const uint32_t* dn_code, const float* dn_rin, const float* dn_rout,
+                              int K_dn, int use_lut, uint16_t* y, void* ws, size_t ws_bytes,
+                              void* stream) {
+  ESC_REQUIRE(dtype == ESC_ROWS_F16 || dtype == ESC_ROWS_BF16 || dtype == ESC_ROWS_F32,
+              "row element type must be ESC_ROWS_F16, ESC_ROWS_BF16 or ESC_ROWS_F32, got %d",
+              dtype);
   if (int rc = ensure_wait_flag()) return rc;
-  return moe_expert_path(x, ids, scores, T, top_k, E, H, I, gu_code, gu_rin, gu_rout, K_gu,
+  return moe_expert_path(x, dtype, ids, scores, T, top_k, E, H, I, gu_code, gu_rin, gu_rout, K_gu,
                          dn_code, dn_rin, dn_rout, K_dn, use_lut, y, ws, ws_bytes, 0, stream);
 }
 
@@ -1945,8 +1974,8 @@ int esc_moe_expert_path_one_launch(const uint16_t* x, const int32_t* ids, const 
               "up to 7936 and I a multiple of 128 (got T=%d top_k=%d H=%d I=%d)",
               kFusedMaxRows, T, top_k, H, I);
   if (int rc = ensure_wait_flag()) return rc;
-  return moe_expert_path(x, ids, scores, T, top_k, E, H, I, gu_code, gu_rin, gu_rout, K_gu,
-                         dn_code, dn_rin, dn_rout, K_dn, use_lut, y, ws, ws_bytes, 0, stream,
+  return moe_expert_path(x, ESC_ROWS_F16, ids, scores, T, top_k, E, H, I, gu_code, gu_rin, gu_rout,
+                         K_gu, dn_code, dn_rin, dn_rout, K_dn, use_lut, y, ws, ws_bytes, 0, stream,
                          true);
 }
 
@@ -1975,8 +2004,8 @@ int esc_moe_expert_path_static(const uint16_t* x, const int32_t* ids, const floa
   }
   void* ptr = nullptr;
   if (int rc = ensure_scratch(&ptr)) return rc;
-  return moe_expert_path(x, ids, scores, T, top_k, E, H, I, gu_code, gu_rin, gu_rout, K_gu,
-                         dn_code, dn_rin, dn_rout, K_dn, use_lut, y, ptr, kStaticScratchBytes,
+  return moe_expert_path(x, ESC_ROWS_F16, ids, scores, T, top_k, E, H, I, gu_code, gu_rin, gu_rout,
+                         K_gu, dn_code, dn_rin, dn_rout, K_dn, use_lut, y, ptr, kStaticScratchBytes,
                          kStaticIntBytes, stream);
 }
 

@@ -116,6 +116,7 @@ struct FusedMoe {
   int* host_err; // device-wide flag in pinned host memory: a spin bound was hit
                  // (the next expert-path call on the device reports it)
   int spin_limit;  // polls before a wait gives up (kSpinLimit; the host may lower it)
+  int xdt;         // element type of the layers' x: kRowsF16 or kRowsBF16
   int L, T, top_k, H, I;
   int NB;   // I / 128        h-blocks
   int NKC;  // H / (16*KTA)   gate_up items per (row, h-block), <= 62
@@ -334,7 +335,7 @@ __device__ __forceinline__ void publish_gate_up(const FusedMoe& p, int l, int a)
 // The inputs of gate_up item a that wave `wave` < KTA/8 transforms: its two
 // values of x and their two input scales.
 struct GateUpIn {
-  half_t x0, x1;
+  uint16_t x0, x1;  // f16 or bf16 bits (FusedMoe::xdt)
   float r0, r1;
 };
 
@@ -348,8 +349,8 @@ __device__ __forceinline__ GateUpIn gate_up_in(const FusedMoe& p, const MoeLayer
     const int c = 16 * KTA * kc + 128 * wave + 2 * lane;
     const auto* xr = as_global(L.x + (size_t)t * p.H + c);
     const auto* ri = as_global(L.gu_rin + (size_t)e * p.H + c);
-    in.x0 = __builtin_bit_cast(half_t, xr[0]);
-    in.x1 = __builtin_bit_cast(half_t, xr[1]);
+    in.x0 = xr[0];
+    in.x1 = xr[1];
     in.r0 = ri[0];
     in.r1 = ri[1];
   }
@@ -359,11 +360,12 @@ __device__ __forceinline__ GateUpIn gate_up_in(const FusedMoe& p, const MoeLayer
 // Input transform of the item's 16*KTA inputs (one wave per 128-block) into
 // s_x as decode input pairs.
 template <int KTA>
-__device__ __forceinline__ void gate_up_transform(const GateUpIn& in, uint32_t* s_x) {
+__device__ __forceinline__ void gate_up_transform(const FusedMoe& p, const GateUpIn& in,
+                                                  uint32_t* s_x) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   if (wave < KTA / 8) {
-    float v0 = (float)in.x0 * in.r0;
-    float v1 = (float)in.x1 * in.r1;
+    float v0 = row_value16(in.x0, p.xdt) * in.r0;
+    float v1 = row_value16(in.x1, p.xdt) * in.r1;
     h128_wave(v0, v1);
     s_x[64 * wave + lane] = paired_word(pack2(to_f16(v0 * kRS), to_f16(v1 * kRS)));
   }
@@ -372,7 +374,7 @@ __device__ __forceinline__ void gate_up_transform(const GateUpIn& in, uint32_t* 
 template <int K, int KTA, bool PUBLISH = true, bool COH = true, int NW = 4>
 __device__ void run_gate_up(const FusedMoe& p, int l, int a, const ItemCode<K, KTA, NW>& code,
                             uint32_t* s_x, float (*s_red)[64][4]) {
-  gate_up_transform<KTA>(gate_up_in<KTA>(p, p.layer(l), a), s_x);
+  gate_up_transform<KTA>(p, gate_up_in<KTA>(p, p.layer(l), a), s_x);
   __syncthreads();
   compute_item<K, KTA, PUBLISH, COH, true, NW>(code, s_x, s_red,
                                               p.partA + ((size_t)l * p.nA + a) * 256);
@@ -628,7 +630,7 @@ __global__ __launch_bounds__(64 * NW) void k_moe_gate_up_items(FusedMoe p) {
     const auto code = load_gate_up<KG, KTA, NW>(p, L, a);
     const GateUpIn in = gate_up_in<KTA>(p, L, a);
     const auto w = decode_item<KG, KTA, NW>(code);
-    gate_up_transform<KTA>(in, s_x);
+    gate_up_transform<KTA>(p, in, s_x);
     __syncthreads();
     compute_item<KG, KTA, false, false, true, NW>(w, s_x, s_red, p.partA + (size_t)a * 256);
   } else {

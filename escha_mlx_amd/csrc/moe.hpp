@@ -8,19 +8,20 @@
 
 namespace esc {
 
-// xh[row] = f16(H128(f32(x[tok]) * rin[ids[row]]) * RS), 128-block blk of the
+// xh[row] = f16(H128(f32(x[tok]) * rin[ids[row]]) * RS) (DT: x's element type,
+// converted exactly to float32), 128-block blk of the
 // rows row = tok * top_k + s of up to NS slots s from s0 of one token, by one
 // wave: the token's inputs are read once, every slot's scales are requested
 // before any is used (slots past the last re-read it and store nothing).
-template <int NS>
-__device__ __forceinline__ void moe_input_wave(const uint16_t* __restrict__ x,
+template <int NS, int DT>
+__device__ __forceinline__ void moe_input_wave(const void* __restrict__ x,
                                                const int* __restrict__ ids, int top_k,
                                                const float* __restrict__ rin, int H, float rs,
                                                uint16_t* __restrict__ xh, int blk, int tok,
                                                int s0) {
   const int lane = threadIdx.x & 63;
   const int c = blk * 128 + 2 * lane, row0 = tok * top_k + s0, n = top_k - s0;
-  const float2 xv = row_pair<kRowsF16>(x, (size_t)tok * H + c);
+  const float2 xv = row_pair<DT>(x, (size_t)tok * H + c);
   float2 r[NS];
 #pragma unroll
   for (int j = 0; j < NS; ++j)
@@ -36,12 +37,13 @@ __device__ __forceinline__ void moe_input_wave(const uint16_t* __restrict__ x,
 }
 
 // grid (H/128, T*k), block 64.
-__global__ __launch_bounds__(64) void k_moe_input(const uint16_t* __restrict__ x,
+template <int DT>
+__global__ __launch_bounds__(64) void k_moe_input(const void* __restrict__ x,
                                                   const int* __restrict__ ids, int top_k,
                                                   const float* __restrict__ rin, int H, float rs,
                                                   uint16_t* __restrict__ xh) {
   const int row = blockIdx.y, tok = row / top_k;
-  moe_input_wave<1>(x, ids, top_k, rin, H, rs, xh, blockIdx.x, tok, row - tok * top_k);
+  moe_input_wave<1, DT>(x, ids, top_k, rin, H, rs, xh, blockIdx.x, tok, row - tok * top_k);
 }
 
 // The chain's two independent first steps in one launch: block 0 groups the
@@ -50,8 +52,8 @@ __global__ __launch_bounds__(64) void k_moe_input(const uint16_t* __restrict__ x
 // (a token's inputs and ids read once per four slots, 4-byte accesses) where
 // the rows fill the GPU all the same; NS = 1 below that.  grid
 // 1 + ceil(H/128 * T * ceil(top_k/NS) / 16), block 1024.
-template <int NS>
-__global__ __launch_bounds__(1024) void k_moe_prep(const uint16_t* __restrict__ x,
+template <int NS, int DT>
+__global__ __launch_bounds__(1024) void k_moe_prep(const void* __restrict__ x,
                                                    const int* __restrict__ ids, int top_k,
                                                    const float* __restrict__ rin, int H, float rs,
                                                    uint16_t* __restrict__ xh, int m, int E, int R,
@@ -66,7 +68,7 @@ __global__ __launch_bounds__(1024) void k_moe_prep(const uint16_t* __restrict__ 
   const int w = __builtin_amdgcn_readfirstlane((blockIdx.x - 1) * 16 + (threadIdx.x >> 6));
   const int p = w / nhb, tok = p / ns;  // (token, slots), blk fastest
   if (tok < m / top_k)
-    moe_input_wave<NS>(x, ids, top_k, rin, H, rs, xh, w % nhb, tok, (p - tok * ns) * NS);
+    moe_input_wave<NS, DT>(x, ids, top_k, rin, H, rs, xh, w % nhb, tok, (p - tok * ns) * NS);
 }
 
 // The grouped split-K GEMM of k_gemv_fast_rows with the table decode, as a

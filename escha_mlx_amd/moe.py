@@ -156,25 +156,25 @@ class EschaMoEExperts(torch.nn.Module):
 
     def forward(self, x: torch.Tensor, ids: torch.Tensor, scores: torch.Tensor) -> torch.Tensor:
         """y f16 [T, H], the routed sum rounded to f16 (models/qwen3_5_moe.py:253).
-        x f16 takes the fused expert path; bf16 / f32 rows are transformed from
-        their float32 values (models/qwen3_5_moe.py:103-110), then the staged
-        chain runs."""
+        bf16 / f32 rows are transformed from their float32 values
+        (models/qwen3_5_moe.py:103-110)."""
         x = ops.as_rows(x)
         ids = ids.to(torch.int32).contiguous()
         scores = scores.to(torch.float32).contiguous()
-        if x.dtype != torch.float16:
-            return self._forward_staged(x, ids, scores, exact=self._exact)
         if self._exact or not self._fused_had:
             # ESCHA_MLX_FUSED_HAD off: every transform is its own launch around
             # the GEMVs (models/qwen3_5_moe.py:103-122), the staged chain
-            return self._forward_staged(x, ids, scores)
+            return self._forward_staged(x, ids, scores,
+                                        exact=self._exact or x.dtype == torch.float16)
         t, h = x.shape
         # ESCHA_HIP_MOE_ONE_LAUNCH: one launch wherever that launch takes the shape
-        one = self._one_launch and ops.moe_one_launch_takes(t, self.top_k, h, self._inter)
+        one = (self._one_launch and x.dtype == torch.float16
+               and ops.moe_one_launch_takes(t, self.top_k, h, self._inter))
         # one zero-initialised workspace per token count and form: the one-launch
         # path keeps its counters there and leaves them zero after every call,
         # and the two forms lay their counters out differently
-        key = (t, x.device, one)
+        # (float32 rows take the chain, which keeps none, at every shape)
+        key = (t, x.device, "chain" if x.dtype == torch.float32 else one)
         ws = self._ws.get(key)
         if ws is None:
             need = ops.moe_expert_path_workspace(t, self.top_k, self.num_experts, h, self._inter)

@@ -316,6 +316,18 @@ int esc_moe_expert_path(const uint16_t* x, const int32_t* ids, const float* scor
                         int K_dn, int use_lut, uint16_t* y, void* ws, size_t ws_bytes,
                         void* stream);
 
+/* esc_moe_expert_path for rows x of another element type (ESC_ROWS_*), transformed
+ * from their exact float32 values (escha_mlx/models/qwen3_5_moe.py:103-110);
+ * same workspace size, y f16.  float32 rows take the split-K or grouped chain at
+ * every shape, which leaves floats where the other paths keep counters: a ws moved
+ * from float32 rows to others is zero-filled again. */
+int esc_moe_expert_path_typed(const void* x, int dtype, const int32_t* ids, const float* scores,
+                              int T, int top_k, int E, int H, int I, const uint32_t* gu_code,
+                              const float* gu_rin, const float* gu_rout, int K_gu,
+                              const uint32_t* dn_code, const float* dn_rin, const float* dn_rout,
+                              int K_dn, int use_lut, uint16_t* y, void* ws, size_t ws_bytes,
+                              void* stream);
+
 /* esc_moe_expert_path as one persistent launch at every shape it takes
  * (T*top_k <= 64, top_k <= 32, H a multiple of 256 up to 7936, I a multiple
  * of 128; others return ESC_EINVAL): gate_up items, the SwiGLU hand-off,

@@ -144,3 +144,30 @@ def test_moe_experts_typed_rows(dtype, exact, monkeypatch):
             np.abs(want.astype(np.float32)).max() < 5e-3
     if dtype == torch.float32:
         assert not torch.equal(blk(x.half(), ids, sc), y)
+
+
+# the item kernels (two launches; one persistent launch at H = 256), the per-row
+# and the grouped split-K chains, and the grouped GEMM
+@pytest.mark.parametrize("E,H,I,T,k", [(16, 512, 512, 2, 4), (16, 256, 128, 2, 4), (256, 256, 128, 20, 4),
+                                       (32, 256, 128, 20, 4), (4, 384, 128, 24, 2)],
+                         ids=["two_launch", "one_launch", "per_row", "grouped", "grouped_gemm"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32], ids=["bf16", "f32"])
+def test_moe_experts_typed_paths(E, H, I, T, k, dtype, monkeypatch):
+    """Every route of the expert path on bf16 / f32 rows against the oracle on the
+    same float32 rows (5e-3 of the max, as the f16 rows); repeatable, and rows that
+    are exact in f16 give the f16 call's bits where both take the same kernels."""
+    K_gu, K_dn = 2, 3
+    c = _moe_case(E, H, I, K_gu, K_dn, T, k, 400 + E + T)
+    rng = np.random.default_rng(401)
+    v, x = _rows(rng, (T, H), dtype)
+    c = dict(c, x=v)
+    blk = _block(c, E, k, K_gu, K_dn, monkeypatch, False)
+    ids, sc = ops().route_topk(torch.from_numpy(c["logits"]).to(DEV), k)
+    y = blk(x, ids, sc)
+    ids_np, sc_np = ids.cpu().numpy(), sc.cpu().numpy()
+    want = _oracle_moe(c, ids_np, sc_np, E, H, I, K_gu, K_dn, np.unique(ids_np)).astype(np.float32)
+    assert np.abs(y.cpu().numpy().astype(np.float32) - want).max() / np.abs(want).max() < 5e-3
+    assert torch.equal(blk(x, ids, sc), y)
+    x16 = x.half()
+    if dtype == torch.bfloat16 or T * k > 64:
+        assert torch.equal(blk(x16.to(dtype), ids, sc), blk(x16.to(dtype).half(), ids, sc))
