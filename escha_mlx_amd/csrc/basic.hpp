@@ -1,15 +1,9 @@
-// Table build, tile decode, 128-point transforms, router top-k, row grouping.
+// Tile decode, 128-point transforms, router top-k, row grouping.
 #pragma once
 
 #include "codec.hpp"
 
 namespace esc {
-
-// ---------------------------------------------------------------- table
-__global__ __launch_bounds__(256) void k_lut_init() {
-  uint32_t s = blockIdx.x * 256u + threadIdx.x;
-  g_lut[s] = decode_hash_bits(s);
-}
 
 // ---------------------------------------------------------------- decode
 // code [TK][TN][8K] -> w [IC][OC] f16 (escha_mlx/msl.py:183-202, ref.py:126-134).
@@ -22,7 +16,7 @@ __global__ __launch_bounds__(256) void k_decode_tiles(const uint32_t* __restrict
   const int t = threadIdx.x;
   const uint32_t* wp = code + (size_t)tile * (8 * K);
   uint32_t s = step_state<K>([&](int i) { return wp[i]; }, t);
-  uint16_t v = LUT ? g_lut[s] : decode_hash_bits(s);
+  uint16_t v = LUT ? g_lut.v[s] : decode_hash_bits(s);
   w[(size_t)(16 * kt + step_row(t)) * OC + 16 * nt + step_col(t)] = v;
 }
 
@@ -129,32 +123,48 @@ __device__ __forceinline__ float2 row_pair(const void* rows, size_t i) {
 // f32 rows the reference's unfused branch (escha_mlx/dense.py:290-292,
 // models/qwen3_5_moe.py:108-110), converted exactly to float32 here with no
 // f16 rounding before the transform.
-template <int DT>
+// TWO: the rows are read once for two projections (rin / out and rin1 / out1).
+template <int DT, bool TWO = false>
 __global__ __launch_bounds__(256) void k_input_transform(const void* __restrict__ rows,
                                                          const float* __restrict__ rin,
                                                          const int* __restrict__ row_expert,
                                                          int m, int IC, float rs,
-                                                         uint16_t* __restrict__ out) {
+                                                         uint16_t* __restrict__ out,
+                                                         const float* __restrict__ rin1 = nullptr,
+                                                         uint16_t* __restrict__ out1 = nullptr) {
   constexpr int RPW = kTransformRows / 4;
   const int blk = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int c = blk * 128 + 2 * lane;
   const int row0 = blockIdx.y * kTransformRows + RPW * wave;
+  float2 xv[RPW];
   float v[RPW][2];
 #pragma unroll
   for (int j = 0; j < RPW; ++j) {
     const int row = min(row0 + j, m - 1);
-    const float2 xv = row_pair<DT>(rows, (size_t)row * IC + c);
+    xv[j] = row_pair<DT>(rows, (size_t)row * IC + c);
     const float* r = rin + (row_expert ? (size_t)row_expert[row] * IC : 0) + c;
-    v[j][0] = xv.x * r[0];
-    v[j][1] = xv.y * r[1];
+    v[j][0] = xv[j].x * r[0];
+    v[j][1] = xv[j].y * r[1];
   }
+  auto finish = [&](uint16_t* o) {
 #pragma unroll
-  for (int j = 0; j < RPW; ++j) {
-    h128_wave(v[j][0], v[j][1]);
-    if (row0 + j < m)
-      *reinterpret_cast<uint32_t*>(out + (size_t)(row0 + j) * IC + c) =
-          (uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[j][0] * rs)) |
-          ((uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[j][1] * rs)) << 16);
+    for (int j = 0; j < RPW; ++j) {
+      h128_wave(v[j][0], v[j][1]);
+      if (row0 + j < m)
+        *reinterpret_cast<uint32_t*>(o + (size_t)(row0 + j) * IC + c) =
+            (uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[j][0] * rs)) |
+            ((uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[j][1] * rs)) << 16);
+    }
+  };
+  finish(out);
+  if constexpr (TWO) {
+    const float r0 = rin1[c], r1 = rin1[c + 1];
+#pragma unroll
+    for (int j = 0; j < RPW; ++j) {
+      v[j][0] = xv[j].x * r0;
+      v[j][1] = xv[j].y * r1;
+    }
+    finish(out1);
   }
 }
 
@@ -201,62 +211,89 @@ __global__ __launch_bounds__(256) void k_output_transform(const float* __restric
 }
 
 // ---------------------------------------------------------------- router
+// The wave's largest value in every lane (v_max_f32 over DPP moves and the two
+// row swaps; no LDS round trip).
+__device__ __forceinline__ float wave_max(float v) {
+  v = fmaxf(v, lane_xor<1>(v));
+  v = fmaxf(v, lane_xor<2>(v));
+  v = fmaxf(v, lane_xor<4>(v));
+  v = fmaxf(v, lane_xor<8>(v));
+  const unsigned x = __builtin_bit_cast(unsigned, v);
+  const auto p = __builtin_amdgcn_permlane16_swap(x, x, false, false);
+  const unsigned p0 = p[0], p1 = p[1];
+  v = fmaxf(__builtin_bit_cast(float, p0), __builtin_bit_cast(float, p1));
+  const unsigned y = __builtin_bit_cast(unsigned, v);
+  const auto q = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+  const unsigned q0 = q[0], q1 = q[1];
+  return fmaxf(__builtin_bit_cast(float, q0), __builtin_bit_cast(float, q1));
+}
+
+// The top_k of one token's E logits by one wave (NPER = ceil(E / 64) values per
+// lane, NaN never chosen): lane k holds the k-th id and value, descending, ties to
+// the lower id.  Each pick is a lane-local scan, one wave maximum and a ballot of
+// the lanes that hold it (a shuffle reduction of (value, id) pairs waits on twelve
+// LDS round trips per pick: 9.5 us for 8 of 256, against 3 us).
+template <int NPER>
+__device__ __forceinline__ void topk_wave(float (&v)[NPER], int E, int top_k, int& my_id,
+                                          float& my_v) {
+  const int lane = threadIdx.x & 63;
+  my_id = 0;
+  my_v = 0.f;
+  for (int k = 0; k < top_k; ++k) {
+    float bv = -__builtin_inff();
+    int bi = 0x7fffffff;
+#pragma unroll
+    for (int i = 0; i < NPER; ++i) {
+      const int e = lane + 64 * i;
+      // ids grow with i: a tie keeps the earlier one
+      if (e < E && (v[i] > bv || (v[i] == bv && bi == 0x7fffffff))) {
+        bv = v[i];
+        bi = e;
+      }
+    }
+    const float m = wave_max(bv);
+    unsigned long long ties = __ballot(bv == m && bi != 0x7fffffff);
+    int id = 0x7fffffff;
+    while (ties) {  // the lowest id among the lanes that hold the maximum
+      const int l = __builtin_ctzll(ties);
+      id = min(id, __builtin_amdgcn_readlane(bi, l));
+      ties &= ties - 1;
+    }
+    if (lane == k) {
+      my_id = id;
+      my_v = m;
+    }
+#pragma unroll
+    for (int i = 0; i < NPER; ++i)
+      if (lane + 64 * i == id) v[i] = -__builtin_inff();
+  }
+}
+
 // logits [T][E] f32 -> ids [T][k] (descending, ties -> lower id), scores [T][k]
 // = softmax over the k selected logits (escha_mlx/ref.py:326-331).
-// One wave per token; E <= 1024 held as 16 values per lane.
+// One wave per token; E <= 64 NPER.
+template <int NPER>
 __global__ __launch_bounds__(64) void k_route_topk(const float* __restrict__ logits, int E,
                                                    int top_k, int* __restrict__ ids,
                                                    float* __restrict__ scores) {
   const int tok = blockIdx.x, lane = threadIdx.x;
   const float* lg = logits + (size_t)tok * E;
-  constexpr int kPer = 16;
-  float v[kPer];
+  float v[NPER];
 #pragma unroll
-  for (int i = 0; i < kPer; ++i) {
-    int e = lane + 64 * i;
-    v[i] = e < E ? lg[e] : -__builtin_inff();
-  }
-  float top0 = 0.f, sel[32];
-  int selid[32];
-  for (int k = 0; k < top_k; ++k) {
-    // lane-local best (value desc, id asc)
-    float bv = -__builtin_inff();
-    int bi = 0x7fffffff;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      int e = lane + 64 * i;
-      if (e < E && (v[i] > bv || (v[i] == bv && e < bi))) {
-        bv = v[i];
-        bi = e;
-      }
-    }
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-      float ov = __shfl_xor(bv, m);
-      int oi = __shfl_xor(bi, m);
-      if (ov > bv || (ov == bv && oi < bi)) {
-        bv = ov;
-        bi = oi;
-      }
-    }
-    sel[k] = bv;
-    selid[k] = bi;
-    if (k == 0) top0 = bv;
-#pragma unroll
-    for (int i = 0; i < kPer; ++i)
-      if (lane + 64 * i == bi) v[i] = -__builtin_inff();
-  }
-  if (lane == 0) {
-    float den = 0.f;
-    float ex[32];
-    for (int k = 0; k < top_k; ++k) {
-      ex[k] = expf(sel[k] - top0);
-      den += ex[k];
-    }
-    for (int k = 0; k < top_k; ++k) {
-      ids[(size_t)tok * top_k + k] = selid[k];
-      scores[(size_t)tok * top_k + k] = ex[k] / den;
-    }
+  for (int i = 0; i < NPER; ++i) v[i] = lg[min(lane + 64 * i, E - 1)];
+  int id;
+  float val;
+  topk_wave(v, E, top_k, id, val);
+  const float top0 =
+      __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, val), 0));
+  const float ex = expf(val - top0);
+  // the denominator in slot order
+  float den = 0.f;
+  for (int k = 0; k < top_k; ++k)
+    den += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, ex), k));
+  if (lane < top_k) {
+    ids[(size_t)tok * top_k + lane] = id;
+    scores[(size_t)tok * top_k + lane] = ex / den;
   }
 }
 

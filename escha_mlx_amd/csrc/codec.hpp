@@ -94,10 +94,24 @@ __device__ __forceinline__ uint32_t step_state(WordFn w, int t) {
   return window16(w(a), w((a + 1) % kWords), start & 31);
 }
 
-// Table decode: 65,536 f16 values, built on the device by the hash itself
-// (bit-identical by construction) and staged through LDS by the kernels that
-// use it.  One copy per device, filled once by esc_init().
-__device__ uint16_t g_lut[65536];
+// Table decode: the 65,536 values of the hash, computed when the library is
+// compiled and part of its device image, so any kernel may read them from its
+// first launch on (no set-up launch, no synchronisation); staged through LDS by
+// the kernels that use it.
+struct DecodeTable {
+  uint16_t v[65536];
+};
+constexpr DecodeTable make_decode_table() {
+  DecodeTable t{};
+  for (uint32_t s = 0; s < 65536; ++s) {
+    const uint32_t r = ((s * kHashMul) & kHashMask) ^ kHashXor;
+    const half_t lo = __builtin_bit_cast(half_t, (uint16_t)(r & 0xFFFFu));
+    const half_t hi = __builtin_bit_cast(half_t, (uint16_t)(r >> 16));
+    t.v[s] = __builtin_bit_cast(uint16_t, (half_t)(lo + hi));
+  }
+  return t;
+}
+__device__ DecodeTable g_lut = make_decode_table();
 
 // Copying the table into LDS: 8,192 pieces of 16 bytes.  A load-then-store
 // loop waits one round trip to L2 per piece a thread copies; these issue
@@ -105,7 +119,7 @@ __device__ uint16_t g_lut[65536];
 // 1024) waits 1024 / B round trips.
 constexpr int kTablePieces = 65536 / 8;
 __device__ __forceinline__ void copy_table(uint16_t* s_dst) {
-  const uint4* src = reinterpret_cast<const uint4*>(g_lut);
+  const uint4* src = reinterpret_cast<const uint4*>(g_lut.v);
   uint4* dst = reinterpret_cast<uint4*>(s_dst);
   const int nt = blockDim.x;
   for (int i0 = threadIdx.x; i0 < kTablePieces; i0 += 8 * nt) {
@@ -123,7 +137,7 @@ struct TablePieces {
   uint4 v[8];
 };
 __device__ __forceinline__ void table_fetch(TablePieces& t) {
-  const uint4* src = reinterpret_cast<const uint4*>(g_lut);
+  const uint4* src = reinterpret_cast<const uint4*>(g_lut.v);
 #pragma unroll
   for (int k = 0; k < 8; ++k) t.v[k] = src[threadIdx.x + 1024 * k];
 }
@@ -141,7 +155,7 @@ __device__ __forceinline__ void table_put(const TablePieces& t, uint16_t* s_dst)
 __device__ __forceinline__ void table_dma(uint16_t* s_dst) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const char* src = reinterpret_cast<const char*>(g_lut);
+  const char* src = reinterpret_cast<const char*>(g_lut.v);
   char* dst = reinterpret_cast<char*>(s_dst);
 #pragma unroll
   for (int k = 0; k < 8; ++k) {

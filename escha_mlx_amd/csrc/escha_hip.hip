@@ -55,15 +55,14 @@ constexpr int kMaxDevices = 64;
 std::mutex g_init_mu;
 bool g_lut_ready[kMaxDevices];
 
+// The decode table is part of the device image; this records that a table
+// decode was asked for on the device (esc_moe_expert_path_static asks that
+// esc_init or such a call came first).
 int ensure_lut() {
   int dev = 0;
   if (int rc = hip_check(hipGetDevice(&dev), "hipGetDevice")) return rc;
   if (dev < 0 || dev >= kMaxDevices) return fail(ESC_EINVAL, "device index %d out of range", dev);
   std::lock_guard<std::mutex> lk(g_init_mu);
-  if (g_lut_ready[dev]) return ESC_OK;
-  hipLaunchKernelGGL(esc::k_lut_init, dim3(256), dim3(256), 0, 0);
-  if (int rc = launched("k_lut_init")) return rc;
-  if (int rc = hip_check(hipDeviceSynchronize(), "esc_init sync")) return rc;
   g_lut_ready[dev] = true;
   return ESC_OK;
 }
@@ -209,6 +208,14 @@ struct ExactOutF {
   }
 };
 
+// f(std::integral_constant<int, DT>) for the row element type dtype.
+template <typename F>
+void by_rows_type(int dtype, F f) {
+  if (dtype == ESC_ROWS_BF16) f(std::integral_constant<int, esc::kRowsBF16>{});
+  else if (dtype == ESC_ROWS_F32) f(std::integral_constant<int, esc::kRowsF32>{});
+  else f(std::integral_constant<int, esc::kRowsF16>{});
+}
+
 // ---- split-K GEMV geometry: KS kt per block (multiple of 4, divides TK)
 int fast_splits(int K, int M, int TK, int TN, int target = 1024) {
   const int tpw = K == 2 ? 16 : 8;
@@ -286,13 +293,16 @@ struct MmaPlan {
 size_t mma2_part_bytes(int M, int TN, int S) {
   return (size_t)S * ((M + 15) / 16) * ((TN + 15) / 16) * 16384;
 }
-MmaPlan mma_plan(int M, int TK, int TN, bool split) {
-  const int cus = device_cus(), NS = TK / 4, ncb = (TN + 15) / 16;
+// fixed_S > 0: that many splits; ncb2: column blocks of a second product in the
+// launch.
+MmaPlan mma_plan(int M, int TK, int TN, bool split, int fixed_S = 0, int ncb2 = 0) {
+  const int cus = device_cus(), NS = TK / 4, ncb = (TN + 15) / 16 + ncb2;
   MmaPlan best{8, 1, 0};
   double best_cost = 1e30;
   for (int S = 1; S == 1 || (split && S * kMmaMinSteps <= NS); ++S) {
     const size_t part = S > 1 ? mma2_part_bytes(M, TN, S) : 0;
     if (part > kMmaPartMax) break;
+    if (fixed_S && S != fixed_S) continue;
     const double extra = S > 1 ? 2.0 * part / 4.5e6 + 5.0 : 0.0;
     for (int nrb = 8; nrb >= 2; nrb -= 2) {
       const long wgs = (long)((M + 16 * nrb - 1) / (16 * nrb)) * ncb * S;
@@ -311,9 +321,12 @@ MmaPlan mma_plan(int M, int TK, int TN, bool split) {
 }
 
 template <int MODE>
-int gemm_mma2_launch(int K, int nrb, int S, const esc::MmaArgs& a, hipStream_t s) {
-  const dim3 grid(((a.M + 16 * nrb - 1) / (16 * nrb)) * ((a.TN + 15) / 16), S);
-  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a); };
+int gemm_mma2_launch(int K, int nrb, int S, const esc::MmaArgs& a, hipStream_t s,
+                     const esc::MmaArgs* second = nullptr) {
+  const int rb = (a.M + 16 * nrb - 1) / (16 * nrb), n0 = rb * ((a.TN + 15) / 16);
+  const dim3 grid(n0 + (second ? rb * ((second->TN + 15) / 16) : 0), S);
+  const esc::MmaArgs& b = second ? *second : a;
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, grid, dim3(256), 0, s, a, b, n0); };
   if (K == 2) {
     if (nrb == 2) go(esc::k_gemm_mma2<2, 2, MODE>);
     else if (nrb == 4) go(esc::k_gemm_mma2<2, 4, MODE>);
@@ -328,22 +341,35 @@ int gemm_mma2_launch(int K, int nrb, int S, const esc::MmaArgs& a, hipStream_t s
   return launched("k_gemm_mma2");
 }
 
+// The splits' partials of a summed and output-transformed.
+int mma2_reduce(int K, int S, const esc::MmaArgs& a, hipStream_t s) {
+  const dim3 grid((a.TN + 15) / 16, (a.M + 15) / 16);
+  if (K == 2)
+    hipLaunchKernelGGL(esc::k_mma2_reduce<2>, grid, dim3(256), 0, s, a, S);
+  else
+    hipLaunchKernelGGL(esc::k_mma2_reduce<3>, grid, dim3(256), 0, s, a, S);
+  return launched("k_mma2_reduce");
+}
+
 // The many-row GEMM with its output transform: one launch, or the splits'
 // partials into a.mid (plan.part_bytes) and their reduction.
 int gemm_mma2_out(int K, const MmaPlan& plan, const esc::MmaArgs& a, hipStream_t s) {
   if (plan.S == 1) return gemm_mma2_launch<esc::kMmaOut>(K, plan.nrb, 1, a, s);
   if (int rc = gemm_mma2_launch<esc::kMmaPart>(K, plan.nrb, plan.S, a, s)) return rc;
-  const dim3 grid((a.TN + 15) / 16, (a.M + 15) / 16);
-  if (K == 2)
-    hipLaunchKernelGGL(esc::k_mma2_reduce<2>, grid, dim3(256), 0, s, a, plan.S);
-  else
-    hipLaunchKernelGGL(esc::k_mma2_reduce<3>, grid, dim3(256), 0, s, a, plan.S);
-  return launched("k_mma2_reduce");
+  return mma2_reduce(K, plan.S, a, s);
 }
 
 // ---- one-launch linear for M < 16 (linear.hpp)
 constexpr int kLinearSmallRows = 16;
 constexpr int kLinearSmallRowsLut = 8;
+
+// Linears below kLinearSmallRows rows read f16 rows only.
+int check_rows_type(int dtype, int M) {
+  ESC_REQUIRE(dtype == ESC_ROWS_F16 || ((dtype == ESC_ROWS_BF16 || dtype == ESC_ROWS_F32) &&
+                                        (M >= kLinearSmallRows || M == 0)),
+              "row element type %d with %d rows", dtype, M);
+  return ESC_OK;
+}
 
 // k_proj_rows1: partial slots per 256-column group, at least the workgroups
 // a group of TK units can span: every workgroup holds at least 8 units when
@@ -352,25 +378,18 @@ int rows1_maxc(int TK) { return TK / 8 + 2; }
 // K=3 step pairs of every 8 that k_proj_rows1 decodes from the table
 constexpr int kTablePairs3 = 4;
 
-// One row (M = 1): the persistent table-mix kernel (k_proj_rows1) for the
-// table decode of a projection of at least kRows1MinUnits units (kt x
-// 256-column groups); the one-launch split-K kernel (k_linear_small) by hash
-// otherwise, also when the table decode was asked for (the two decodes give
-// the same weights; by hash the split-K kernel is ahead of its table form at
-// every size).  Measured on MI355X with HIP-graph replay: K=2 5120 x 5120
-// (6,400 units) 12.35 us by hash split-K against 14.8 us in the persistent
-// kernel; K=3 5120 -> 17408 (21,760 units) 20.0 against 22.6 us, and
-// 17408 -> 5120 level (23.2 against 23.1 us).
+// One row (M = 1): the persistent table-mix kernel (k_proj_rows1) for a
+// projection of at least kRows1MinUnits units (kt x 256-column groups), the
+// one-launch split-K kernel (k_linear_small) by hash otherwise, whichever decode was
+// asked for (the two decodes give the same weights).  Measured on MI355X, per call:
+// K=2 5120 -> 17408 and 17408 -> 5120 (21,760 units) 19.5 and 20.2 us in the
+// persistent kernel against 28.1 and 28.9 us, 8192 x 8192 (16,384 units) 16.3
+// against 21.1 us; K=3 21.1 and 22.3 against 25.8 and 26.7 us; K=2 5120 x 5120 (6,400
+// units, HIP-graph replay) 14.8 against 12.35 us.
 constexpr long kRows1MinUnits = 16384;
-bool rows1_single(int M, int IC, int OC, bool lut) {
-  return M == 1 && lut && OC % 256 == 0 && (long)(IC / 16) * (OC / 256) >= kRows1MinUnits;
+bool rows1_single(int M, int IC, int OC) {
+  return M == 1 && OC % 256 == 0 && (long)(IC / 16) * (OC / 256) >= kRows1MinUnits;
 }
-// The decode a one-launch linear runs: the table only where the persistent
-// kernel takes it (one row); 2..15 rows run the row-blocked split-K kernel by
-// hash (the table form stages 128 KiB of LDS per workgroup and holds 8 rows:
-// measured on MI355X at 4 rows, K=2 5120 x 5120 21.3 us by hash against
-// 23.7 us, K=3 5120 -> 17408 30.9 against 48.9 us).
-bool linear_uses_lut(int M, int IC, int OC, bool lut) { return rows1_single(M, IC, OC, lut); }
 size_t rows1_part_bytes(int TK, int TN) { return (size_t)(TN / 16) * rows1_maxc(TK) * 256 * 4; }
 
 struct LinearPlan {
@@ -489,20 +508,20 @@ int linear_pair_k(int K0, int K1, const esc::LinearSmallArgs& a0, const esc::Lin
 // k_proj_rows1 over a.np projections whose x .. TK, TN are filled: each
 // projection's plan from its own shape (one workgroup per CU, or more when a
 // wave would run more than kProjMaxP units), its workgroups after the
-// previous projection's.  K=2 with the table decodes kTablePairsLayers of 8
-// pairs from it, K=3 4 of 8.
+// previous projection's.  K=2 decodes kTablePairsLayers of 8 pairs from the
+// table, K=3 4 of 8, whichever decode was asked for (q, k and v of 5120 inputs in
+// one launch, K=2: 18.7 us against 20.8 by hash alone; level at 2048 and 4096).
 template <int K, int NT>
 int launch_rows1_k(const esc::ProjArgs& a, int grid, hipStream_t s) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
-  if constexpr (NT > 0)
-    std::call_once(once, [] {
-      err = hipFuncSetAttribute((const void*)esc::k_proj_rows1<K, NT>,
-                                hipFuncAttributeMaxDynamicSharedMemorySize, 65536 * 2);
-    });
+  std::call_once(once, [] {
+    err = hipFuncSetAttribute((const void*)esc::k_proj_rows1<K, NT>,
+                              hipFuncAttributeMaxDynamicSharedMemorySize, 65536 * 2);
+  });
   if (int rc = hip_check(err, "hipFuncSetAttribute")) return rc;
-  const size_t lds = NT > 0 ? 65536 * 2 : esc::kProjLdsWork;
-  hipLaunchKernelGGL((esc::k_proj_rows1<K, NT>), dim3(grid), dim3(64 * esc::kProjWaves), lds, s, a);
+  hipLaunchKernelGGL((esc::k_proj_rows1<K, NT>), dim3(grid), dim3(64 * esc::kProjWaves), 65536 * 2,
+                     s, a);
   return launched("k_proj_rows1");
 }
 
@@ -521,9 +540,7 @@ int rows1_workgroups(long n, long wgs) {
 // (one round of workgroups for several small projections); otherwise each
 // projection's from its own size alone, so that its outputs are those of
 // its own launch.
-int launch_rows1(esc::ProjArgs& a, int K, bool lut, hipStream_t s, bool merged = false) {
-  // one workgroup per CU (two per CU without the table measured slower:
-  // fewer units per wave, more partials per group)
+int launch_rows1(esc::ProjArgs& a, int K, hipStream_t s, bool merged = false) {
   const int cus = device_cus();
   long total = 0;
   for (int i = 0; i < a.np; ++i) {
@@ -539,12 +556,8 @@ int launch_rows1(esc::ProjArgs& a, int K, bool lut, hipStream_t s, bool merged =
     q.wg0 = (int)grid;
     grid += q.G;
   }
-  if (lut)
-    if (int rc = ensure_lut()) return rc;
-  if (K == 2)
-    return lut ? launch_rows1_k<2, esc::kTablePairsLayers>(a, (int)grid, s)
-               : launch_rows1_k<2, 0>(a, (int)grid, s);
-  return lut ? launch_rows1_k<3, kTablePairs3>(a, (int)grid, s) : launch_rows1_k<3, 0>(a, (int)grid, s);
+  return K == 2 ? launch_rows1_k<2, esc::kTablePairsLayers>(a, (int)grid, s)
+                : launch_rows1_k<3, kTablePairs3>(a, (int)grid, s);
 }
 
 // k_combine, 8 columns per thread where the rows allow 16-byte accesses.
@@ -688,12 +701,10 @@ int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t*
   if (int rc = check_proj(K, IC, OC)) return rc;
   ESC_REQUIRE(x && rin && code && rout && y, "null pointer");
   ESC_REQUIRE(M >= 0, "negative row count");
-  ESC_REQUIRE(dtype == ESC_ROWS_F16 || ((dtype == ESC_ROWS_BF16 || dtype == ESC_ROWS_F32) &&
-                                        (M >= kLinearSmallRows || M == 0)),
-              "row element type %d with %d rows", dtype, M);
+  if (int rc = check_rows_type(dtype, M)) return rc;
   if (M == 0) return ESC_OK;
-  use_lut = linear_uses_lut(M, IC, OC, use_lut != 0);
-  const LinearPlan lp = linear_plan(M, K, IC, OC, use_lut != 0);
+  (void)use_lut;  // the decode is the kernel's own choice: both give the same weights
+  const LinearPlan lp = linear_plan(M, K, IC, OC, rows1_single(M, IC, OC));
   const size_t need = M < kLinearSmallRows ? lp.total : lp.min_total;
   if (!ws || ws_bytes < need)
     return fail(ESC_ENOSPACE, "workspace %zu bytes < required %zu", ws_bytes, need);
@@ -702,7 +713,7 @@ int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t*
   char* w = static_cast<char*>(ws);
   const uint16_t* x16 = static_cast<const uint16_t*>(x);
   uint16_t* y16 = static_cast<uint16_t*>(y);
-  if (rows1_single(M, IC, OC, use_lut != 0)) {
+  if (rows1_single(M, IC, OC)) {
     // one row: the persistent kernel, its counters at off_cnt and its
     // partials at off_part (linear_plan sizes both)
     esc::ProjArgs a{};
@@ -711,10 +722,10 @@ int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t*
     a.pr[0] = esc::ProjOne{x16, rin, code, rout, bias, y16,
                            reinterpret_cast<float*>(w + lp.off_part),
                            reinterpret_cast<int*>(w + lp.off_cnt), TK, TN};
-    return launch_rows1(a, K, use_lut != 0, s);
+    return launch_rows1(a, K, s);
   }
   if (M < kLinearSmallRows) {
-    // the split-K kernel, by hash (linear_uses_lut)
+    // the split-K kernel, by hash
     float* part = reinterpret_cast<float*>(w + lp.off_part);
     int* cnt = reinterpret_cast<int*>(w + lp.off_cnt);
     const esc::LinearSmallArgs a =
@@ -730,6 +741,38 @@ int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t*
   const esc::MmaArgs a{xh, code, M, TK, TN, reinterpret_cast<float*>(w + lp.off_mid),
                        rout, bias, rs, y, dtype};
   return gemm_mma2_out(K, plan, a, s);
+}
+
+int esc_linear_xh(const uint16_t* xh, const uint32_t* code, const float* rout,
+                  const uint16_t* bias, int M, int K, int IC, int OC, float rs, void* y,
+                  int y_dtype, void* ws, size_t ws_bytes, void* stream) {
+  if (int rc = check_proj(K, IC, OC)) return rc;
+  ESC_REQUIRE(xh && code && rout && y, "null pointer");
+  ESC_REQUIRE(M >= kLinearSmallRows || M == 0, "%d rows (%d or more)", M, kLinearSmallRows);
+  if (int rc = check_rows_type(y_dtype, M)) return rc;
+  if (M == 0) return ESC_OK;
+  const int TK = IC / 16, TN = OC / 16;
+  MmaPlan plan = mma_plan(M, TK, TN, true);
+  if (plan.S > 1 && (!ws || ws_bytes < plan.part_bytes)) plan = mma_plan(M, TK, TN, false);
+  const esc::MmaArgs a{xh, code, M, TK, TN, static_cast<float*>(ws), rout, bias, rs, y, y_dtype};
+  return gemm_mma2_out(K, plan, a, S(stream));
+}
+
+int esc_act_transform(const void* g, const void* u, int dtype, const float* rin, int m, int I,
+                      float rs, uint16_t* xh, void* stream) {
+  ESC_REQUIRE(g && u && rin && xh, "null pointer");
+  ESC_REQUIRE(I > 0 && I % 128 == 0, "Hadamard dimension must be divisible by 128, got %d", I);
+  ESC_REQUIRE(m >= 0, "negative row count");
+  ESC_REQUIRE(dtype == ESC_ROWS_F16 || dtype == ESC_ROWS_BF16 || dtype == ESC_ROWS_F32,
+              "row element type must be ESC_ROWS_F16, ESC_ROWS_BF16 or ESC_ROWS_F32, got %d",
+              dtype);
+  if (m == 0) return ESC_OK;
+  const dim3 grid(I / 128, (m + esc::kTransformRows - 1) / esc::kTransformRows);
+  by_rows_type(dtype, [&](auto dt) {
+    hipLaunchKernelGGL(esc::k_act_transform<decltype(dt)::value>, grid, dim3(256), 0, S(stream), g,
+                       u, rin, m, I, rs, xh);
+  });
+  return launched("k_act_transform");
 }
 
 size_t esc_gemm_mfma_out_workspace(int M, int K, int IC, int OC) {
@@ -765,10 +808,21 @@ int esc_linear_pair(const uint16_t* x, int M, int IC, const float* rin0, const u
                     const uint32_t* code1, const float* rout1, const uint16_t* bias1, int K1,
                     int OC1, int use_lut, float rs, uint16_t* y0, uint16_t* y1, void* ws,
                     size_t ws_bytes, void* stream) {
+  return esc_linear_pair_typed(x, ESC_ROWS_F16, M, IC, rin0, code0, rout0, bias0, K0, OC0, rin1,
+                               code1, rout1, bias1, K1, OC1, use_lut, rs, y0, y1, ws, ws_bytes,
+                               stream);
+}
+
+int esc_linear_pair_typed(const void* x, int dtype, int M, int IC, const float* rin0,
+                          const uint32_t* code0, const float* rout0, const uint16_t* bias0, int K0,
+                          int OC0, const float* rin1, const uint32_t* code1, const float* rout1,
+                          const uint16_t* bias1, int K1, int OC1, int use_lut, float rs, void* y0v,
+                          void* y1v, void* ws, size_t ws_bytes, void* stream) {
   if (int rc = check_proj(K0, IC, OC0)) return rc;
   if (int rc = check_proj(K1, IC, OC1)) return rc;
-  ESC_REQUIRE(x && rin0 && code0 && rout0 && y0 && rin1 && code1 && rout1 && y1, "null pointer");
+  ESC_REQUIRE(x && rin0 && code0 && rout0 && y0v && rin1 && code1 && rout1 && y1v, "null pointer");
   ESC_REQUIRE(M >= 0, "negative row count");
+  if (int rc = check_rows_type(dtype, M)) return rc;
   if (M == 0) return ESC_OK;
   const size_t need = esc_linear_pair_workspace(M, K0, K1, IC, OC0, OC1);
   if (!ws || ws_bytes < need)
@@ -778,21 +832,45 @@ int esc_linear_pair(const uint16_t* x, int M, int IC, const float* rin0, const u
   const size_t off1 = (ws0 + 255) & ~size_t(255);
   char* w = static_cast<char*>(ws);
   if (M >= kLinearSmallRows) {
-    // many rows: each projection's GEMM fills the GPU on its own
-    if (int rc = esc_linear(x, rin0, code0, rout0, bias0, M, K0, IC, OC0, use_lut, rs, y0, w, ws0,
-                            stream))
-      return rc;
-    return esc_linear(x, rin1, code1, rout1, bias1, M, K1, IC, OC1, use_lut, rs, y1, w + off1,
-                      ws_bytes - off1, stream);
+    const int TK = IC / 16;
+    const LinearPlan p0 = linear_plan(M, K0, IC, OC0, false);
+    const LinearPlan p1 = linear_plan(M, K1, IC, OC1, false);
+    if (K0 != K1 || p0.mma.S != p1.mma.S) {
+      if (int rc = esc_linear_typed(x, dtype, rin0, code0, rout0, bias0, M, K0, IC, OC0, use_lut,
+                                    rs, y0v, w, ws0, stream))
+        return rc;
+      return esc_linear_typed(x, dtype, rin1, code1, rout1, bias1, M, K1, IC, OC1, use_lut, rs,
+                              y1v, w + off1, ws_bytes - off1, stream);
+    }
+    // both transforms in one pass over x, both products in one launch, with the
+    // splits of their own calls (the row blocks do not change a sum's order)
+    hipStream_t s = S(stream);
+    const int Sp = p0.mma.S;
+    char* w1 = w + off1;
+    uint16_t* xh0 = reinterpret_cast<uint16_t*>(w + p0.off_xh);
+    uint16_t* xh1 = reinterpret_cast<uint16_t*>(w1 + p1.off_xh);
+    const dim3 tg(IC / 128, (M + esc::kTransformRows - 1) / esc::kTransformRows);
+    by_rows_type(dtype, [&](auto dt) {
+      hipLaunchKernelGGL((esc::k_input_transform<decltype(dt)::value, true>), tg, dim3(256), 0, s,
+                         x, rin0, nullptr, M, IC, rs, xh0, rin1, xh1);
+    });
+    if (int rc = launched("k_input_transform")) return rc;
+    const esc::MmaArgs a0{xh0, code0, M, TK, OC0 / 16, reinterpret_cast<float*>(w + p0.off_mid),
+                          rout0, bias0, rs, y0v, dtype};
+    const esc::MmaArgs a1{xh1, code1, M, TK, OC1 / 16, reinterpret_cast<float*>(w1 + p1.off_mid),
+                          rout1, bias1, rs, y1v, dtype};
+    const int nrb = mma_plan(M, TK, OC0 / 16, true, Sp, (OC1 + 255) / 256).nrb;
+    if (Sp == 1) return gemm_mma2_launch<esc::kMmaOut>(K0, nrb, 1, a0, s, &a1);
+    if (int rc = gemm_mma2_launch<esc::kMmaPart>(K0, nrb, Sp, a0, s, &a1)) return rc;
+    if (int rc = mma2_reduce(K0, Sp, a0, s)) return rc;
+    return mma2_reduce(K0, Sp, a1, s);
   }
-  const bool r0 = rows1_single(M, IC, OC0, use_lut != 0), r1 = rows1_single(M, IC, OC1, use_lut != 0);
-  // the pair kernel runs the decode each projection's own call would
-  if (!r0 && !r1) use_lut = 0;
-  if (use_lut)
-    if (int rc = ensure_lut()) return rc;
+  const uint16_t* x16 = static_cast<const uint16_t*>(x);
+  uint16_t *y0 = static_cast<uint16_t*>(y0v), *y1 = static_cast<uint16_t*>(y1v);
+  const bool r0 = rows1_single(M, IC, OC0), r1 = rows1_single(M, IC, OC1);
   const int TK = IC / 16;
-  const LinearPlan p0 = linear_plan(M, K0, IC, OC0, use_lut != 0);
-  const LinearPlan p1 = linear_plan(M, K1, IC, OC1, use_lut != 0);
+  const LinearPlan p0 = linear_plan(M, K0, IC, OC0, r0);
+  const LinearPlan p1 = linear_plan(M, K1, IC, OC1, r1);
   char* w1 = w + off1;
   if (r0 && r1 && K0 == K1) {
     // one row: both projections in one persistent launch, each with its own
@@ -800,30 +878,30 @@ int esc_linear_pair(const uint16_t* x, int M, int IC, const float* rin0, const u
     esc::ProjArgs a{};
     a.np = 2;
     a.rs = rs;
-    a.pr[0] = esc::ProjOne{x, rin0, code0, rout0, bias0, y0,
+    a.pr[0] = esc::ProjOne{x16, rin0, code0, rout0, bias0, y0,
                            reinterpret_cast<float*>(w + p0.off_part),
                            reinterpret_cast<int*>(w + p0.off_cnt), TK, OC0 / 16};
-    a.pr[1] = esc::ProjOne{x, rin1, code1, rout1, bias1, y1,
+    a.pr[1] = esc::ProjOne{x16, rin1, code1, rout1, bias1, y1,
                            reinterpret_cast<float*>(w1 + p1.off_part),
                            reinterpret_cast<int*>(w1 + p1.off_cnt), TK, OC1 / 16};
-    return launch_rows1(a, K0, use_lut != 0, S(stream));
+    return launch_rows1(a, K0, S(stream));
   }
   if (r0 || r1 || p0.R != p1.R) {
     // one row with the projections on different kernels (or K), or row
     // groups of different sizes: each as its own call
-    if (int rc = esc_linear(x, rin0, code0, rout0, bias0, M, K0, IC, OC0, use_lut, rs, y0, w, ws0,
+    if (int rc = esc_linear(x16, rin0, code0, rout0, bias0, M, K0, IC, OC0, use_lut, rs, y0, w, ws0,
                             stream))
       return rc;
-    return esc_linear(x, rin1, code1, rout1, bias1, M, K1, IC, OC1, use_lut, rs, y1, w + off1,
+    return esc_linear(x16, rin1, code1, rout1, bias1, M, K1, IC, OC1, use_lut, rs, y1, w + off1,
                       ws_bytes - off1, stream);
   }
   const esc::LinearSmallArgs a0 =
-      small_args(x, rin0, code0, rout0, bias0, M, TK, OC0 / 16, p0, rs,
+      small_args(x16, rin0, code0, rout0, bias0, M, TK, OC0 / 16, p0, rs,
                  reinterpret_cast<float*>(w + p0.off_part), reinterpret_cast<int*>(w + p0.off_cnt), y0);
   const esc::LinearSmallArgs a1 =
-      small_args(x, rin1, code1, rout1, bias1, M, TK, OC1 / 16, p1, rs,
+      small_args(x16, rin1, code1, rout1, bias1, M, TK, OC1 / 16, p1, rs,
                  reinterpret_cast<float*>(w1 + p1.off_part), reinterpret_cast<int*>(w1 + p1.off_cnt), y1);
-  // the split-K pair kernel, by hash (linear_uses_lut)
+  // the split-K pair kernel, by hash
   return linear_pair_k<false>(K0, K1, a0, a1, S(stream));
 }
 
@@ -877,7 +955,7 @@ int esc_linear_multi(const uint16_t* x, int M, int IC, int K, int n, const uint3
       a.pr[i] = esc::ProjOne{x, rin[i], code[i], rout[i], bias ? bias[i] : nullptr, y[i], part,
                              cnt, IC / 16, OC[i] / 16};
     }
-    return launch_rows1(a, K, use_lut != 0, S(stream), true);
+    return launch_rows1(a, K, S(stream), true);
   }
   // several rows: each projection's esc_linear plan and workspace, as one
   // k_linear_multi launch when all run the split-K kernel with one row group
@@ -1028,8 +1106,11 @@ int esc_route_topk(const float* logits, int T, int E, int top_k, int32_t* ids, f
   ESC_REQUIRE(top_k >= 1 && top_k <= 32 && top_k <= E, "top_k %d not in [1, min(32, E)]", top_k);
   ESC_REQUIRE(T >= 0, "negative token count");
   if (T == 0) return ESC_OK;
-  hipLaunchKernelGGL(esc::k_route_topk, dim3(T), dim3(64), 0, S(stream), logits, E, top_k, ids,
-                     scores);
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(T), dim3(64), 0, S(stream), logits, E, top_k, ids, scores);
+  };
+  if (E <= 256) go(esc::k_route_topk<4>);
+  else go(esc::k_route_topk<16>);
   return launched("k_route_topk");
 }
 
@@ -1267,18 +1348,18 @@ namespace {
 // Rows per expert group of the split-K chain: once there are as many routed
 // rows as experts, rows of one expert share each decoded weight (groups laid
 // out by moe.build_groups, one row per B column of the matrix-core multiply,
-// so a group costs one decode whatever its row count); below that almost
-// every expert has one row.
-constexpr int kMoeGroupRows = 8;
-int moe_group_rows(int M, int E) { return M >= E ? kMoeGroupRows : 0; }
+// so a group costs one decode whatever its row count, up to 16); below that
+// almost every expert has one row.  16 rows per group from four rows per expert
+// (measured on MI355X, 256 experts, hidden 2048, intermediate 512, top-8, whole
+// call, 8 against 16 rows: 48 tokens 112 / 115 us, 128 145 / 140, 200 167 / 150).
+int moe_group_rows(int M, int E) { return M >= 4L * E ? 16 : M >= E ? 8 : 0; }
 
-// f(std::integral_constant<int, DT>) for the row element type dtype.
-template <typename F>
-void by_rows_type(int dtype, F f) {
-  if (dtype == ESC_ROWS_BF16) f(std::integral_constant<int, esc::kRowsBF16>{});
-  else if (dtype == ESC_ROWS_F32) f(std::integral_constant<int, esc::kRowsF32>{});
-  else f(std::integral_constant<int, esc::kRowsF16>{});
-}
+// Whether the grouped chain decodes with the table (k_gemv_rows_table, which
+// stages 128 KiB per CU) or by hash, whichever decode was asked for: the weights
+// are the same, and the table wins from about 2^28 weights to decode (measured
+// as above, hash against table: 256 experts 48 tokens 128 / 115 us, 200 tokens 164
+// / 150; 64 experts, 201 M weights, 66 / 73; 64 experts of 1024 x 256 42 / 46).
+bool moe_rows_table(int groups, int H, int I) { return (double)groups * 3 * H * I >= (1 << 28); }
 
 int moe_input(const void* x, int dtype, const int32_t* ids, int top_k, const float* rin, int H,
               float rs, uint16_t* xh, int M, hipStream_t s) {
@@ -1291,15 +1372,16 @@ int moe_input(const void* x, int dtype, const int32_t* ids, int top_k, const flo
 
 // Row blocks of 16 per group of the grouped matrix-core GEMM (k_moe_mma), 0:
 // the split-K chain.  Measured on MI355X (256 experts, hidden 2048, intermediate
-// 512, top-8; whole call, the split-K chain by hash / by table in brackets): 4
-// rows per expert 184 us (165 / -), 8 rows 186 (246 / 211), 16 rows 208 (394 /
-// 349), 64 rows 357 (1200 / -).  So from 8 rows per expert, at the row-block
-// size with the least work: a group costs 0.43 + 0.071 NRB (208, 263, 292 and
-// 337 us with one group of 2, 4, 6 and 8 row blocks per expert), and an expert
-// with Poisson(M / E) rows takes sum over j of P(rows > 16 NRB j) groups.
-constexpr int kMoeMmaRowsPerExpert = 8;
+// 512, top-8; whole call, the split-K chain in brackets): 6 rows per expert 175 us
+// (150), 9 rows 175 (164), 12 rows 180 (187), 16 rows 183 (218), 64 rows 306 (1200
+// in groups of 8); 64 experts, 8 rows 78 (80 by hash), 12 rows 79 (99), 4 rows 78
+// (66).  So from 8 rows per expert, or 11 where the experts' weights fill the chip
+// (the split-K chain then decodes with the table), at the row-block size with the
+// least work: a group costs 0.43 + 0.071 NRB (208, 263, 292 and 337 us with one
+// group of 2, 4, 6 and 8 row blocks per expert), and an expert with Poisson(M / E)
+// rows takes sum over j of P(rows > 16 NRB j) groups.
 int moe_mma_nrb(int M, int E, int H, int I) {
-  if (E > 4096 || M / E < kMoeMmaRowsPerExpert) return 0;
+  if (E > 4096 || M / E < (moe_rows_table(E, H, I) ? 11 : 8)) return 0;
   // 32-bit byte offsets into the transformed rows
   if ((size_t)M * std::max(H, I) * 2 > 0xFFFFFFF0u) return 0;
   const double lam = (double)M / E, dev = std::sqrt(2.0 * lam);
@@ -1325,6 +1407,7 @@ int moe_mma_nrb(int M, int E, int H, int I) {
 
 struct MoePlan {
   int M, S1, S2, R, n_groups, nrb;
+  bool table;  // the grouped chain's decode
   size_t off_xh, off_p1, off_xh2, off_p2, off_rows, off_gexp, off_nact, off_d16, total;
 };
 // base: bytes at the start of the workspace left to the caller (the
@@ -1332,12 +1415,14 @@ struct MoePlan {
 MoePlan moe_plan(int T, int top_k, int E, int H, int I, int K_gu, int K_dn, size_t base = 0) {
   MoePlan p;
   p.M = T * top_k;
-  p.R = E <= 4096 ? moe_group_rows(p.M, E) : 0;
+  // a fixed scratch keeps 8 rows per group, whose row lists are the smaller
+  p.R = E <= 4096 ? std::min(moe_group_rows(p.M, E), base ? 8 : 16) : 0;
   p.n_groups = p.R ? (p.M + E * (p.R - 1) + p.R - 1) / p.R : 0;
-  // non-empty groups, about: the experts a uniform routing touches, or M/R
-  const int eff = p.R ? std::max((p.M + p.R - 1) / p.R,
+  // non-empty groups, about: the experts a uniform routing touches, or M/8
+  const int eff = p.R ? std::max((p.M + 7) / 8,
                                  (int)(E * (1.0 - std::pow(1.0 - 1.0 / E, (double)p.M))))
                       : p.M;
+  p.table = p.R && moe_rows_table(eff, H, I);
   // the grouped GEMVs aim for 2048 blocks: at 32 tokens (E = 256, H = 2048,
   // I = 512, top-8) 1,201 GB/s against 1,171 at 1024, 1,147 at 512 and
   // 1,161 at 4096 on MI355X; below about 16 tokens the kt bound sets S first
@@ -1370,51 +1455,50 @@ MoePlan moe_plan(int T, int top_k, int E, int H, int I, int K_gu, int K_dn, size
   return p;
 }
 
-template <int K, bool LUT>
-struct GroupRowsF {
-  template <int R>
-  static int go(const uint16_t* xh, const uint32_t* code, const int* rows, const int* gexp,
-                int n_groups, int M, int TK, int TN, int S, float* part, hipStream_t s) {
-    const int tpw = K == 2 ? 16 : 8;
-    hipLaunchKernelGGL((esc::k_gemv_fast_rows<K, LUT, R>), dim3((TN + tpw - 1) / tpw, n_groups, S),
-                       dim3(256), 0, s, xh, code, rows, gexp, M, TK, TN, TK / S, part);
-    return launched("k_gemv_fast_rows");
-  }
-  static int run(int R, const uint16_t* xh, const uint32_t* code, const int* rows, const int* gexp,
-                 int n_groups, int M, int TK, int TN, int S, float* part, hipStream_t s) {
-    if (R != kMoeGroupRows) return fail(ESC_EINVAL, "rows per expert group %d", R);
-    return go<kMoeGroupRows>(xh, code, rows, gexp, n_groups, M, TK, TN, S, part, s);
-  }
-};
+// The grouped GEMM by hash: short-lived workgroups over every group there may be.
+template <int K, int R>
+int launch_rows_hash(const uint16_t* xh, const uint32_t* code, const int* rows, const int* gexp,
+                     int n_groups, int M, int TK, int TN, int S, float* part, hipStream_t s) {
+  const int tpw = K == 2 ? 16 : 8;
+  hipLaunchKernelGGL((esc::k_gemv_fast_rows<K, false, R>), dim3((TN + tpw - 1) / tpw, n_groups, S),
+                     dim3(256), 0, s, xh, code, rows, gexp, M, TK, TN, TK / S, part);
+  return launched("k_gemv_fast_rows");
+}
 
 // The grouped GEMM with the table decode: the persistent k_gemv_rows_table
 // (one workgroup per CU, the table staged once), its item count from the
 // groups build_groups filled (nact, on the device).
-template <int K>
+template <int K, int R>
 int launch_rows_table(const uint16_t* xh, const uint32_t* code, const int* rows, const int* gexp,
                       const int* nact, int M, int TK, int TN, int S, float* part, hipStream_t s) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
-    err = hipFuncSetAttribute((const void*)esc::k_gemv_rows_table<K, kMoeGroupRows>,
+    err = hipFuncSetAttribute((const void*)esc::k_gemv_rows_table<K, R>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, 65536 * 2);
   });
   if (int rc = hip_check(err, "hipFuncSetAttribute")) return rc;
-  hipLaunchKernelGGL((esc::k_gemv_rows_table<K, kMoeGroupRows>), dim3(device_cus()), dim3(1024),
-                     65536 * 2, s, xh, code, rows, gexp, nact, M, TK, TN, TK / S, S, part);
+  hipLaunchKernelGGL((esc::k_gemv_rows_table<K, R>), dim3(device_cus()), dim3(1024), 65536 * 2, s,
+                     xh, code, rows, gexp, nact, M, TK, TN, TK / S, S, part);
   return launched("k_gemv_rows_table");
 }
 
-int group_rows(int K, int lut, int R, const uint16_t* xh, const uint32_t* code, const int* rows,
-               const int* gexp, const int* nact, int n_groups, int M, int TK, int TN, int S,
-               float* part, hipStream_t s) {
-  if (lut) {
-    if (R != kMoeGroupRows) return fail(ESC_EINVAL, "rows per expert group %d", R);
-    return K == 2 ? launch_rows_table<2>(xh, code, rows, gexp, nact, M, TK, TN, S, part, s)
-                  : launch_rows_table<3>(xh, code, rows, gexp, nact, M, TK, TN, S, part, s);
-  }
-  return K == 2 ? GroupRowsF<2, false>::run(R, xh, code, rows, gexp, n_groups, M, TK, TN, S, part, s)
-                : GroupRowsF<3, false>::run(R, xh, code, rows, gexp, n_groups, M, TK, TN, S, part, s);
+template <int K, int R>
+int group_rows_k(const uint16_t* xh, const uint32_t* code, const int* rows, const int* gexp,
+                 const int* nact, const MoePlan& p, int TK, int TN, int S, float* part,
+                 hipStream_t s) {
+  return p.table ? launch_rows_table<K, R>(xh, code, rows, gexp, nact, p.M, TK, TN, S, part, s)
+                 : launch_rows_hash<K, R>(xh, code, rows, gexp, p.n_groups, p.M, TK, TN, S, part, s);
+}
+
+int group_rows(int K, const uint16_t* xh, const uint32_t* code, const int* rows, const int* gexp,
+               const int* nact, const MoePlan& p, int TK, int TN, int S, float* part,
+               hipStream_t s) {
+  if (K == 2)
+    return p.R == 16 ? group_rows_k<2, 16>(xh, code, rows, gexp, nact, p, TK, TN, S, part, s)
+                     : group_rows_k<2, 8>(xh, code, rows, gexp, nact, p, TK, TN, S, part, s);
+  return p.R == 16 ? group_rows_k<3, 16>(xh, code, rows, gexp, nact, p, TK, TN, S, part, s)
+                   : group_rows_k<3, 8>(xh, code, rows, gexp, nact, p, TK, TN, S, part, s);
 }
 
 template <int K, bool GU>
@@ -1844,8 +1928,7 @@ int moe_expert_path(const void* x, int dtype, const int32_t* ids, const float* s
       if (int rc = moe_mma<false>(K_dn, p.nrb, a, s)) return rc;
       return combine_rows(d16, scores, T, top_k, H, y, s);
     }
-    if (int rc = group_rows(K_gu, use_lut, p.R, xh, gu_code, rows, gexp, nact, p.n_groups, p.M,
-                            H / 16, 2 * I / 16, p.S1, p1, s))
+    if (int rc = group_rows(K_gu, xh, gu_code, rows, gexp, nact, p, H / 16, 2 * I / 16, p.S1, p1, s))
       return rc;
   } else if (int rc = moe_input(x, dtype, ids, top_k, gu_rin, H, rs, xh, p.M, s)) {
     return rc;
@@ -1865,8 +1948,7 @@ int moe_expert_path(const void* x, int dtype, const int32_t* ids, const float* s
   }
   if (int rc = launched("k_moe_mid")) return rc;
   if (p.R) {
-    if (int rc = group_rows(K_dn, use_lut, p.R, xh2, dn_code, rows, gexp, nact, p.n_groups, p.M,
-                            I / 16, H / 16, p.S2, p2, s))
+    if (int rc = group_rows(K_dn, xh2, dn_code, rows, gexp, nact, p, I / 16, H / 16, p.S2, p2, s))
       return rc;
   } else if (int rc = by_k_lut<FastF>(K_dn, use_lut, xh2, dn_code, ids, p.M, I / 16, H / 16, p.S2,
                                       p2, s)) {

@@ -343,25 +343,31 @@ __device__ __forceinline__ size_t mma2_part_index(int z, int rb16, int nrb16, in
   return ((((size_t)z * nrb16 + rb16) * ncb + cb) * 4 + wave) * 256 + 64 * a;
 }
 
+// Two products of the same rows and splits may share a launch (p1 from workgroup
+// n0 on): gate and up of 2048 rows hold 4.25 tiles per CU each, 8.5 together, and
+// a launch takes what its busiest CU holds.
 template <int K, int NRB, int MODE>
-__global__ __launch_bounds__(256, 2) void k_gemm_mma2(MmaArgs p) {
+__global__ __launch_bounds__(256, 2) void k_gemm_mma2(MmaArgs p0, MmaArgs p1, int n0) {
   using G = Geo<K>;
   using D = Mma2<K, NRB>;
   constexpr int TPS = D::TPS, GPW = D::GPW, NA = D::NA, BR = D::BR, XCH = D::XCH;
   __shared__ uint4 s_x[2][BR * 8];        // [stage][row][chunk ^ (row & 7)]
 
+  const bool second = (int)blockIdx.x >= n0;
+  const MmaArgs p = second ? p1 : p0;
+  const int b = second ? (int)blockIdx.x - n0 : (int)blockIdx.x;
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
   const int M = p.M, TK = p.TK, TN = p.TN;
   const int IC = TK * 16, OC = TN * 16;
   const int ncb = (TN + 15) / 16;
   int rb, cb;
   if (ncb % 8 == 0) {
-    const int per = ncb / 8, qq = blockIdx.x / 8, x = blockIdx.x % 8;
+    const int per = ncb / 8, qq = b / 8, x = b % 8;
     rb = qq / per;
     cb = 8 * (qq % per) + x;
   } else {
-    rb = blockIdx.x / ncb;
-    cb = blockIdx.x % ncb;
+    rb = b / ncb;
+    cb = b % ncb;
   }
   const int row0 = rb * BR;
   int tile0 = cb * 16 + 4 * wave;

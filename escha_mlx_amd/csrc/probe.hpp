@@ -21,7 +21,7 @@ __global__ __launch_bounds__(1024) void k_decode_probe(const uint32_t* __restric
   static_assert(PF >= 1 && PF <= 3, "prefetch depth");
   extern __shared__ uint16_t s_tab[];
   if constexpr (NT > 0) {
-    const uint4* src = reinterpret_cast<const uint4*>(g_lut);
+    const uint4* src = reinterpret_cast<const uint4*>(g_lut.v);
     uint4* dst = reinterpret_cast<uint4*>(s_tab);
     for (int i = threadIdx.x; i < 65536 / 8; i += blockDim.x) dst[i] = src[i];
     __syncthreads();

@@ -17,10 +17,9 @@
 // partials; a single launch chooses G from the projection's own shape, so its
 // outputs do not depend on what else shares the launch.
 //
-// With the table (NT > 0; staged in LDS once per workgroup) NT of every 8
-// step pairs are decoded from it and the rest by hash (fast_tile_mix for K=2,
-// fast_tile_mix3 for K=3); NT = 0 decodes by hash.  Reduction, in a fixed
-// order (deterministic, no float atomics):
+// NT of every 8 step pairs are decoded from the table (staged in LDS once per
+// workgroup) and the rest by hash (fast_tile_mix for K=2, fast_tile_mix3 for
+// K=3).  Reduction, in a fixed order (deterministic, no float atomics):
 //   1. every wave's partial of each group it touched goes to LDS; the
 //      workgroup sums them in wave order, one wave per group, and publishes
 //      one float32 partial per (workgroup, group) with agent-scope stores;
@@ -67,7 +66,8 @@ struct ProjArgs {
 // LDS of the kernel beyond the table: each wave's partials of its two
 // groups (phase 1 -> 2) and the finishers' column sums; both live in the
 // table's space once every wave has finished decoding.
-constexpr int kProjLdsWork = (kProjWaves * 2 * 256 + kProjWaves * 256) * 4;
+// the partials and sums that reuse the table's LDS
+static_assert((kProjWaves * 2 * 256 + kProjWaves * 256) * 4 <= 65536 * 2, "");
 
 // unit -> (column group, kt)
 struct ProjUnit {
@@ -150,10 +150,10 @@ __device__ __forceinline__ int proj_col(int lane, int ci) {
 }
 
 // grid: the projections' workgroups one after the other (projection j's
-// from pr[j].wg0), 16 waves each; dynamic LDS: the table (NT > 0) or
-// kProjLdsWork bytes.
+// from pr[j].wg0), 16 waves each; dynamic LDS: the table.
 template <int K, int NT>
 __global__ __launch_bounds__(64 * kProjWaves) void k_proj_rows1(ProjArgs p) {
+  static_assert(NT > 0, "");
   extern __shared__ uint16_t s_dyn[];
   __shared__ int s_grp[kProjWaves][2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -188,17 +188,15 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_proj_rows1(ProjArgs p) {
 
   const uint32_t xa = proj_inputs(ina, p.rs);
   const uint32_t xb = two_blocks ? proj_inputs(inb, p.rs) : xa;
-  if constexpr (NT > 0) {
-    // The table's pieces are requested once the first unit's code and the
-    // inputs are in registers (the compiler waits for every outstanding load
-    // after a DMA into LDS, so a wait placed later would also wait for the
-    // table), and land while the first unit decodes.
+  // The table's pieces are requested once the first unit's code and the
+  // inputs are in registers (the compiler waits for every outstanding load
+  // after a DMA into LDS, so a wait placed later would also wait for the
+  // table), and land while the first unit decodes.
 #pragma unroll
-    for (int h = 0; h < (K == 3 ? 2 : 1); ++h)
+  for (int h = 0; h < (K == 3 ? 2 : 1); ++h)
 #pragma unroll
-      for (int j = 0; j < Geo<K>::WPL; ++j) __asm__ volatile("" : : "v"(w[h].w[j]));
-    table_dma(s_dyn);
-  }
+    for (int j = 0; j < Geo<K>::WPL; ++j) __asm__ volatile("" : : "v"(w[h].w[j]));
+  table_dma(s_dyn);
 
   float acc[4] = {0.f, 0.f, 0.f, 0.f}, accA[4] = {0.f, 0.f, 0.f, 0.f};
   // unit u: the next unit's code requested (this one again at the end: in
@@ -227,17 +225,14 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_proj_rows1(ProjArgs p) {
   // the first units are decoded by hash before the table is in LDS, so their
   // decode runs while the table's pieces are still arriving (the table is
   // the hash's image and the step order is the same: bit-identical)
-  const int uh = NT > 0 ? min(b, a + kProjHashUnits) : a;
+  const int uh = min(b, a + kProjHashUnits);
 #pragma unroll 1
   for (int u = a; u < uh; ++u) {
     prio_left(b - u);
     unit(u, std::integral_constant<int, 0>{}, 0u);
   }
-  uint32_t tb = 0;
-  if constexpr (NT > 0) {
-    wait_vm();  // this wave's table pieces are in LDS
-    tb = (uint32_t)(size_t)s_dyn;
-  }
+  wait_vm();  // this wave's table pieces are in LDS
+  const uint32_t tb = (uint32_t)(size_t)s_dyn;
   __syncthreads();
 
   if (busy) {

@@ -143,6 +143,10 @@ class EschaLinear(torch.nn.Module):
     def K(self) -> int:
         return self._w.K
 
+    def plain(self) -> bool:
+        """Whether 16 rows and more take the matrix-core GEMM with fused transforms."""
+        return (self._mat and self._fused_had and not self._exact and self._block_r_pin is None)
+
     def _linear_ws(self, m: int, device) -> torch.Tensor | None:
         if m >= ops.LINEAR_SMALL_ROWS:
             return None  # no counters: a fresh workspace per call
@@ -210,20 +214,22 @@ def project_pair(first: EschaLinear, second: EschaLinear, x: torch.Tensor):
     shape = x.shape
     rows = x.reshape(-1, shape[-1]).contiguous()
     m = rows.shape[0]
+    many = m >= ops.LINEAR_SMALL_ROWS
     compatible = (
-        rows.dtype == torch.float16
+        (rows.dtype == torch.float16 or many and rows.dtype in ops.ROWS_DTYPES)
         and w0.IC == w1.IC == rows.shape[-1]
         and first._lut == second._lut
         and first._fused_had and second._fused_had
         and not (first._exact or second._exact)
         and first._block_r_pin is None and second._block_r_pin is None
-        and (m < ops.LINEAR_SMALL_ROWS or (first._mat and second._mat))
+        and (not many or (first._mat and second._mat))
     )
     if not compatible:
         return first(x), second(x)
     key = (m, rows.device, id(second))
-    ws = first._pair_ws.get(key)
-    if ws is None:
+    # no counters from 16 rows on: a fresh workspace per call
+    ws = None if many else first._pair_ws.get(key)
+    if ws is None and not many:
         need = ops.linear_pair_workspace(m, w0.K, w1.K, w0.IC, w0.OC, w1.OC)
         ws = first._pair_ws[key] = torch.zeros(max(need, 4), dtype=torch.uint8, device=rows.device)
     y0, y1 = ops.linear_pair(rows, (w0.code, w0.rin, w0.rout, w0.K, w0.OC, first.bias),
@@ -286,6 +292,15 @@ class EschaMLP(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         shape = x.shape
         gate, up = project_pair(self.gate_proj, self.up_proj, x)
+        down = self.down_proj
+        m = gate.numel() // gate.shape[-1]
+        if m >= ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_DTYPES and down.plain():
+            # the activation and down's input transform in one pass
+            w = down._w
+            xh = ops.act_transform(gate.reshape(m, w.IC), up.reshape(m, w.IC), w.rin)
+            dtype = x.dtype if x.dtype in ops.ROWS_DTYPES else torch.float16
+            y = ops.linear_xh(xh, w.code, w.rout, w.K, w.IC, w.OC, bias=down.bias, dtype=dtype)
+            return y.reshape(*shape[:-1], w.OC).to(x.dtype)
         g = gate.reshape(-1, gate.shape[-1]).to(torch.float16).contiguous()
         u = up.reshape(-1, up.shape[-1]).to(torch.float16).contiguous()
         h = ops.moe_shared_act(g, u)

@@ -278,25 +278,60 @@ def linear_pair(x: torch.Tensor, p0: tuple, p1: tuple, lut: bool | None = None, 
                 ws: torch.Tensor | None = None):
     """Two coded linears over the same rows in one dispatch (dense.py:365-437):
     p0 / p1 = (code_u32, rin, rout, K, OC, bias or None); returns (y0, y1),
-    each bit-identical to ``linear`` on its own.  ws must be zero-filled
-    before its first use."""
+    each bit-identical to ``linear`` on its own (from 16 rows x may be bf16 or
+    f32, as there).  ws must be zero-filled before its first use."""
     c0, rin0, rout0, K0, OC0, b0 = p0
     c1, rin1, rout1, K1, OC1, b1 = p1
     _dev(x, c0, rin0, rout0, b0, c1, rin1, rout1, b1)
     m, IC = x.shape
-    if x.dtype != torch.float16:
+    if x.dtype != torch.float16 and not (m >= LINEAR_SMALL_ROWS and x.dtype in ROWS_DTYPES):
         raise ValueError("x must be float16")
-    y0 = torch.empty((m, OC0), dtype=torch.float16, device=x.device)
-    y1 = torch.empty((m, OC1), dtype=torch.float16, device=x.device)
+    y0 = torch.empty((m, OC0), dtype=x.dtype, device=x.device)
+    y1 = torch.empty((m, OC1), dtype=x.dtype, device=x.device)
     if m == 0:
         return y0, y1
-    need = linear_pair_workspace(m, K0, K1, IC, OC0, OC1)
     if ws is None:
-        ws = torch.zeros(max(need, 4), dtype=torch.uint8, device=x.device)
-    _lib.call("esc_linear_pair", _ptr(x), m, IC, _ptr(rin0), _ptr(_as_u32(c0)), _ptr(rout0),
+        need = linear_pair_workspace(m, K0, K1, IC, OC0, OC1)
+        alloc = torch.zeros if m < LINEAR_SMALL_ROWS else torch.empty  # counters below 16 rows
+        ws = alloc(max(need, 4), dtype=torch.uint8, device=x.device)
+    _lib.call("esc_linear_pair_typed", _ptr(x), ROWS_DTYPES[x.dtype], m, IC, _ptr(rin0), _ptr(_as_u32(c0)), _ptr(rout0),
               _ptr(b0), K0, OC0, _ptr(rin1), _ptr(_as_u32(c1)), _ptr(rout1), _ptr(b1), K1, OC1,
               _lut_flag(lut), rs, _ptr(y0), _ptr(y1), _ptr(ws), ws.numel(), _stream())
     return y0, y1
+
+
+def act_transform(g: torch.Tensor, u: torch.Tensor, rin: torch.Tensor, rs: float = RS
+                  ) -> torch.Tensor:
+    """g, u [m, I] (f16, or bf16 / f32 rounded to f16 first) -> the next projection's
+    transformed inputs f16 [m, I]: scaled_had(moe_shared_act(g, u), rin) in one pass."""
+    _dev(g, u, rin)
+    m, i = g.shape
+    if g.dtype not in ROWS_DTYPES or u.dtype != g.dtype or tuple(u.shape) != (m, i):
+        raise ValueError("g and u must be [m, I] of one floating type")
+    if rin.dtype != torch.float32 or tuple(rin.shape) != (i,):
+        raise ValueError(f"transform vector must be float32 ({i},)")
+    xh = torch.empty((m, i), dtype=torch.float16, device=g.device)
+    _lib.call("esc_act_transform", _ptr(g), _ptr(u), ROWS_DTYPES[g.dtype], _ptr(rin), m, i, rs,
+              _ptr(xh), _stream())
+    return xh
+
+
+def linear_xh(xh: torch.Tensor, code_u32: torch.Tensor, rout: torch.Tensor, K: int, IC: int,
+              OC: int, bias: torch.Tensor | None = None, dtype: torch.dtype = torch.float16,
+              rs: float = RS) -> torch.Tensor:
+    """``linear`` from rows already input-transformed (16 rows and more) -> y [m, OC] of
+    `dtype`, the same bits."""
+    _dev(xh, code_u32, rout, bias)
+    m = xh.shape[0]
+    if xh.dtype != torch.float16 or tuple(xh.shape) != (m, IC):
+        raise ValueError(f"xh must be f16 [m, {IC}]")
+    y = torch.empty((m, OC), dtype=dtype, device=xh.device)
+    if m == 0:
+        return y
+    ws = torch.empty(max(linear_workspace(m, K, IC, OC), 4), dtype=torch.uint8, device=xh.device)
+    _lib.call("esc_linear_xh", _ptr(xh), _ptr(_as_u32(code_u32)), _ptr(rout), _ptr(bias), m, K, IC,
+              OC, rs, _ptr(y), ROWS_DTYPES[dtype], _ptr(ws), ws.numel(), _stream())
+    return y
 
 
 def _ptr_array(ts) -> ctypes.Array:

@@ -180,8 +180,9 @@ int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t*
 /* Two coded linears over the same rows x f16 [M][IC] in one dispatch:
  * y0 = esc_linear(x; rin0, code0, rout0, bias0, K0, OC0) and likewise y1
  * (K0 and K1 may differ), each bit-identical to its own esc_linear call.
- * M < 16: one launch whose workgroups run either projection's plan; M >= 16:
- * the two linears one after the other.  ws: esc_linear_pair_workspace bytes
+ * M < 16: one launch whose workgroups run either projection's plan; M >= 16: one
+ * pass over x for both input transforms and one launch for both products where K
+ * and the split counts agree, else the two linears one after the other.  ws: esc_linear_pair_workspace bytes
  * (projection 0's esc_linear workspace, then projection 1's), zero-filled
  * before its first use.  Replaces dense.project_pair with msl.dense_gemm_pair
  * / dense_gemm_pair_out and the pair transforms (escha_mlx/dense.py:365-437,
@@ -192,6 +193,29 @@ int esc_linear_pair(const uint16_t* x, int M, int IC, const float* rin0, const u
                     const uint32_t* code1, const float* rout1, const uint16_t* bias1, int K1,
                     int OC1, int use_lut, float rs, uint16_t* y0, uint16_t* y1, void* ws,
                     size_t ws_bytes, void* stream);
+
+/* esc_linear_pair for rows of another element type, as esc_linear_typed. */
+int esc_linear_pair_typed(const void* x, int dtype, int M, int IC, const float* rin0,
+                          const uint32_t* code0, const float* rout0, const uint16_t* bias0, int K0,
+                          int OC0, const float* rin1, const uint32_t* code1, const float* rout1,
+                          const uint16_t* bias1, int K1, int OC1, int use_lut, float rs, void* y0,
+                          void* y1, void* ws, size_t ws_bytes, void* stream);
+
+/* esc_linear from rows that are already input-transformed (M >= 16): y [M][OC] of
+ * element type y_dtype, the bits of esc_linear_typed where ws has
+ * esc_linear_workspace bytes (its first bytes hold the splits' partials; a smaller
+ * or null ws takes one launch).  The second half of EschaLinear.__call__
+ * (escha_mlx/dense.py:346-362). */
+int esc_linear_xh(const uint16_t* xh, const uint32_t* code, const float* rout,
+                  const uint16_t* bias, int M, int K, int IC, int OC, float rs, void* y,
+                  int y_dtype, void* ws, size_t ws_bytes, void* stream);
+
+/* The SwiGLU of esc_moe_shared_act and the next projection's input transform in
+ * one pass: xh f16 [m][I] = f16(H128(f32(h) * rin) * rs), h = f16((g / (1 + exp(-g)))
+ * * u), g and u [m][I] of element type dtype, rounded to f16 first (the fused MLP of
+ * escha_mlx/models/qwen3_5.py:63-87 with escha_mlx/dense.py:287-298). */
+int esc_act_transform(const void* g, const void* u, int dtype, const float* rin, int m, int I,
+                      float rs, uint16_t* xh, void* stream);
 
 /* n (1 to 4) coded linears of the same input rows x f16 [M][IC]:
  * y[i] = esc_linear(x; rin[i], code[i], rout[i], bias[i], K, OC[i]) for the

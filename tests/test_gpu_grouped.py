@@ -63,3 +63,26 @@ def test_build_groups_many_rows(m, E):
     ri, ge = R.build_groups(re, E, 16, ng)
     assert np.array_equal(rows_idx.cpu().numpy(), ri)
     assert np.array_equal(group_expert.cpu().numpy(), ge)
+
+
+@pytest.mark.parametrize("T,E,k", [(2, 1, 1), (3, 64, 8), (2, 65, 32), (4, 256, 8), (2, 257, 2), (2, 1024, 32)])
+def test_route_topk_edges(T, E, k):
+    """Widths around each per-lane count, ties within and across lanes, masked
+    logits (the type's lowest value, -inf) and NaN, which is never chosen: ids
+    exact, scores as the router test's 2e-6."""
+    rng = np.random.default_rng(T + E + k)
+    lg = rng.integers(-6, 6, size=(T, E)).astype(np.float32)  # many ties
+    free = np.arange(E) % 3 != 1
+    if free.sum() >= k and E > 64:
+        lg[0, ~free] = np.finfo(np.float32).min
+        lg[1, ~free] = -np.inf
+    ids, sc = ops().route_topk(torch.from_numpy(lg).to(DEV), k)
+    want_ids, want_sc = R.route_topk(lg, k)
+    assert np.array_equal(ids.cpu().numpy(), want_ids)
+    assert np.allclose(sc.cpu().numpy(), want_sc, rtol=2e-6, atol=0)
+    if E >= 2 * k:
+        nan = rng.integers(-6, 6, size=(T, E)).astype(np.float32)
+        nan[:, 1::2] = np.nan
+        ids, _ = ops().route_topk(torch.from_numpy(nan).to(DEV), k)
+        want, _ = R.route_topk(np.where(np.isnan(nan), -np.inf, nan), k)
+        assert np.array_equal(ids.cpu().numpy(), want)

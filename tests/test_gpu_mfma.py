@@ -218,3 +218,50 @@ def test_linear_split_steps(K, ic, oc, m, dtype):
     one = ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d, ws=ws)
     want = ops().gemm_mfma_out(ops().scaled_had(x, rin_d, None), code, rout_d, K, ic, oc, bias=bias_d)
     assert torch.equal(one, want.to(dtype))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("K,ic,ocs,m", [(2, 512, (384, 1280), 17), (3, 1280, (256, 256), 40),
+                                        (2, 2560, (640, 512), 33)])
+def test_pair_many_rows_bit_identical(K, ic, ocs, m, dtype):
+    """Two projections of the same rows from 16 rows on (one transform pass, one
+    product launch where the splits agree): the bits of each one's own call."""
+    rng = np.random.default_rng(7 * K + m)
+    x = torch.from_numpy(rng.standard_normal((m, ic)).astype(np.float32)).to(dtype).to(DEV)
+    ps = []
+    for oc in ocs:
+        _, code = _code(rng, ic, oc, K)
+        rin = torch.from_numpy(rng.choice([-1.0, 1.0], ic).astype(np.float32)).to(DEV)
+        bias = torch.from_numpy((rng.standard_normal(oc) * 0.05).astype(np.float16)).to(DEV)
+        ps.append((code, rin, torch.from_numpy(_rout(rng, oc)).to(DEV), K, oc, bias))
+    got = ops().linear_pair(x, ps[0], ps[1])
+    for y, (code, rin, rout, _, oc, bias) in zip(got, ps):
+        assert torch.equal(y, ops().linear(x, code, rin, rout, K, ic, oc, bias=bias))
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("m,I", [(1, 128), (17, 384), (70, 1280)])
+def test_act_transform_is_act_then_transform(m, I, dtype):
+    """One pass against the two calls it replaces, bit for bit (infinities and large
+    negative gates included), and linear_xh against linear's own GEMM."""
+    rng = np.random.default_rng(m + I)
+    g = rng.standard_normal((m, I)).astype(np.float32) * 4
+    g[0, :3] = [-60.0, 60.0, np.inf]
+    g = torch.from_numpy(g).to(dtype).to(DEV)
+    u = torch.from_numpy(rng.standard_normal((m, I)).astype(np.float32)).to(dtype).to(DEV)
+    rin = torch.from_numpy(rng.choice([-1.0, 1.0], I).astype(np.float32)).to(DEV)
+    got = ops().act_transform(g, u, rin)
+    h = ops().moe_shared_act(g.half(), u.half())
+    want = ops().scaled_had(h, rin, None)
+    assert np.array_equal(got.cpu().numpy().view(np.uint16)[1:], want.cpu().numpy().view(np.uint16)[1:])
+    a, b = got[0].float(), want[0].float()
+    assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(a.nan_to_num(), b.nan_to_num())
+    if m >= 16:
+        _, code = _code(rng, I, 256, 2)
+        rout = torch.from_numpy(_rout(rng, 256)).to(DEV)
+        y = ops().linear_xh(got[1:], code, rout, 2, I, 256, dtype=dtype)
+        assert y.dtype == dtype and y.shape == (m - 1, 256)
+        ref = ops().linear_xh(want[1:].contiguous(), code, rout, 2, I, 256)
+        assert torch.equal(y, ref.to(dtype))
