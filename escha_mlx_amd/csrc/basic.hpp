@@ -271,16 +271,17 @@ __device__ __forceinline__ void topk_wave(float (&v)[NPER], int E, int top_k, in
 
 // logits [T][E] f32 -> ids [T][k] (descending, ties -> lower id), scores [T][k]
 // = softmax over the k selected logits (escha_mlx/ref.py:326-331).
-// One wave per token; E <= 64 NPER.
-template <int NPER>
-__global__ __launch_bounds__(64) void k_route_topk(const float* __restrict__ logits, int E,
+// One wave per token; E <= 64 NPER.  LT: float, or half_t (the router's own f16
+// logits, the same values as a float32 copy of them).
+template <int NPER, typename LT>
+__global__ __launch_bounds__(64) void k_route_topk(const LT* __restrict__ logits, int E,
                                                    int top_k, int* __restrict__ ids,
                                                    float* __restrict__ scores) {
   const int tok = blockIdx.x, lane = threadIdx.x;
-  const float* lg = logits + (size_t)tok * E;
+  const LT* lg = logits + (size_t)tok * E;
   float v[NPER];
 #pragma unroll
-  for (int i = 0; i < NPER; ++i) v[i] = lg[min(lane + 64 * i, E - 1)];
+  for (int i = 0; i < NPER; ++i) v[i] = (float)lg[min(lane + 64 * i, E - 1)];
   int id;
   float val;
   topk_wave(v, E, top_k, id, val);

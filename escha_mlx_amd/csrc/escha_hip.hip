@@ -560,6 +560,17 @@ int launch_rows1(esc::ProjArgs& a, int K, hipStream_t s, bool merged = false) {
                 : launch_rows1_k<3, kTablePairs3>(a, (int)grid, s);
 }
 
+template <typename LT>
+int route_rows(const LT* logits, int T, int E, int top_k, int32_t* ids, float* scores,
+               hipStream_t s) {
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(T), dim3(64), 0, s, logits, E, top_k, ids, scores);
+  };
+  if (E <= 256) go(esc::k_route_topk<4, LT>);
+  else go(esc::k_route_topk<16, LT>);
+  return launched("k_route_topk");
+}
+
 // k_combine, 8 columns per thread where the rows allow 16-byte accesses.
 int combine_rows(const uint16_t* d16, const float* scores, int T, int top_k, int H, uint16_t* y,
                  hipStream_t s) {
@@ -1106,12 +1117,7 @@ int esc_route_topk(const float* logits, int T, int E, int top_k, int32_t* ids, f
   ESC_REQUIRE(top_k >= 1 && top_k <= 32 && top_k <= E, "top_k %d not in [1, min(32, E)]", top_k);
   ESC_REQUIRE(T >= 0, "negative token count");
   if (T == 0) return ESC_OK;
-  auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(T), dim3(64), 0, S(stream), logits, E, top_k, ids, scores);
-  };
-  if (E <= 256) go(esc::k_route_topk<4>);
-  else go(esc::k_route_topk<16>);
-  return launched("k_route_topk");
+  return route_rows(logits, T, E, top_k, ids, scores, S(stream));
 }
 
 int esc_swiglu(const uint16_t* gu, int m, int I, uint16_t* h, void* stream) {
@@ -1291,6 +1297,32 @@ int rows_gemv(const uint16_t* x, const void* w, const float* scale, int M, int K
   }
   return ESC_OK;
 }
+
+// Projections of the same rows: one k_rows_gemm_multi launch (32 rows a
+// workgroup: a router and a shared expert are narrow) where all are narrow enough
+// to share the chip, else each as its own call.
+int rows_multi(int n, const uint16_t* x, const void* const* w, const float* const* scale,
+               uint16_t* const* y, const int* O, int M, int K, hipStream_t s) {
+  long blocks = 0;
+  esc::RowsMulti a{};
+  a.n = n;
+  for (int i = 0; i < n; ++i) {
+    a.w[i] = w[i], a.scale[i] = scale[i], a.y[i] = y[i], a.O[i] = O[i];
+    a.blk0[i] = (int)blocks;
+    blocks += (long)((O[i] + 63) / 64) * ((M + 31) / 32);
+  }
+  // (K: what the f16 GEMV of a few rows takes too)
+  if (K % 64 == 0 && K <= 4096 && blocks <= 4L * device_cus()) {
+    hipLaunchKernelGGL(esc::k_rows_gemm_multi<2>, dim3((unsigned)blocks), dim3(256), 0, s, x, a, M, K);
+    return launched("k_rows_gemm_multi");
+  }
+  for (int i = 0; i < n; ++i) {
+    const int rc = scale[i] ? rows_gemv<true>(x, w[i], scale[i], M, K, O[i], y[i], s)
+                            : rows_gemv<false>(x, w[i], nullptr, M, K, O[i], y[i], s);
+    if (rc) return rc;
+  }
+  return ESC_OK;
+}
 }  // namespace
 
 extern "C" {
@@ -1327,7 +1359,7 @@ int esc_moe_block_out(const uint16_t* y, const uint16_t* sh, const uint16_t* shg
   ESC_REQUIRE(m >= 0 && H > 0, "bad m=%d / H=%d", m, H);
   if (m == 0) return ESC_OK;
   hipLaunchKernelGGL(esc::k_block_out, dim3((H + 255) / 256, m), dim3(256), 0, S(stream), y, sh,
-                     shg, H, out);
+                     shg, H, static_cast<void*>(out), ESC_ROWS_F16);
   return launched("k_block_out");
 }
 
@@ -1967,6 +1999,64 @@ int moe_expert_path(const void* x, int dtype, const int32_t* ids, const float* s
   return launched("k_moe_combine");
 }
 
+// ---- the whole MoE block: offsets of its scratch
+struct BlockScratch {
+  size_t logits, shg, g, u, hh, ids, scores, y, sh, total;
+};
+BlockScratch block_scratch(int T, int top_k, int E, int H, int Ish) {
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at += (bytes + 255) & ~size_t(255);
+    return o;
+  };
+  BlockScratch b{};
+  b.logits = take((size_t)T * E * 2);
+  b.shg = take((size_t)T * 2);
+  b.g = take((size_t)T * Ish * 2);
+  b.u = take((size_t)T * Ish * 2);
+  b.hh = take((size_t)T * Ish * 2);
+  b.ids = take((size_t)T * top_k * 4);
+  b.scores = take((size_t)T * top_k * 4);
+  b.y = take((size_t)T * H * 2);
+  b.sh = take((size_t)T * H * 2);
+  b.total = at;
+  return b;
+}
+
+// Tokens up to which k_block_head / k_block_tail take the block's projections.
+constexpr int kBlockFewTokens = 4;
+
+template <int NR>
+int block_head_nr(const esc::BlockHead& a, hipStream_t s) {
+  const dim3 grid((a.E + 1 + 2 * a.Ish + 3) / 4), blk(256);
+  switch ((a.H + 511) / 512) {
+    case 1: hipLaunchKernelGGL((esc::k_block_head<NR, 1>), grid, blk, 0, s, a); break;
+    case 2: hipLaunchKernelGGL((esc::k_block_head<NR, 2>), grid, blk, 0, s, a); break;
+    case 3: hipLaunchKernelGGL((esc::k_block_head<NR, 3>), grid, blk, 0, s, a); break;
+    case 4: hipLaunchKernelGGL((esc::k_block_head<NR, 4>), grid, blk, 0, s, a); break;
+    case 5:
+    case 6: hipLaunchKernelGGL((esc::k_block_head<NR, 6>), grid, blk, 0, s, a); break;
+    default: hipLaunchKernelGGL((esc::k_block_head<NR, 8>), grid, blk, 0, s, a);
+  }
+  return launched("k_block_head");
+}
+int block_head(const esc::BlockHead& a, hipStream_t s) {
+  return a.T == 1 ? block_head_nr<1>(a, s) : a.T == 2 ? block_head_nr<2>(a, s) : block_head_nr<4>(a, s);
+}
+
+template <int NR>
+int block_tail_nr(const esc::BlockTail& a, hipStream_t s) {
+  const dim3 grid((a.H + 3) / 4), blk(256);
+  if (a.Ish <= 1024) hipLaunchKernelGGL((esc::k_block_tail<NR, 1>), grid, blk, 0, s, a);
+  else if (a.Ish <= 2048) hipLaunchKernelGGL((esc::k_block_tail<NR, 2>), grid, blk, 0, s, a);
+  else hipLaunchKernelGGL((esc::k_block_tail<NR, 4>), grid, blk, 0, s, a);
+  return launched("k_block_tail");
+}
+int block_tail(const esc::BlockTail& a, hipStream_t s) {
+  return a.T == 1 ? block_tail_nr<1>(a, s) : a.T == 2 ? block_tail_nr<2>(a, s) : block_tail_nr<4>(a, s);
+}
+
 // ---- the expert path without allocation: a file-scope device scratch array
 // Its counters sit in the first kStaticIntBytes (zeroed once per device at
 // set-up, left zero by every call), the float data after them.
@@ -2089,6 +2179,66 @@ int esc_moe_expert_path_static(const uint16_t* x, const int32_t* ids, const floa
   return moe_expert_path(x, ESC_ROWS_F16, ids, scores, T, top_k, E, H, I, gu_code, gu_rin, gu_rout,
                          K_gu, dn_code, dn_rin, dn_rout, K_dn, use_lut, y, ptr, kStaticScratchBytes,
                          kStaticIntBytes, stream);
+}
+
+size_t esc_moe_block_scratch(int T, int top_k, int E, int H, int Ish) {
+  if (T <= 0 || top_k <= 0 || E <= 0 || H <= 0 || Ish <= 0) return 0;
+  return block_scratch(T, top_k, E, H, Ish).total;
+}
+
+int esc_moe_block(const void* x, int dtype, const uint16_t* xf, int T, int top_k, int E, int H,
+                  int I, int Ish, const uint16_t* gate_w, const uint16_t* shg_w,
+                  const int8_t* sg_w, const float* sg_s, const int8_t* su_w, const float* su_s,
+                  const int8_t* sd_w, const float* sd_s, const uint32_t* gu_code,
+                  const float* gu_rin, const float* gu_rout, int K_gu, const uint32_t* dn_code,
+                  const float* dn_rin, const float* dn_rout, int K_dn, int use_lut, void* out,
+                  void* scratch, size_t scratch_bytes, void* ws, size_t ws_bytes, void* stream) {
+  ESC_REQUIRE(x && xf && gate_w && shg_w && sg_w && sg_s && su_w && su_s && sd_w && sd_s && out,
+              "null pointer");
+  ESC_REQUIRE(dtype == ESC_ROWS_F16 || dtype == ESC_ROWS_BF16 || dtype == ESC_ROWS_F32,
+              "row element type must be ESC_ROWS_F16, ESC_ROWS_BF16 or ESC_ROWS_F32, got %d",
+              dtype);
+  ESC_REQUIRE(T >= 0, "negative token count");
+  ESC_REQUIRE(E > 0 && E <= 1024, "expert count %d not in [1, 1024]", E);
+  ESC_REQUIRE(top_k >= 1 && top_k <= 32 && top_k <= E, "top_k %d not in [1, min(32, E)]", top_k);
+  ESC_REQUIRE(Ish > 0, "bad shared expert width %d", Ish);
+  if (T == 0) return ESC_OK;
+  const BlockScratch b = block_scratch(T, top_k, E, H, Ish);
+  if (!scratch || scratch_bytes < b.total)
+    return fail(ESC_ENOSPACE, "scratch %zu bytes < required %zu", scratch_bytes, b.total);
+  char* p = static_cast<char*>(scratch);
+  auto u16 = [&](size_t off) { return reinterpret_cast<uint16_t*>(p + off); };
+  uint16_t *logits = u16(b.logits), *shg = u16(b.shg), *g = u16(b.g), *u = u16(b.u);
+  uint16_t *y = u16(b.y), *sh = u16(b.sh);
+  int32_t* ids = reinterpret_cast<int32_t*>(p + b.ids);
+  float* scores = reinterpret_cast<float*>(p + b.scores);
+  hipStream_t s = S(stream);
+  // what the separate calls take: 128..4096 inputs of 16
+  const bool few = T <= kBlockFewTokens && H % 16 == 0 && H >= 128 && H <= 4096 && Ish % 16 == 0 &&
+                   Ish >= 128 && Ish <= 4096;
+  if (few) {
+    if (int rc = block_head({xf, gate_w, shg_w, sg_w, su_w, sg_s, su_s, logits, shg, g, u, T, E, H,
+                             Ish}, s))
+      return rc;
+  } else {
+    const void* w[] = {gate_w, shg_w, sg_w, su_w};
+    const float* sc[] = {nullptr, nullptr, sg_s, su_s};
+    uint16_t* o[] = {logits, shg, g, u};
+    const int O[] = {E, 1, Ish, Ish};
+    if (int rc = rows_multi(4, xf, w, sc, o, O, T, H, s)) return rc;
+  }
+  if (int rc = route_rows(reinterpret_cast<const esc::half_t*>(logits), T, E, top_k, ids, scores, s))
+    return rc;
+  if (int rc = esc_moe_expert_path_typed(x, dtype, ids, scores, T, top_k, E, H, I, gu_code, gu_rin,
+                                         gu_rout, K_gu, dn_code, dn_rin, dn_rout, K_dn, use_lut, y,
+                                         ws, ws_bytes, stream))
+    return rc;
+  if (few) return block_tail({g, u, shg, y, sd_w, sd_s, out, dtype, T, H, Ish}, s);
+  if (int rc = esc_moe_shared_act(g, u, T, Ish, u16(b.hh), stream)) return rc;
+  if (int rc = esc_w8a16(u16(b.hh), sd_w, sd_s, T, Ish, H, sh, stream)) return rc;
+  hipLaunchKernelGGL(esc::k_block_out, dim3((H + 255) / 256, T), dim3(256), 0, s, y, sh, shg, H, out,
+                     dtype);
+  return launched("k_block_out");
 }
 
 size_t esc_moe_layers_workspace(int L, int T, int top_k, int H, int I) {

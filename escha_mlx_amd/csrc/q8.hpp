@@ -315,15 +315,18 @@ __device__ __forceinline__ void rows_store4(uint16_t* y, int row, int o, int O, 
 // VALU per weight and 16 NRB rows) and the matrix pipe.  Measured on MI355X: 1000
 // rows x 4096 channels, K = 2048: see rows_gemm.  K a multiple of 64, at most
 // 8192; grid ceil(O / 64) * ceil(M / (16 NRB)), column blocks fastest, block 256.
+template <int NRB>
+using RowsGemmLds = f32x4_t[4][4][NRB < 4 ? NRB : 4][64];  // [channels][wave][row block][lane]
+
 template <bool Q8, int NRB>
-__global__ __launch_bounds__(256, 2) void k_rows_gemm(const uint16_t* __restrict__ x,
-                                                      const void* __restrict__ wv,
-                                                      const float* __restrict__ scale, int M,
-                                                      int K, int O, uint16_t* __restrict__ y) {
+__device__ __forceinline__ void rows_gemm_body(const uint16_t* __restrict__ x,
+                                               const void* __restrict__ wv,
+                                               const float* __restrict__ scale, int M, int K,
+                                               int O, uint16_t* __restrict__ y, int cb, int rb,
+                                               RowsGemmLds<NRB>& s_acc) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int c = lane & 15, g = lane >> 4;
-  const int ncb = (O + 63) / 64;
-  const int o0 = (blockIdx.x % ncb) * 64, row0 = (blockIdx.x / ncb) * 16 * NRB;
+  const int o0 = cb * 64, row0 = rb * 16 * NRB;
   const int NS = K / 64, s0 = NS * wave / 4, s1 = NS * (wave + 1) / 4;
   // channels past O and rows past M read the last one and are not stored;
   // uniform bases and 32-bit byte offsets (at most 128 rows of 16 KiB)
@@ -375,7 +378,6 @@ __global__ __launch_bounds__(256, 2) void k_rows_gemm(const uint16_t* __restrict
   // rounds of up to four row blocks: every wave hands the channels of the
   // others over and sums its own
   constexpr int RR = NRB < 4 ? NRB : 4;
-  __shared__ f32x4_t s_acc[4][4][RR][64];  // [channel group][wave][row block][lane]
 #pragma unroll
   for (int r0 = 0; r0 < NRB; r0 += RR) {
     if (r0) __syncthreads();
@@ -399,6 +401,41 @@ __global__ __launch_bounds__(256, 2) void k_rows_gemm(const uint16_t* __restrict
       rows_store4(y, row, o, O, v);
     }
   }
+}
+
+template <bool Q8, int NRB>
+__global__ __launch_bounds__(256, 2) void k_rows_gemm(const uint16_t* __restrict__ x,
+                                                      const void* __restrict__ wv,
+                                                      const float* __restrict__ scale, int M,
+                                                      int K, int O, uint16_t* __restrict__ y) {
+  __shared__ RowsGemmLds<NRB> s_acc;
+  const int ncb = (O + 63) / 64;
+  rows_gemm_body<Q8, NRB>(x, wv, scale, M, K, O, y, blockIdx.x % ncb, blockIdx.x / ncb, s_acc);
+}
+
+// Several projections of the same rows in one launch (an MoE block's router gate,
+// shared-expert gate logit, and shared gate and up): each alone leaves most of the
+// chip idle.  blk0: the projection's first workgroup.
+constexpr int kRowsMultiMax = 4;
+struct RowsMulti {
+  const void* w[kRowsMultiMax];
+  const float* scale[kRowsMultiMax];  // null: f16 weights
+  uint16_t* y[kRowsMultiMax];
+  int O[kRowsMultiMax], blk0[kRowsMultiMax];
+  int n;
+};
+
+template <int NRB>
+__global__ __launch_bounds__(256, 2) void k_rows_gemm_multi(const uint16_t* __restrict__ x,
+                                                            RowsMulti a, int M, int K) {
+  __shared__ RowsGemmLds<NRB> s_acc;
+  int i = 0;
+  while (i + 1 < a.n && (int)blockIdx.x >= a.blk0[i + 1]) ++i;
+  const int O = a.O[i], b = blockIdx.x - a.blk0[i], ncb = (O + 63) / 64;
+  if (a.scale[i])
+    rows_gemm_body<true, NRB>(x, a.w[i], a.scale[i], M, K, O, a.y[i], b % ncb, b / ncb, s_acc);
+  else
+    rows_gemm_body<false, NRB>(x, a.w[i], nullptr, M, K, O, a.y[i], b % ncb, b / ncb, s_acc);
 }
 
 // The same product where there are tiles enough to fill the chip: k_gemm_mma2's
@@ -527,21 +564,199 @@ __global__ __launch_bounds__(256) void k_act_transform(const void* __restrict__ 
   }
 }
 
+// sigmoid of an f16 logit, in float32.
+__device__ __forceinline__ float sigmoid16(uint16_t v) {
+  return 1.0f / (1.0f + expf(-(float)__builtin_bit_cast(half_t, v)));
+}
+
+// One element of the block's output in element type dt: f16(f32(y) + f32(sh) *
+// sg), converted.
+__device__ __forceinline__ void block_store(void* out, int dt, size_t i, half_t y, half_t sh,
+                                            float sg) {
+  const half_t v = to_f16((float)y + (float)sh * sg);
+  if (dt == kRowsF32)
+    static_cast<float*>(out)[i] = (float)v;
+  else
+    static_cast<uint16_t*>(out)[i] =
+        dt == kRowsBF16 ? (uint16_t)pack2_bf16((float)v, 0.f) : __builtin_bit_cast(uint16_t, v);
+}
+
+// acc[m] = sum over one weight row (chunks 16-byte pieces, piece lane + 64j by
+// lane) of x row m (m < M <= NR) x weight, summed over the wave: k_rows_gemv's
+// products and order at 64 lanes per row.
+template <bool Q8, int NR, int CPL>
+__device__ __forceinline__ void wave_row_dot(const uint16_t* __restrict__ x, int M, int K,
+                                             const void* __restrict__ row, float s, float* acc) {
+  constexpr int CW = Q8 ? 16 : 8;
+  const int lane = threadIdx.x & 63, chunks = K / CW;
+  const float ms = -128.f * s;
+  uint4 w[CPL];
+#pragma unroll
+  for (int j = 0; j < CPL; ++j)
+    w[j] = static_cast<const uint4*>(row)[min(lane + 64 * j, chunks - 1)];
+  uint4 xv[NR][CPL][CW / 8];
+#pragma unroll
+  for (int m = 0; m < NR; ++m)
+#pragma unroll
+    for (int j = 0; j < CPL; ++j)
+#pragma unroll
+      for (int i = 0; i < CW / 8; ++i)
+        xv[m][j][i] = reinterpret_cast<const uint4*>(
+            x + (size_t)min(m, M - 1) * K)[min(lane + 64 * j, chunks - 1) * (CW / 8) + i];
+#pragma unroll
+  for (int m = 0; m < NR; ++m) acc[m] = 0.f;
+#pragma unroll
+  for (int j = 0; j < CPL; ++j) {
+    // pieces past the row's end: zero weights (an int8 zero is 128 - 128, so the
+    // converted words are cleared)
+    const bool has = lane + 64 * j < chunks;
+    uint32_t wp[CW / 2];
+    const uint32_t ww[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
+    if constexpr (Q8) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w8_to_f16x4(ww[i], s, ms, wp[2 * i], wp[2 * i + 1]);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) wp[i] = ww[i];
+    }
+#pragma unroll
+    for (int m = 0; m < NR; ++m) {
+      float t = acc[m];
+#pragma unroll
+      for (int i = 0; i < CW / 8; ++i) {
+        t = dot2(xv[m][j][i].x, wp[4 * i], t);
+        t = dot2(xv[m][j][i].y, wp[4 * i + 1], t);
+        t = dot2(xv[m][j][i].z, wp[4 * i + 2], t);
+        t = dot2(xv[m][j][i].w, wp[4 * i + 3], t);
+      }
+      acc[m] = has ? t : acc[m];
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < NR; ++m) acc[m] = row_sum<64>(acc[m]);
+}
+
+// An MoE block's first projections for up to NR decode tokens, one output channel
+// per wave: the router's E logits and the shared expert's gate logit (f16 weights),
+// the shared gate and up (int8).  One launch for four: at one token each is a few
+// us of latency (1,281 rows of 2 to 4 KiB).  CF = ceil(H / 512).  grid
+// ceil((E + 1 + 2 Ish) / 4), block 256.
+struct BlockHead {
+  const uint16_t *x, *gate_w, *shg_w;
+  const int8_t *sg_w, *su_w;
+  const float *sg_s, *su_s;
+  uint16_t *logits, *shg, *g, *u;  // [T][E], [T], [T][Ish]
+  int T, E, H, Ish;
+};
+template <int NR, int CF>
+__global__ __launch_bounds__(256) void k_block_head(BlockHead a) {
+  const int lane = threadIdx.x & 63;
+  int o = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  float acc[NR];
+  uint16_t* y;
+  int ldy;
+  if (o <= a.E) {
+    const uint16_t* row = o < a.E ? a.gate_w + (size_t)o * a.H : a.shg_w;
+    wave_row_dot<false, NR, CF>(a.x, a.T, a.H, row, 0.f, acc);
+    y = o < a.E ? a.logits + o : a.shg;
+    ldy = o < a.E ? a.E : 1;
+  } else {
+    o -= a.E + 1;
+    if (o >= 2 * a.Ish) return;
+    const bool up = o >= a.Ish;
+    if (up) o -= a.Ish;
+    const float s = (up ? a.su_s : a.sg_s)[o];
+    wave_row_dot<true, NR, (CF + 1) / 2>(a.x, a.T, a.H, (up ? a.su_w : a.sg_w) + (size_t)o * a.H,
+                                         s, acc);
+    y = (up ? a.u : a.g) + o;
+    ldy = a.Ish;
+  }
+#pragma unroll
+  for (int m = 0; m < NR; ++m)
+    if (lane == 0 && m < a.T) y[(size_t)m * ldy] = __builtin_bit_cast(uint16_t, to_f16(acc[m]));
+}
+
+// The block's end for up to NR tokens, one output channel per wave: the shared
+// expert's activation of its Ish inputs (each wave its own copy: 16 exponentials per
+// lane), its down projection, and out = y + sh * sigmoid(shg).  Three launches in
+// one.  CQ = ceil(Ish / 1024).  grid ceil(H / 4), block 256.
+struct BlockTail {
+  const uint16_t *g, *u, *shg, *y;  // y: the routed sum [T][H]
+  const int8_t* sd_w;
+  const float* sd_s;
+  void* out;
+  int odt, T, H, Ish;
+};
+template <int NR, int CQ>
+__global__ __launch_bounds__(256) void k_block_tail(BlockTail a) {
+  const int lane = threadIdx.x & 63;
+  const int o = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+  if (o >= a.H) return;
+  const int chunks = a.Ish / 16;
+  const float s = a.sd_s[o], ms = -128.f * s;
+  uint4 w[CQ];
+#pragma unroll
+  for (int j = 0; j < CQ; ++j)
+    w[j] = reinterpret_cast<const uint4*>(a.sd_w + (size_t)o * a.Ish)[min(lane + 64 * j, chunks - 1)];
+  half_t yv = (half_t)0.f;
+  uint16_t sg = 0;
+  if (lane < a.T) {
+    yv = __builtin_bit_cast(half_t, a.y[(size_t)lane * a.H + o]);
+    sg = a.shg[lane];
+  }
+  float acc[NR];
+#pragma unroll
+  for (int m = 0; m < NR; ++m) {
+    acc[m] = 0.f;
+    const int row = min(m, a.T - 1);
+#pragma unroll
+    for (int j = 0; j < CQ; ++j) {
+      const size_t at = (size_t)row * a.Ish + 16 * min(lane + 64 * j, chunks - 1);
+      const uint4* gp = reinterpret_cast<const uint4*>(a.g + at);
+      const uint4* up = reinterpret_cast<const uint4*>(a.u + at);
+      const uint4 g0 = gp[0], g1 = gp[1], u0 = up[0], u1 = up[1];
+      const uint32_t gw[8] = {g0.x, g0.y, g0.z, g0.w, g1.x, g1.y, g1.z, g1.w};
+      const uint32_t uw[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
+      const uint32_t ww[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
+      uint32_t wp[8];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) w8_to_f16x4(ww[i], s, ms, wp[2 * i], wp[2 * i + 1]);
+      float t = acc[m];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        half_t hh[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const float gf = (float)__builtin_bit_cast(half_t, (uint16_t)(gw[i] >> (16 * e)));
+          const float uf = (float)__builtin_bit_cast(half_t, (uint16_t)(uw[i] >> (16 * e)));
+          hh[e] = to_f16((gf / (1.0f + expf(-gf))) * uf);
+        }
+        t = dot2(pack2(hh[0], hh[1]), wp[i], t);
+      }
+      acc[m] = lane + 64 * j < chunks ? t : acc[m];
+    }
+    acc[m] = row_sum<64>(acc[m]);
+  }
+  // lane m writes token m
+#pragma unroll
+  for (int m = 0; m < NR; ++m)
+    if (lane == m && m < a.T)
+      block_store(a.out, a.odt, (size_t)m * a.H + o, yv, to_f16(acc[m]), sigmoid16(sg));
+}
+
 // Block output (escha_mlx/ref.py:346-349, models/qwen3_5_moe.py:270-272):
 // out = f16(f32(y) + f32(sh) * sigmoid(f32(shg))), y the f16 routed sum, sh
 // the shared expert's f16 output, shg [m] the f16 shared gate logit.
-// grid (ceil(H/256), m), block 256.
+// odt: the element type out is written in.  grid (ceil(H/256), m), block 256.
 __global__ __launch_bounds__(256) void k_block_out(const uint16_t* __restrict__ yr,
                                                    const uint16_t* __restrict__ sh,
                                                    const uint16_t* __restrict__ shg, int H,
-                                                   uint16_t* __restrict__ out) {
+                                                   void* __restrict__ out, int odt) {
   const int c = blockIdx.x * 256 + threadIdx.x, row = blockIdx.y;
   if (c >= H) return;
   const size_t o = (size_t)row * H + c;
-  const float sg = 1.0f / (1.0f + expf(-(float)__builtin_bit_cast(half_t, shg[row])));
-  const float v = (float)__builtin_bit_cast(half_t, yr[o]) +
-                  (float)__builtin_bit_cast(half_t, sh[o]) * sg;
-  out[o] = __builtin_bit_cast(uint16_t, to_f16(v));
+  block_store(out, odt, o, __builtin_bit_cast(half_t, yr[o]), __builtin_bit_cast(half_t, sh[o]),
+              sigmoid16(shg[row]));
 }
 
 }  // namespace esc

@@ -60,6 +60,11 @@ def apply_bias() -> bool:
     return envs.parse_bool("ESCHA_MLX_BIAS", False)
 
 
+def hooked(*modules: torch.nn.Module) -> bool:
+    """Whether a module has forward hooks, which a fused path would pass by."""
+    return any(m._forward_hooks or m._forward_pre_hooks for m in modules)
+
+
 def dense_block_r(m: int, pin: int | None = None) -> int:
     """Rows per group: min(m, 16) snapped down to a power of two (msl.py:1562-1601)."""
     if pin is not None:
@@ -294,7 +299,8 @@ class EschaMLP(torch.nn.Module):
         gate, up = project_pair(self.gate_proj, self.up_proj, x)
         down = self.down_proj
         m = gate.numel() // gate.shape[-1]
-        if m >= ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_DTYPES and down.plain():
+        if (m >= ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_DTYPES and down.plain()
+                and type(down) is EschaLinear and not hooked(down)):
             # the activation and down's input transform in one pass
             w = down._w
             xh = ops.act_transform(gate.reshape(m, w.IC), up.reshape(m, w.IC), w.rin)

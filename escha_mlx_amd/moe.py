@@ -22,7 +22,7 @@ from __future__ import annotations
 import numpy as np
 import torch
 
-from . import envs, ops, quant
+from . import dense, envs, ops, quant
 
 RS = ops.RS
 
@@ -154,6 +154,19 @@ class EschaMoEExperts(torch.nn.Module):
                                     lut=self._lut)
         return ops.moe_combine(d16, scores.reshape(-1).contiguous(), self.top_k)
 
+    def _workspace(self, t: int, x: torch.Tensor, one: bool) -> torch.Tensor:
+        # one zero-initialised workspace per token count and form: the one-launch
+        # path keeps its counters there and leaves them zero after every call,
+        # and the two forms lay their counters out differently
+        # (float32 rows take the chain, which keeps none, at every shape)
+        key = (t, x.device, "chain" if x.dtype == torch.float32 else one)
+        ws = self._ws.get(key)
+        if ws is None:
+            need = ops.moe_expert_path_workspace(t, self.top_k, self.num_experts, x.shape[1],
+                                                 self._inter)
+            ws = self._ws[key] = torch.zeros(max(need, 4), dtype=torch.uint8, device=x.device)
+        return ws
+
     def forward(self, x: torch.Tensor, ids: torch.Tensor, scores: torch.Tensor) -> torch.Tensor:
         """y f16 [T, H], the routed sum rounded to f16 (models/qwen3_5_moe.py:253).
         bf16 / f32 rows are transformed from their float32 values
@@ -170,15 +183,7 @@ class EschaMoEExperts(torch.nn.Module):
         # ESCHA_HIP_MOE_ONE_LAUNCH: one launch wherever that launch takes the shape
         one = (self._one_launch and x.dtype == torch.float16
                and ops.moe_one_launch_takes(t, self.top_k, h, self._inter))
-        # one zero-initialised workspace per token count and form: the one-launch
-        # path keeps its counters there and leaves them zero after every call,
-        # and the two forms lay their counters out differently
-        # (float32 rows take the chain, which keeps none, at every shape)
-        key = (t, x.device, "chain" if x.dtype == torch.float32 else one)
-        ws = self._ws.get(key)
-        if ws is None:
-            need = ops.moe_expert_path_workspace(t, self.top_k, self.num_experts, h, self._inter)
-            ws = self._ws[key] = torch.zeros(max(need, 4), dtype=torch.uint8, device=x.device)
+        ws = self._workspace(t, x, one)
         gu, dn = self._gu, self._dn
         return ops.moe_expert_path(x, ids, scores, gu.code, gu.rin, gu.rout, gu.K, dn.code,
                                    dn.rin, dn.rout, dn.K, lut=self._lut, ws=ws, one_launch=one)
@@ -228,6 +233,17 @@ class EschaSparseMoeBlock(torch.nn.Module):
         shape = x.shape
         rows = ops.as_rows(x.reshape(-1, shape[-1]))
         xf = rows.to(torch.float16).contiguous()
+        ex = self.experts
+        if (not ex._exact and ex._fused_had and not ex._one_launch and rows.shape[0]
+                and not dense.hooked(ex, self.sh_gate, self.sh_up, self.sh_down)):
+            gu, dn = ex._gu, ex._dn
+            out = ops.moe_block(rows, xf, self.top_k, self.gate_w, self.shg_w,
+                                (self.sh_gate.w8, self.sh_gate.scale),
+                                (self.sh_up.w8, self.sh_up.scale),
+                                (self.sh_down.w8, self.sh_down.scale),
+                                (gu.code, gu.rin, gu.rout, gu.K), (dn.code, dn.rin, dn.rout, dn.K),
+                                ex._workspace(rows.shape[0], rows, False), lut=ex._lut)
+            return out.reshape(shape).to(x.dtype)
         logits = ops.gemv_f16w(xf, self.gate_w).to(torch.float32)
         ids, scores = route(logits, self.top_k)
         y = self.experts(rows, ids, scores)

@@ -494,6 +494,35 @@ def moe_expert_path(x, ids, scores, gu_code, gu_rin, gu_rout, K_gu, dn_code, dn_
     return y
 
 
+def moe_block(x, xf, top_k, gate_w, shg_w, sh_gate, sh_up, sh_down, gu, dn, ws, lut=None):
+    """The whole MoE block for rows x [T, H] (xf: the rows as f16; x itself if they are)
+    -> [T, H] in x's type (models/qwen3_5_moe.py:257-273).  sh_*: (int8 [N, K], f32 [N])
+    of the shared expert, gu / dn: (code, rin, rout, K) of the experts, ws: a
+    workspace of moe_expert_path_workspace bytes, zero-filled before its first use."""
+    _dev(x, xf, gate_w, shg_w, *sh_gate, *sh_up, *sh_down, *gu[:3], *dn[:3], ws)
+    t, h = x.shape
+    E, I, ish = gate_w.shape[0], gu[2].shape[1] // 2, sh_gate[0].shape[0]
+    if x.dtype not in ROWS_DTYPES or xf.dtype != torch.float16 or tuple(xf.shape) != (t, h):
+        raise ValueError("x must be [T, H] of a floating type and xf its f16 rows")
+    shapes = {"gate_w": (gate_w, (E, h)), "shg_w": (shg_w, (1, h)), "sh_gate": (sh_gate[0], (ish, h)),
+              "sh_up": (sh_up[0], (ish, h)), "sh_down": (sh_down[0], (h, ish))}
+    for name, (w, want) in shapes.items():
+        if tuple(w.shape) != want:
+            raise ValueError(f"{name} must be {want}, got {tuple(w.shape)}")
+    out = torch.empty_like(x)
+    if t == 0:
+        return out
+    scratch = torch.empty(_lib.load().esc_moe_block_scratch(t, top_k, E, h, ish),
+                          dtype=torch.uint8, device=x.device)
+    _lib.call("esc_moe_block", _ptr(x), ROWS_DTYPES[x.dtype], _ptr(xf), t, top_k, E, h, I, ish,
+              _ptr(gate_w), _ptr(shg_w), _ptr(sh_gate[0]), _ptr(sh_gate[1]), _ptr(sh_up[0]),
+              _ptr(sh_up[1]), _ptr(sh_down[0]), _ptr(sh_down[1]), _ptr(_as_u32(gu[0])), _ptr(gu[1]),
+              _ptr(gu[2]), gu[3], _ptr(_as_u32(dn[0])), _ptr(dn[1]), _ptr(dn[2]), dn[3],
+              _lut_flag(lut), _ptr(out), _ptr(scratch), scratch.numel(), _ptr(ws), ws.numel(),
+              _stream())
+    return out
+
+
 def moe_expert_path_static_max() -> int:
     """Bytes of the device scratch array esc_moe_expert_path_static uses."""
     return int(_lib.load().esc_moe_expert_path_static_max())

@@ -411,6 +411,23 @@ typedef struct {
   uint16_t* y;
 } esc_moe_layer;
 
+/* The whole MoE block for T tokens (EschaSparseMoeBlock.__call__,
+ * escha_mlx/models/qwen3_5_moe.py:257-273): router logits f16 = xf @ gate_w^T
+ * ([E][H] f16), top_k of them, the routed experts (esc_moe_expert_path_typed on x of
+ * element type dtype), the shared expert (int8 gate, up [Ish][H], down [H][Ish] with
+ * float32 scales per row) scaled by sigmoid(xf @ shg_w), added to the f16 routed sum;
+ * out [T][H] of x's element type.  xf: x rounded to f16 (x itself for f16 rows).
+ * The same values as the separate calls up to the order of float32 sums.  scratch:
+ * esc_moe_block_scratch bytes; ws: esc_moe_expert_path_workspace bytes, as there. */
+size_t esc_moe_block_scratch(int T, int top_k, int E, int H, int Ish);
+int esc_moe_block(const void* x, int dtype, const uint16_t* xf, int T, int top_k, int E, int H,
+                  int I, int Ish, const uint16_t* gate_w, const uint16_t* shg_w,
+                  const int8_t* sg_w, const float* sg_s, const int8_t* su_w, const float* su_s,
+                  const int8_t* sd_w, const float* sd_s, const uint32_t* gu_code,
+                  const float* gu_rin, const float* gu_rout, int K_gu, const uint32_t* dn_code,
+                  const float* dn_rin, const float* dn_rout, int K_dn, int use_lut, void* out,
+                  void* scratch, size_t scratch_bytes, void* ws, size_t ws_bytes, void* stream);
+
 /* L independent token-layers of routed experts in one launch (throughput
  * mode: large items, the layers' work overlaps).  layers = device array of L
  * records; every layer has the same T, top_k, E, H, I, K_gu, K_dn.  ws must be

@@ -190,3 +190,39 @@ def test_many_rows_vs_f64(m, K, O, q8):
     assert np.array_equal(got[0].view(np.uint16), wf[:, K - 1].view(np.uint16))
     err = (np.abs(got - want).max(axis=1) / np.abs(want).max(axis=1)).max()
     assert err < 2e-3, err
+
+
+# ---- the MoE block as one call: its few-token kernels at 1, 2, 3 and 4 tokens, the
+# merged projections above; hidden sizes around a 512-input piece, shared widths of
+# one piece, a ragged piece and two pieces per lane
+@pytest.mark.parametrize("T,H,ish", [(1, 512, 128), (2, 640, 384), (3, 2048, 512), (4, 1664, 1152),
+                                     (5, 640, 384), (40, 1024, 512)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["f16", "bf16", "f32"])
+def test_moe_block_call_vs_separate_calls(T, H, ish, dtype):
+    """Against the same module with a hook on its shared gate, which takes the
+    separate calls: the same rounding points, float32 sums in another order, so
+    single f16 roundings differ (the block tests' 5e-3 of the largest output)."""
+    from escha_mlx_amd import moe
+    E, I, k = 24, 256, 3
+    rng = np.random.default_rng(T + H + ish)
+
+    def experts(K, ic, oc):
+        code = rng.integers(-32768, 32768, size=(E, ic // 16, oc // 16, 16 * K), dtype=np.int16)
+        sign = lambda n: rng.choice([-1.0, 1.0], (E, n)).astype(np.float32)
+        return moe.EschaExperts(code, sign(ic), sign(oc) * 0.04, device=DEV)
+
+    gu, dn = experts(2, H, 2 * I), experts(3, I, H)
+    q8 = lambda n, kk: rng.integers(-127, 128, size=(n, kk), dtype=np.int8)
+    sc = lambda n, kk: (rng.uniform(0.5, 1.5, n) * 0.013 / np.sqrt(kk)).astype(np.float32)
+    shared = {"gate_w8": q8(ish, H), "gate_scale": sc(ish, H), "up_w8": q8(ish, H),
+              "up_scale": sc(ish, H), "down_w8": q8(H, ish), "down_scale": sc(H, ish)}
+    blk = moe.EschaSparseMoeBlock(H, E, k, gu, dn, rng.standard_normal((E, H)) / np.sqrt(H),
+                                  rng.standard_normal((1, H)) / np.sqrt(H), shared)
+    x = torch.from_numpy(rng.standard_normal((T, H)).astype(np.float32)).to(dtype).to(DEV)
+    y = blk(x)
+    assert y.dtype == dtype and torch.equal(blk(x), y)
+    handle = blk.sh_gate.register_forward_hook(lambda *a: None)
+    want = blk(x)
+    handle.remove()
+    assert _rel(y.float().cpu().numpy(), want.float().cpu().numpy()) < 5e-3
