@@ -363,10 +363,10 @@ int gemm_mma2_out(int K, const MmaPlan& plan, const esc::MmaArgs& a, hipStream_t
 constexpr int kLinearSmallRows = 16;
 constexpr int kLinearSmallRowsLut = 8;
 
-// Linears below kLinearSmallRows rows read f16 rows only.
+// Linears below kLinearSmallRows rows read 16-bit rows only.
 int check_rows_type(int dtype, int M) {
-  ESC_REQUIRE(dtype == ESC_ROWS_F16 || ((dtype == ESC_ROWS_BF16 || dtype == ESC_ROWS_F32) &&
-                                        (M >= kLinearSmallRows || M == 0)),
+  ESC_REQUIRE(dtype == ESC_ROWS_F16 || dtype == ESC_ROWS_BF16 ||
+                  (dtype == ESC_ROWS_F32 && (M >= kLinearSmallRows || M == 0)),
               "row element type %d with %d rows", dtype, M);
   return ESC_OK;
 }
@@ -460,49 +460,47 @@ LinearPlan linear_plan(int M, int K, int IC, int OC, bool lut) {
   return p;
 }
 
-esc::LinearSmallArgs small_args(const uint16_t* x, const float* rin, const uint32_t* code,
+esc::LinearSmallArgs small_args(const void* x, const float* rin, const uint32_t* code,
                                 const float* rout, const uint16_t* bias, int M, int TK, int TN,
-                                const LinearPlan& lp, float rs, float* part, int* cnt,
-                                uint16_t* y) {
-  return {x, rin, code, rout, bias, M, TK, TN, lp.KS, lp.R, lp.S, lp.groups, lp.row_groups, rs,
-          part, cnt, y};
+                                const LinearPlan& lp, float rs, char* ws, void* y, int dt,
+                                int ydt, const void* x2 = nullptr) {
+  return {static_cast<const uint16_t*>(x), rin, code, rout, bias, M, TK, TN, lp.KS, lp.R, lp.S,
+          lp.groups, lp.row_groups, rs, reinterpret_cast<float*>(ws + lp.off_part),
+          reinterpret_cast<int*>(ws + lp.off_cnt), y, static_cast<const uint16_t*>(x2), dt, ydt};
 }
 
-template <int K, bool LUT>
-struct LinearSmallF {
-  static int run(const esc::LinearSmallArgs& a, hipStream_t s) {
-    // one row: VALU GEMV; several rows: matrix-core row-blocked GEMM
-    constexpr int RMAX = LUT ? kLinearSmallRowsLut : kLinearSmallRows;
-    if (a.R < 1 || a.R > RMAX) return fail(ESC_EINVAL, "rows per group %d > %d", a.R, RMAX);
-    const dim3 grid(a.groups, a.row_groups, a.S);
-    if (a.R == 1)
-      hipLaunchKernelGGL((esc::k_linear_small<K, LUT, 1>), grid, dim3(256), 0, s, a);
-    else
-      hipLaunchKernelGGL((esc::k_linear_small<K, LUT, RMAX>), grid, dim3(256), 0, s, a);
-    return launched("k_linear_small");
-  }
-};
+// one row: VALU GEMV; several rows: matrix-core row-blocked GEMM
+template <int K, bool ACT>
+int linear_small_launch(const esc::LinearSmallArgs& a, hipStream_t s) {
+  if (a.R < 1 || a.R > kLinearSmallRows)
+    return fail(ESC_EINVAL, "rows per group %d > %d", a.R, kLinearSmallRows);
+  const dim3 grid(a.groups, a.row_groups, a.S);
+  if (a.R == 1)
+    hipLaunchKernelGGL((esc::k_linear_small<K, 1, ACT>), grid, dim3(256), 0, s, a);
+  else
+    hipLaunchKernelGGL((esc::k_linear_small<K, kLinearSmallRows, ACT>), grid, dim3(256), 0, s, a);
+  return launched("k_linear_small");
+}
 
-template <int K0, int K1, bool LUT>
+template <int K0, int K1>
 int linear_pair_launch(const esc::LinearSmallArgs& a0, const esc::LinearSmallArgs& a1,
                        hipStream_t s) {
-  constexpr int RMAX = LUT ? kLinearSmallRowsLut : kLinearSmallRows;
+  constexpr int RMAX = kLinearSmallRows;
   if (a0.R != a1.R || a0.R < 1 || a0.R > RMAX)
     return fail(ESC_EINVAL, "rows per group %d / %d (max %d)", a0.R, a1.R, RMAX);
   const long n = (long)a0.groups * a0.row_groups * a0.S + (long)a1.groups * a1.row_groups * a1.S;
   if (a0.R == 1)
-    hipLaunchKernelGGL((esc::k_linear_pair<K0, K1, LUT, 1>), dim3(n), dim3(256), 0, s, a0, a1);
+    hipLaunchKernelGGL((esc::k_linear_pair<K0, K1, 1>), dim3(n), dim3(256), 0, s, a0, a1);
   else
-    hipLaunchKernelGGL((esc::k_linear_pair<K0, K1, LUT, RMAX>), dim3(n), dim3(256), 0, s, a0, a1);
+    hipLaunchKernelGGL((esc::k_linear_pair<K0, K1, RMAX>), dim3(n), dim3(256), 0, s, a0, a1);
   return launched("k_linear_pair");
 }
 
-template <bool LUT>
 int linear_pair_k(int K0, int K1, const esc::LinearSmallArgs& a0, const esc::LinearSmallArgs& a1,
                   hipStream_t s) {
-  if (K0 == 2) return K1 == 2 ? linear_pair_launch<2, 2, LUT>(a0, a1, s)
-                              : linear_pair_launch<2, 3, LUT>(a0, a1, s);
-  return K1 == 2 ? linear_pair_launch<3, 2, LUT>(a0, a1, s) : linear_pair_launch<3, 3, LUT>(a0, a1, s);
+  if (K0 == 2) return K1 == 2 ? linear_pair_launch<2, 2>(a0, a1, s)
+                              : linear_pair_launch<2, 3>(a0, a1, s);
+  return K1 == 2 ? linear_pair_launch<3, 2>(a0, a1, s) : linear_pair_launch<3, 3>(a0, a1, s);
 }
 
 // k_proj_rows1 over a.np projections whose x .. TK, TN are filled: each
@@ -511,16 +509,16 @@ int linear_pair_k(int K0, int K1, const esc::LinearSmallArgs& a0, const esc::Lin
 // previous projection's.  K=2 decodes kTablePairsLayers of 8 pairs from the
 // table, K=3 4 of 8, whichever decode was asked for (q, k and v of 5120 inputs in
 // one launch, K=2: 18.7 us against 20.8 by hash alone; level at 2048 and 4096).
-template <int K, int NT>
+template <int K, int NT, bool ACT>
 int launch_rows1_k(const esc::ProjArgs& a, int grid, hipStream_t s) {
   static std::once_flag once;
   static hipError_t err = hipSuccess;
   std::call_once(once, [] {
-    err = hipFuncSetAttribute((const void*)esc::k_proj_rows1<K, NT>,
+    err = hipFuncSetAttribute((const void*)esc::k_proj_rows1<K, NT, ACT>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, 65536 * 2);
   });
   if (int rc = hip_check(err, "hipFuncSetAttribute")) return rc;
-  hipLaunchKernelGGL((esc::k_proj_rows1<K, NT>), dim3(grid), dim3(64 * esc::kProjWaves), 65536 * 2,
+  hipLaunchKernelGGL((esc::k_proj_rows1<K, NT, ACT>), dim3(grid), dim3(64 * esc::kProjWaves), 65536 * 2,
                      s, a);
   return launched("k_proj_rows1");
 }
@@ -539,7 +537,8 @@ int rows1_workgroups(long n, long wgs) {
 // merged: the workgroups shared out over the projections by their units
 // (one round of workgroups for several small projections); otherwise each
 // projection's from its own size alone, so that its outputs are those of
-// its own launch.
+// its own launch.  With x2 (one projection) the row is the MLP activation of x
+// and x2.
 int launch_rows1(esc::ProjArgs& a, int K, hipStream_t s, bool merged = false) {
   const int cus = device_cus();
   long total = 0;
@@ -556,8 +555,52 @@ int launch_rows1(esc::ProjArgs& a, int K, hipStream_t s, bool merged = false) {
     q.wg0 = (int)grid;
     grid += q.G;
   }
-  return K == 2 ? launch_rows1_k<2, esc::kTablePairsLayers>(a, (int)grid, s)
-                : launch_rows1_k<3, kTablePairs3>(a, (int)grid, s);
+  if (a.pr[0].x2)
+    return K == 2 ? launch_rows1_k<2, esc::kTablePairsLayers, true>(a, (int)grid, s)
+                  : launch_rows1_k<3, kTablePairs3, true>(a, (int)grid, s);
+  return K == 2 ? launch_rows1_k<2, esc::kTablePairsLayers, false>(a, (int)grid, s)
+                : launch_rows1_k<3, kTablePairs3, false>(a, (int)grid, s);
+}
+
+esc::ProjOne rows1_proj(const void* x, const void* x2, const float* rin, const uint32_t* code,
+                        const float* rout, const uint16_t* bias, int IC, int OC, char* part,
+                        char* cnt, void* y) {
+  esc::ProjOne q{};
+  q.x = static_cast<const uint16_t*>(x);
+  q.rin = rin;
+  q.code = code;
+  q.rout = rout;
+  q.bias = bias;
+  q.y = y;
+  q.part = reinterpret_cast<float*>(part);
+  q.cnt = reinterpret_cast<int*>(cnt);
+  q.TK = IC / 16;
+  q.TN = OC / 16;
+  q.x2 = static_cast<const uint16_t*>(x2);
+  return q;
+}
+
+// One linear of fewer than kLinearSmallRows rows (or, with x2, of the MLP
+// activation of x and x2): one launch.
+int linear_few(const void* x, const void* x2, int dt, const float* rin, const uint32_t* code,
+               const float* rout, const uint16_t* bias, int M, int K, int IC, int OC, float rs,
+               void* y, int ydt, const LinearPlan& lp, char* w, hipStream_t s) {
+  if (rows1_single(M, IC, OC)) {
+    // one row: the persistent kernel, its counters at off_cnt and its
+    // partials at off_part (linear_plan sizes both)
+    esc::ProjArgs a{};
+    a.np = 1;
+    a.rs = rs;
+    a.dt = dt;
+    a.ydt = ydt;
+    a.pr[0] = rows1_proj(x, x2, rin, code, rout, bias, IC, OC, w + lp.off_part, w + lp.off_cnt, y);
+    return launch_rows1(a, K, s);
+  }
+  // the split-K kernel, by hash
+  const esc::LinearSmallArgs a = small_args(x, rin, code, rout, bias, M, IC / 16, OC / 16, lp, rs,
+                                            w, y, dt, ydt, x2);
+  if (x2) return K == 2 ? linear_small_launch<2, true>(a, s) : linear_small_launch<3, true>(a, s);
+  return K == 2 ? linear_small_launch<2, false>(a, s) : linear_small_launch<3, false>(a, s);
 }
 
 template <typename LT>
@@ -722,27 +765,9 @@ int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t*
   const int TK = IC / 16, TN = OC / 16;
   hipStream_t s = S(stream);
   char* w = static_cast<char*>(ws);
-  const uint16_t* x16 = static_cast<const uint16_t*>(x);
-  uint16_t* y16 = static_cast<uint16_t*>(y);
-  if (rows1_single(M, IC, OC)) {
-    // one row: the persistent kernel, its counters at off_cnt and its
-    // partials at off_part (linear_plan sizes both)
-    esc::ProjArgs a{};
-    a.np = 1;
-    a.rs = rs;
-    a.pr[0] = esc::ProjOne{x16, rin, code, rout, bias, y16,
-                           reinterpret_cast<float*>(w + lp.off_part),
-                           reinterpret_cast<int*>(w + lp.off_cnt), TK, TN};
-    return launch_rows1(a, K, s);
-  }
-  if (M < kLinearSmallRows) {
-    // the split-K kernel, by hash
-    float* part = reinterpret_cast<float*>(w + lp.off_part);
-    int* cnt = reinterpret_cast<int*>(w + lp.off_cnt);
-    const esc::LinearSmallArgs a =
-        small_args(x16, rin, code, rout, bias, M, TK, TN, lp, rs, part, cnt, y16);
-    return K == 2 ? LinearSmallF<2, false>::run(a, s) : LinearSmallF<3, false>::run(a, s);
-  }
+  if (M < kLinearSmallRows)
+    return linear_few(x, nullptr, dtype, rin, code, rout, bias, M, K, IC, OC, rs, y, dtype, lp, w,
+                      s);
   // many rows: input transform, then the matrix-core GEMM with the output
   // transform in its epilogue, or in its splits' reduction.  A workspace with
   // no room for the partials takes the one launch.
@@ -752,6 +777,23 @@ int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t*
   const esc::MmaArgs a{xh, code, M, TK, TN, reinterpret_cast<float*>(w + lp.off_mid),
                        rout, bias, rs, y, dtype};
   return gemm_mma2_out(K, plan, a, s);
+}
+
+int esc_linear_act(const void* g, const void* u, int dtype, const float* rin,
+                   const uint32_t* code, const float* rout, const uint16_t* bias, int M, int K,
+                   int IC, int OC, float rs, void* y, int y_dtype, void* ws, size_t ws_bytes,
+                   void* stream) {
+  if (int rc = check_proj(K, IC, OC)) return rc;
+  ESC_REQUIRE(g && u && rin && code && rout && y, "null pointer");
+  ESC_REQUIRE(M >= 0 && M < kLinearSmallRows, "%d rows (fewer than %d)", M, kLinearSmallRows);
+  if (M == 0) return ESC_OK;
+  if (int rc = check_rows_type(dtype, M)) return rc;
+  if (int rc = check_rows_type(y_dtype, M)) return rc;
+  const LinearPlan lp = linear_plan(M, K, IC, OC, rows1_single(M, IC, OC));
+  if (!ws || ws_bytes < lp.total)
+    return fail(ESC_ENOSPACE, "workspace %zu bytes < required %zu", ws_bytes, lp.total);
+  return linear_few(g, u, dtype, rin, code, rout, bias, M, K, IC, OC, rs, y, y_dtype, lp,
+                    static_cast<char*>(ws), S(stream));
 }
 
 int esc_linear_xh(const uint16_t* xh, const uint32_t* code, const float* rout,
@@ -876,8 +918,6 @@ int esc_linear_pair_typed(const void* x, int dtype, int M, int IC, const float* 
     if (int rc = mma2_reduce(K0, Sp, a0, s)) return rc;
     return mma2_reduce(K0, Sp, a1, s);
   }
-  const uint16_t* x16 = static_cast<const uint16_t*>(x);
-  uint16_t *y0 = static_cast<uint16_t*>(y0v), *y1 = static_cast<uint16_t*>(y1v);
   const bool r0 = rows1_single(M, IC, OC0), r1 = rows1_single(M, IC, OC1);
   const int TK = IC / 16;
   const LinearPlan p0 = linear_plan(M, K0, IC, OC0, r0);
@@ -889,31 +929,28 @@ int esc_linear_pair_typed(const void* x, int dtype, int M, int IC, const float* 
     esc::ProjArgs a{};
     a.np = 2;
     a.rs = rs;
-    a.pr[0] = esc::ProjOne{x16, rin0, code0, rout0, bias0, y0,
-                           reinterpret_cast<float*>(w + p0.off_part),
-                           reinterpret_cast<int*>(w + p0.off_cnt), TK, OC0 / 16};
-    a.pr[1] = esc::ProjOne{x16, rin1, code1, rout1, bias1, y1,
-                           reinterpret_cast<float*>(w1 + p1.off_part),
-                           reinterpret_cast<int*>(w1 + p1.off_cnt), TK, OC1 / 16};
+    a.dt = a.ydt = dtype;
+    a.pr[0] = rows1_proj(x, nullptr, rin0, code0, rout0, bias0, IC, OC0, w + p0.off_part,
+                         w + p0.off_cnt, y0v);
+    a.pr[1] = rows1_proj(x, nullptr, rin1, code1, rout1, bias1, IC, OC1, w1 + p1.off_part,
+                         w1 + p1.off_cnt, y1v);
     return launch_rows1(a, K0, S(stream));
   }
   if (r0 || r1 || p0.R != p1.R) {
     // one row with the projections on different kernels (or K), or row
     // groups of different sizes: each as its own call
-    if (int rc = esc_linear(x16, rin0, code0, rout0, bias0, M, K0, IC, OC0, use_lut, rs, y0, w, ws0,
-                            stream))
+    if (int rc = esc_linear_typed(x, dtype, rin0, code0, rout0, bias0, M, K0, IC, OC0, use_lut, rs,
+                                  y0v, w, ws0, stream))
       return rc;
-    return esc_linear(x16, rin1, code1, rout1, bias1, M, K1, IC, OC1, use_lut, rs, y1, w + off1,
-                      ws_bytes - off1, stream);
+    return esc_linear_typed(x, dtype, rin1, code1, rout1, bias1, M, K1, IC, OC1, use_lut, rs, y1v,
+                            w1, ws_bytes - off1, stream);
   }
-  const esc::LinearSmallArgs a0 =
-      small_args(x16, rin0, code0, rout0, bias0, M, TK, OC0 / 16, p0, rs,
-                 reinterpret_cast<float*>(w + p0.off_part), reinterpret_cast<int*>(w + p0.off_cnt), y0);
-  const esc::LinearSmallArgs a1 =
-      small_args(x16, rin1, code1, rout1, bias1, M, TK, OC1 / 16, p1, rs,
-                 reinterpret_cast<float*>(w1 + p1.off_part), reinterpret_cast<int*>(w1 + p1.off_cnt), y1);
+  const esc::LinearSmallArgs a0 = small_args(x, rin0, code0, rout0, bias0, M, TK, OC0 / 16, p0, rs,
+                                             w, y0v, dtype, dtype);
+  const esc::LinearSmallArgs a1 = small_args(x, rin1, code1, rout1, bias1, M, TK, OC1 / 16, p1, rs,
+                                             w1, y1v, dtype, dtype);
   // the split-K pair kernel, by hash
-  return linear_pair_k<false>(K0, K1, a0, a1, S(stream));
+  return linear_pair_k(K0, K1, a0, a1, S(stream));
 }
 
 size_t esc_linear_multi_workspace(int M, int n, int K, int IC, const int* OC) {
@@ -937,6 +974,19 @@ int esc_linear_multi(const uint16_t* x, int M, int IC, int K, int n, const uint3
                      const float* const* rin, const float* const* rout,
                      const uint16_t* const* bias, const int* OC, int use_lut, float rs,
                      uint16_t* const* y, void* ws, size_t ws_bytes, void* stream) {
+  ESC_REQUIRE(y, "null pointer");
+  ESC_REQUIRE(n >= 1 && n <= esc::kProjMax, "%d projections (1 to %d)", n, esc::kProjMax);
+  void* yv[esc::kProjMax];
+  for (int i = 0; i < n; ++i) yv[i] = y[i];
+  return esc_linear_multi_typed(x, ESC_ROWS_F16, M, IC, K, n, code, rin, rout, bias, OC, use_lut,
+                                rs, yv, ws, ws_bytes, stream);
+}
+
+int esc_linear_multi_typed(const void* x, int dtype, int M, int IC, int K, int n,
+                           const uint32_t* const* code, const float* const* rin,
+                           const float* const* rout, const uint16_t* const* bias, const int* OC,
+                           int use_lut, float rs, void* const* y, void* ws, size_t ws_bytes,
+                           void* stream) {
   ESC_REQUIRE(x && code && rin && rout && OC && y, "null pointer");
   ESC_REQUIRE(M >= 0, "negative row count");
   ESC_REQUIRE(n >= 1 && n <= esc::kProjMax, "%d projections (1 to %d)", n, esc::kProjMax);
@@ -947,6 +997,7 @@ int esc_linear_multi(const uint16_t* x, int M, int IC, int K, int n, const uint3
     ESC_REQUIRE(M != 1 || OC[i] % 256 == 0, "OC=%d of projection %d is not a multiple of 256",
                 OC[i], i);
   }
+  if (int rc = check_rows_type(dtype, M)) return rc;
   if (M == 0) return ESC_OK;
   const size_t need = esc_linear_multi_workspace(M, n, K, IC, OC);
   if (!ws || ws_bytes < need)
@@ -958,13 +1009,13 @@ int esc_linear_multi(const uint16_t* x, int M, int IC, int K, int n, const uint3
     esc::ProjArgs a{};
     a.np = n;
     a.rs = rs;
+    a.dt = a.ydt = dtype;
     for (int i = 0; i < n; ++i) {
-      int* cnt = reinterpret_cast<int*>(w);
+      char* cnt = w;
       w += ((size_t)(OC[i] / 256) * 4 + 255) / 256 * 256;
-      float* part = reinterpret_cast<float*>(w);
+      a.pr[i] = rows1_proj(x, nullptr, rin[i], code[i], rout[i], bias ? bias[i] : nullptr, IC,
+                           OC[i], w, cnt, y[i]);
       w += rows1_part_bytes(IC / 16, OC[i] / 16);
-      a.pr[i] = esc::ProjOne{x, rin[i], code[i], rout[i], bias ? bias[i] : nullptr, y[i], part,
-                             cnt, IC / 16, OC[i] / 16};
     }
     return launch_rows1(a, K, S(stream), true);
   }
@@ -983,8 +1034,9 @@ int esc_linear_multi(const uint16_t* x, int M, int IC, int K, int n, const uint3
   }
   if (!one) {
     for (int i = 0; i < n; ++i)
-      if (int rc = esc_linear(x, rin[i], code[i], rout[i], bias ? bias[i] : nullptr, M, K, IC,
-                              OC[i], use_lut, rs, y[i], w + off[i], ws_bytes - off[i], stream))
+      if (int rc = esc_linear_typed(x, dtype, rin[i], code[i], rout[i], bias ? bias[i] : nullptr,
+                                    M, K, IC, OC[i], use_lut, rs, y[i], w + off[i],
+                                    ws_bytes - off[i], stream))
         return rc;
     return ESC_OK;
   }
@@ -992,10 +1044,8 @@ int esc_linear_multi(const uint16_t* x, int M, int IC, int K, int n, const uint3
   m.n = n;
   long nw = 0;
   for (int i = 0; i < n; ++i) {
-    char* wi = w + off[i];
-    m.p[i] = small_args(x, rin[i], code[i], rout[i], bias ? bias[i] : nullptr, M, IC / 16, OC[i] / 16,
-                        pl[i], rs, reinterpret_cast<float*>(wi + pl[i].off_part),
-                        reinterpret_cast<int*>(wi + pl[i].off_cnt), y[i]);
+    m.p[i] = small_args(x, rin[i], code[i], rout[i], bias ? bias[i] : nullptr, M, IC / 16,
+                        OC[i] / 16, pl[i], rs, w + off[i], y[i], dtype, dtype);
     nw += (long)pl[i].groups * pl[i].row_groups * pl[i].S;
   }
   ESC_REQUIRE(pl[0].R >= 2 && pl[0].R <= kLinearSmallRows, "rows per group %d", pl[0].R);

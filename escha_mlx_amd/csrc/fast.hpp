@@ -458,6 +458,21 @@ __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
   return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)a) |
          ((uint32_t)__builtin_bit_cast(uint16_t, (__bf16)b) << 16);
 }
+// The f16 value v as element i of y, whose element type is dt (kRowsF16 or
+// kRowsBF16).
+__device__ __forceinline__ void store_row16(void* y, int dt, size_t i, half_t v) {
+  const uint16_t h = __builtin_bit_cast(uint16_t, v);
+  static_cast<uint16_t*>(y)[i] = dt == kRowsBF16 ? (uint16_t)pack2_bf16((float)v, 0.f) : h;
+}
+// The input of a linear: a row element, or (ACT) the MLP's activation of gate and
+// up elements, f16((g / (1 + exp(-g))) * u), bf16 ones rounded to f16 first.
+template <bool ACT>
+__device__ __forceinline__ float linear_input(uint16_t x, uint16_t x2, int dt) {
+  const float v = row_value16(x, dt);
+  if constexpr (!ACT) return v;
+  const float g = (float)(half_t)v, u = (float)(half_t)row_value16(x2, dt);
+  return (float)to_f16((g / (1.0f + expf(-g))) * u);
+}
 __device__ __forceinline__ void st_coherent(float* p, float v) {
   __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __builtin_bit_cast(uint32_t, v),
                      __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -38,24 +38,32 @@ struct LinearSmallArgs {
   float rs;
   float* part;
   int* cnt;
-  uint16_t* y;
+  void* y;
+  const uint16_t* x2;  // ACT: up elements (x: gate)
+  int dt, ydt;         // element types of x (and x2) and of y: kRowsF16 / kRowsBF16
 };
 
-// The workgroup's LDS: decode table (table decode only), the transformed
-// inputs of its rows (after the decode loop: the finishing sums, [R][TPW*16]
+// The workgroup's LDS: the transformed inputs of its rows (after the decode loop: the finishing sums, [R][TPW*16]
 // floats), the VALU path's wave partials.
-template <int K, bool LUT, int RMAX>
+template <int K, int RMAX>
 struct LinearSmallSmem {
-  uint16_t lut[LUT ? 65536 : 1];
   alignas(16) uint32_t x[RMAX][8 * 64];  // up to 64 kt per row
   float red[RMAX > 1 ? 1 : 4][64][Geo<K>::NCOL];
   int last;
   static_assert(Geo<K>::TPW * 16 <= 8 * 64, "finishing sums fit in the input stage");
 };
 
-template <int K, bool LUT, int RMAX>
+// The rows are f16 or bf16 (a.dt), read as float32 before the transform, so bf16
+// decode runs this launch too and not a transform, a split GEMV and a reduction:
+// measured K=3 5120 x 5120, 7 rows 33.7 -> 19.7 us.
+// ACT: the rows are the MLP activation of x and x2 (linear_input), computed with
+// the input transform, so the down projection of a few rows needs no launch and no
+// tensor for it: every column group repeats the activation of its kt range (a few
+// exponentials per lane, under the code's latency).  Measured, the MLP 2048 -> 6144
+// -> 2048, K=2, one row: 47.2 -> 36.0 us.
+template <int K, int RMAX, bool ACT = false>
 __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int ntg, int rg, int z,
-                                                  LinearSmallSmem<K, LUT, RMAX>& sm) {
+                                                  LinearSmallSmem<K, RMAX>& sm) {
   const uint16_t* __restrict__ x = a.x;
   const float* __restrict__ rin = a.rin;
   const uint32_t* __restrict__ code = a.code;
@@ -65,17 +73,14 @@ __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int 
   const float rs = a.rs;
   float* __restrict__ part = a.part;
   int* __restrict__ cnt = a.cnt;
-  uint16_t* __restrict__ y = a.y;
   using G = Geo<K>;
   constexpr int TPS = 16 / G::LPT;
   constexpr int kCols = G::TPW * 16;  // columns per column group
   constexpr int kBlocks = kCols / 128;  // 128-column blocks per group
   constexpr bool kMma = RMAX > 1;
-  uint16_t* s_lut = sm.lut;
   auto& s_x = sm.x;
   auto& s_red = sm.red;
   int& s_last = sm.last;
-  stage_lut<LUT>(s_lut);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int row0 = rg * R;
   const int IC = TK * 16, OC = TN * 16;
@@ -106,7 +111,7 @@ __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int 
   // 8 items
   constexpr int kXB = RMAX > 1 ? 8 : 1;
   for (int base = wave; base < R * nb; base += 4 * kXB) {
-    uint16_t xa[kXB], xb[kXB];
+    uint16_t xa[kXB], xb[kXB], ua[kXB], ub[kXB];
     float ra[kXB], rb[kXB];
     int r = base / nb, b = base - (base / nb) * nb;
 #pragma unroll
@@ -116,6 +121,11 @@ __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int 
         const int cc = 16 * KS * z + 128 * b + 2 * lane;
         xa[j] = x[(size_t)row * IC + cc];
         xb[j] = x[(size_t)row * IC + cc + 1];
+        ua[j] = ub[j] = 0;
+        if constexpr (ACT) {
+          ua[j] = a.x2[(size_t)row * IC + cc];
+          ub[j] = a.x2[(size_t)row * IC + cc + 1];
+        }
         ra[j] = rin[cc];
         rb[j] = rin[cc + 1];
       }
@@ -125,8 +135,8 @@ __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int 
 #pragma unroll
     for (int j = 0; j < kXB; ++j) {
       if (base + 4 * j < R * nb) {
-        float v0 = (float)__builtin_bit_cast(half_t, xa[j]) * ra[j];
-        float v1 = (float)__builtin_bit_cast(half_t, xb[j]) * rb[j];
+        float v0 = linear_input<ACT>(xa[j], ua[j], a.dt) * ra[j];
+        float v1 = linear_input<ACT>(xb[j], ub[j], a.dt) * rb[j];
         h128_wave(v0, v1);
         s_x[r][64 * b + lane] = pack2(to_f16(v0 * rs), to_f16(v1 * rs));
       }
@@ -146,7 +156,7 @@ __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int 
         if (k + 1 < nsteps) nxt = load_lane_words_nt<K>(lp + (size_t)(kt0 + kstep * (k + 1)) * kstride);
         const u32x4_t* xb = reinterpret_cast<const u32x4_t*>(xs + 8 * (4 * k + gk));
         const uint32_t wprev = __shfl(cur.w[G::WPL - 1], src);
-        mma_tile<K, LUT>(cur, wprev, xb[0], xb[1], acc, s_lut);
+        mma_tile<K, false>(cur, wprev, xb[0], xb[1], acc, nullptr);
         cur = nxt;
       }
       if (c < R && row0 + c < M)
@@ -164,7 +174,7 @@ __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int 
       for (int i = 0; i < 8; ++i) xw[i] = s_x[0][8 * (kl0 + k) + i];
       x_pairs(xw, xp[0]);
       const uint32_t wprev = __shfl(cur.w[G::WPL - 1], src);
-      fast_tile_rows<K, LUT, 1>(cur, wprev, xp, s_lut, acc);
+      fast_tile_rows<K, false, 1>(cur, wprev, xp, nullptr, acc);
       cur = nxt;
     }
     // reduce the 4 waves (fixed order) and publish the partials
@@ -303,17 +313,17 @@ __device__ __forceinline__ void linear_small_body(const LinearSmallArgs& a, int 
       y0 = to_f16((float)y0 + bs0);
       y1 = to_f16((float)y1 + bs1);
     }
-    uint16_t* yr = y + (size_t)(row0 + r) * OC + col;
-    yr[0] = __builtin_bit_cast(uint16_t, y0);
-    yr[1] = __builtin_bit_cast(uint16_t, y1);
+    const size_t i = (size_t)(row0 + r) * OC + col;
+    store_row16(a.y, a.ydt, i, y0);
+    store_row16(a.y, a.ydt, i + 1, y1);
   }
 }
 
 
-template <int K, bool LUT, int RMAX>
+template <int K, int RMAX, bool ACT>
 __global__ __launch_bounds__(256) void k_linear_small(LinearSmallArgs a) {
-  __shared__ LinearSmallSmem<K, LUT, RMAX> sm;
-  linear_small_body<K, LUT, RMAX>(a, blockIdx.x, blockIdx.y, blockIdx.z, sm);
+  __shared__ LinearSmallSmem<K, RMAX> sm;
+  linear_small_body<K, RMAX, ACT>(a, blockIdx.x, blockIdx.y, blockIdx.z, sm);
 }
 
 // 1 to 4 projections of the same input rows and K in one launch (an attention
@@ -329,7 +339,7 @@ struct LinearMultiArgs {
 
 template <int K, int RMAX>
 __global__ __launch_bounds__(256) void k_linear_multi(LinearMultiArgs m) {
-  __shared__ LinearSmallSmem<K, false, RMAX> sm;
+  __shared__ LinearSmallSmem<K, RMAX> sm;
   int b = blockIdx.x, i = 0;
   for (; i + 1 < m.n; ++i) {
     const int nw = m.p[i].groups * m.p[i].row_groups * m.p[i].S;
@@ -339,7 +349,7 @@ __global__ __launch_bounds__(256) void k_linear_multi(LinearMultiArgs m) {
   // one body, its arguments chosen per workgroup (as k_linear_pair)
   const LinearSmallArgs& a = m.p[i];
   const int gr = a.groups * a.row_groups;
-  linear_small_body<K, false, RMAX>(a, b % a.groups, (b % gr) / a.groups, b / gr, sm);
+  linear_small_body<K, RMAX>(a, b % a.groups, (b % gr) / a.groups, b / gr, sm);
 }
 
 // Two projections of the same input rows in one launch (the projection-pair
@@ -348,11 +358,11 @@ __global__ __launch_bounds__(256) void k_linear_multi(LinearMultiArgs m) {
 // projection's plan (its own column groups, splits, partials and counters),
 // so each output is bit-identical to its own k_linear_small launch.  The two
 // projections' LDS layouts share one allocation.
-template <int K0, int K1, bool LUT, int RMAX>
+template <int K0, int K1, int RMAX>
 __global__ __launch_bounds__(256) void k_linear_pair(LinearSmallArgs a0, LinearSmallArgs a1) {
   __shared__ union {
-    LinearSmallSmem<K0, LUT, RMAX> p0;
-    LinearSmallSmem<K1, LUT, RMAX> p1;
+    LinearSmallSmem<K0, RMAX> p0;
+    LinearSmallSmem<K1, RMAX> p1;
   } sm;
   const int n0 = a0.groups * a0.row_groups * a0.S;
   const bool first = (int)blockIdx.x < n0;
@@ -362,13 +372,13 @@ __global__ __launch_bounds__(256) void k_linear_pair(LinearSmallArgs a0, LinearS
     // same body would spill)
     const LinearSmallArgs& a = first ? a0 : a1;
     const int gr = a.groups * a.row_groups;
-    linear_small_body<K0, LUT, RMAX>(a, b % a.groups, (b % gr) / a.groups, b / gr, sm.p0);
+    linear_small_body<K0, RMAX>(a, b % a.groups, (b % gr) / a.groups, b / gr, sm.p0);
   } else if (first) {
     const int gr = a0.groups * a0.row_groups;
-    linear_small_body<K0, LUT, RMAX>(a0, b % a0.groups, (b % gr) / a0.groups, b / gr, sm.p0);
+    linear_small_body<K0, RMAX>(a0, b % a0.groups, (b % gr) / a0.groups, b / gr, sm.p0);
   } else {
     const int gr = a1.groups * a1.row_groups;
-    linear_small_body<K1, LUT, RMAX>(a1, b % a1.groups, (b % gr) / a1.groups, b / gr, sm.p1);
+    linear_small_body<K1, RMAX>(a1, b % a1.groups, (b % gr) / a1.groups, b / gr, sm.p1);
   }
 }
 

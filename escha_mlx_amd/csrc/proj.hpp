@@ -42,12 +42,12 @@ constexpr int kProjHashUnits = 1;
 
 // One projection of the launch.
 struct ProjOne {
-  const uint16_t* x;     // [IC] f16 input row
+  const uint16_t* x;     // [IC] input row (f16 or bf16: ProjArgs::dt)
   const float* rin;      // [IC]
   const uint32_t* code;  // [TK][TN][8K]
   const float* rout;     // [OC]
   const uint16_t* bias;  // [OC] f16 or null
-  uint16_t* y;           // [OC] f16
+  void* y;               // [OC] (f16 or bf16: ProjArgs::ydt)
   float* part;           // [TN/16][maxc][256] float32 partials, lane-major
   int* cnt;              // [TN/16] workgroups published per group (zero between calls)
   int TK, TN;            // IC / 16, OC / 16 (TN a multiple of 16)
@@ -55,12 +55,14 @@ struct ProjOne {
   int G;                 // workgroups (at most kProjMaxP units per wave)
   int maxc;              // partial slots per group (>= the workgroups a group spans)
   int wg0;               // first workgroup of this projection in the launch
+  const uint16_t* x2;    // ACT: [IC] up elements (x: gate)
 };
 
 struct ProjArgs {
   ProjOne pr[kProjMax];
-  int np;    // projections
-  float rs;  // the transforms' scale
+  int np;       // projections
+  float rs;     // the transforms' scale
+  int dt, ydt;  // element types of the rows and of the outputs
 };
 
 // LDS of the kernel beyond the table: each wave's partials of its two
@@ -92,19 +94,23 @@ __device__ __forceinline__ const uint32_t* proj_code(const ProjOne& q, const Pro
 
 // the lane's two inputs of block kb and their input scales
 struct ProjIn {
-  uint32_t xw;
+  uint32_t xw, uw;
   float2 ri;
 };
+template <bool ACT>
 __device__ __forceinline__ ProjIn proj_fetch(const ProjOne& q, int kb) {
-  const int lane = threadIdx.x & 63;
-  return ProjIn{*reinterpret_cast<const uint32_t*>(q.x + 128 * kb + 2 * lane),
-                *reinterpret_cast<const float2*>(q.rin + 128 * kb + 2 * lane)};
+  const int lane = threadIdx.x & 63, c = 128 * kb + 2 * lane;
+  ProjIn in{*reinterpret_cast<const uint32_t*>(q.x + c), 0u,
+            *reinterpret_cast<const float2*>(q.rin + c)};
+  if constexpr (ACT) in.uw = *reinterpret_cast<const uint32_t*>(q.x2 + c);
+  return in;
 }
 // the block's 128 inputs, f16(H128(x * rin) * rs), as the decode's paired
 // words (lane j: word j)
-__device__ __forceinline__ uint32_t proj_inputs(const ProjIn& in, float rs) {
-  float v0 = (float)__builtin_bit_cast(half_t, (uint16_t)in.xw) * in.ri.x;
-  float v1 = (float)__builtin_bit_cast(half_t, (uint16_t)(in.xw >> 16)) * in.ri.y;
+template <bool ACT>
+__device__ __forceinline__ uint32_t proj_inputs(const ProjIn& in, float rs, int dt) {
+  float v0 = linear_input<ACT>((uint16_t)in.xw, (uint16_t)in.uw, dt) * in.ri.x;
+  float v1 = linear_input<ACT>((uint16_t)(in.xw >> 16), (uint16_t)(in.uw >> 16), dt) * in.ri.y;
   h128_wave(v0, v1);
   return paired_word(pack2(to_f16(v0 * rs), to_f16(v1 * rs)));
 }
@@ -150,8 +156,11 @@ __device__ __forceinline__ int proj_col(int lane, int ci) {
 }
 
 // grid: the projections' workgroups one after the other (projection j's
-// from pr[j].wg0), 16 waves each; dynamic LDS: the table.
-template <int K, int NT>
+// from pr[j].wg0), 16 waves each; dynamic LDS: the table.  ACT: the row is the MLP
+// activation of x and x2 (linear_input), each wave's own two 128-input blocks of it
+// (K=3 MLP 5120 -> 17408 -> 5120 of one row: 59.3 -> 58.1 us; a bf16 row, read as it
+// is, 5120 -> 17408 K=2: 32.9 -> 20.0 us).
+template <int K, int NT, bool ACT>
 __global__ __launch_bounds__(64 * kProjWaves) void k_proj_rows1(ProjArgs p) {
   static_assert(NT > 0, "");
   extern __shared__ uint16_t s_dyn[];
@@ -177,7 +186,7 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_proj_rows1(ProjArgs p) {
   LaneWords<K> w[K == 3 ? 2 : 1];
   proj_load<K>(proj_code<K>(q, c), half_off, off, w);
   const bool two_blocks = cl.g != c.g || (cl.kt >> 3) != (c.kt >> 3);
-  const ProjIn ina = proj_fetch(q, c.kt >> 3), inb = proj_fetch(q, cl.kt >> 3);
+  const ProjIn ina = proj_fetch<ACT>(q, c.kt >> 3), inb = proj_fetch<ACT>(q, cl.kt >> 3);
   // units [a, ub) use block A, [ub, b) block B; [a, ug) group c.g, [ug, b) cl.g
   const int ub = two_blocks ? b - 1 - (cl.kt & 7) : b;
   const int ug = cl.g != c.g ? b - 1 - cl.kt : b;
@@ -186,8 +195,8 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_proj_rows1(ProjArgs p) {
     s_grp[wave][1] = busy && ug < b ? cl.g : -1;
   }
 
-  const uint32_t xa = proj_inputs(ina, p.rs);
-  const uint32_t xb = two_blocks ? proj_inputs(inb, p.rs) : xa;
+  const uint32_t xa = proj_inputs<ACT>(ina, p.rs, p.dt);
+  const uint32_t xb = two_blocks ? proj_inputs<ACT>(inb, p.rs, p.dt) : xa;
   // The table's pieces are requested once the first unit's code and the
   // inputs are in registers (the compiler waits for every outstanding load
   // after a DMA into LDS, so a wait placed later would also wait for the
@@ -352,7 +361,8 @@ __global__ __launch_bounds__(64 * kProjWaves) void k_proj_rows1(ProjArgs p) {
         y0 = to_f16((float)y0 + (float)__builtin_bit_cast(half_t, (uint16_t)bw[blk]));
         y1 = to_f16((float)y1 + (float)__builtin_bit_cast(half_t, (uint16_t)(bw[blk] >> 16)));
       }
-      *reinterpret_cast<uint32_t*>(q.y + col0 + cc) = pack2(y0, y1);
+      reinterpret_cast<uint32_t*>(q.y)[(col0 + cc) >> 1] =
+          p.ydt == kRowsBF16 ? pack2_bf16((float)y0, (float)y1) : pack2(y0, y1);
     }
     lds_wave_sync();
   }

@@ -148,32 +148,36 @@ class EschaLinear(torch.nn.Module):
     def K(self) -> int:
         return self._w.K
 
+    def small(self) -> bool:
+        """Whether 16-bit rows below 16 take the one-launch linear."""
+        return self._fused_had and not self._exact and self._block_r_pin is None
+
     def plain(self) -> bool:
         """Whether 16 rows and more take the matrix-core GEMM with fused transforms."""
-        return (self._mat and self._fused_had and not self._exact and self._block_r_pin is None)
+        return self._mat and self.small()
 
-    def _linear_ws(self, m: int, device) -> torch.Tensor | None:
+    def _linear_ws(self, rows: torch.Tensor) -> torch.Tensor | None:
+        m, w = rows.shape[0], self._w
         if m >= ops.LINEAR_SMALL_ROWS:
             return None  # no counters: a fresh workspace per call
-        key = (m, device)
-        if key not in self._ws:
-            need = ops.linear_workspace(m, self._w.K, self._w.IC, self._w.OC)
-            self._ws[key] = torch.zeros(max(need, 4), dtype=torch.uint8, device=device)
-        return self._ws[key]
+        key = (m, rows.device)
+        if rows.dtype == torch.float16 and key in self._ws:
+            return self._ws[key]
+        return ops.kept_ws(self._ws, key, rows, ops.linear_workspace, m, w.K, w.IC, w.OC)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         w = self._w
         shape = x.shape
         # bf16 / f32 rows are transformed from their float32 values
-        # (dense.py:287-292); below 16 rows in a launch of its own, then the
-        # f16 rows' kernels run from xh
+        # (dense.py:287-292); f32 rows below 16 in a launch of its own, then the
+        # row-blocked kernels run from xh
         rows = ops.as_rows(x.reshape(-1, shape[-1]))
         m = rows.shape[0]
         if (not self._exact and self._block_r_pin is None and self._fused_had
-                and (self._mat if m >= ops.LINEAR_SMALL_ROWS else rows.dtype == torch.float16)):
+                and (self._mat if m >= ops.LINEAR_SMALL_ROWS else rows.dtype in ops.ROWS_16)):
             # the whole linear in esc_linear (one launch below 16 rows)
-            y = ops.linear(rows, w.code, w.rin, w.rout, w.K, w.IC, w.OC, bias=self.bias,
-                           lut=self._lut, ws=self._linear_ws(m, rows.device))
+            y = ops.linear_typed(rows, w.code, w.rin, w.rout, w.K, w.IC, w.OC, bias=self.bias,
+                                 lut=self._lut, ws=self._linear_ws(rows))
             return y.reshape(*shape[:-1], w.OC).to(x.dtype)
         xh = ops.scaled_had(rows, w.rin, None)
         r = dense_block_r(m, self._block_r_pin)
@@ -221,7 +225,7 @@ def project_pair(first: EschaLinear, second: EschaLinear, x: torch.Tensor):
     m = rows.shape[0]
     many = m >= ops.LINEAR_SMALL_ROWS
     compatible = (
-        (rows.dtype == torch.float16 or many and rows.dtype in ops.ROWS_DTYPES)
+        (rows.dtype in ops.ROWS_16 or many and rows.dtype == torch.float32)
         and w0.IC == w1.IC == rows.shape[-1]
         and first._lut == second._lut
         and first._fused_had and second._fused_had
@@ -231,15 +235,13 @@ def project_pair(first: EschaLinear, second: EschaLinear, x: torch.Tensor):
     )
     if not compatible:
         return first(x), second(x)
-    key = (m, rows.device, id(second))
     # no counters from 16 rows on: a fresh workspace per call
-    ws = None if many else first._pair_ws.get(key)
-    if ws is None and not many:
-        need = ops.linear_pair_workspace(m, w0.K, w1.K, w0.IC, w0.OC, w1.OC)
-        ws = first._pair_ws[key] = torch.zeros(max(need, 4), dtype=torch.uint8, device=rows.device)
-    y0, y1 = ops.linear_pair(rows, (w0.code, w0.rin, w0.rout, w0.K, w0.OC, first.bias),
-                             (w1.code, w1.rin, w1.rout, w1.K, w1.OC, second.bias),
-                             lut=first._lut, ws=ws)
+    ws = None if many else ops.kept_ws(first._pair_ws, (m, rows.device, id(second)), rows,
+                                       ops.linear_pair_workspace, m, w0.K, w1.K, w0.IC, w0.OC,
+                                       w1.OC)
+    y0, y1 = ops.linear_pair_typed(rows, (w0.code, w0.rin, w0.rout, w0.K, w0.OC, first.bias),
+                                   (w1.code, w1.rin, w1.rout, w1.K, w1.OC, second.bias),
+                                   lut=first._lut, ws=ws)
     return (y0.reshape(*shape[:-1], w0.OC).to(x.dtype), y1.reshape(*shape[:-1], w1.OC).to(x.dtype))
 
 
@@ -261,7 +263,7 @@ def project_many(linears, x: torch.Tensor):
     ws_ = [lin._w for lin in linears]
     m = rows.shape[0]
     compatible = (
-        rows.dtype == torch.float16 and 2 <= len(linears) <= 4 and 1 <= m < 16
+        rows.dtype in ops.ROWS_16 and 2 <= len(linears) <= 4 and 1 <= m < 16
         and len({w.K for w in ws_}) == 1 and all(w.IC == rows.shape[-1] for w in ws_)
         and (m > 1 or all(w.OC % 256 == 0 for w in ws_))
         and len({lin._lut for lin in linears}) == 1
@@ -271,13 +273,10 @@ def project_many(linears, x: torch.Tensor):
         if len(linears) == 2:
             return list(project_pair(linears[0], linears[1], x))
         return [lin(x) for lin in linears]
-    key = (rows.device, m, tuple(id(lin) for lin in linears[1:]))
-    ws = first._multi_ws.get(key)
-    if ws is None:
-        need = ops.linear_multi_workspace(ws_[0].K, ws_[0].IC, [w.OC for w in ws_], m)
-        ws = first._multi_ws[key] = torch.zeros(max(need, 4), dtype=torch.uint8, device=rows.device)
-    ys = ops.linear_multi(rows, [(w.code, w.rin, w.rout, w.K, w.OC, lin.bias)
-                                 for w, lin in zip(ws_, linears)], lut=first._lut, ws=ws)
+    ws = ops.kept_ws(first._multi_ws, (rows.device, m, tuple(id(lin) for lin in linears[1:])),
+                     rows, ops.linear_multi_workspace, ws_[0].K, ws_[0].IC, [w.OC for w in ws_], m)
+    ys = ops.linear_multi_typed(rows, [(w.code, w.rin, w.rout, w.K, w.OC, lin.bias)
+                                       for w, lin in zip(ws_, linears)], lut=first._lut, ws=ws)
     return [y.reshape(*shape[:-1], w.OC).to(x.dtype) for y, w in zip(ys, ws_)]
 
 
@@ -298,11 +297,19 @@ class EschaMLP(torch.nn.Module):
         shape = x.shape
         gate, up = project_pair(self.gate_proj, self.up_proj, x)
         down = self.down_proj
+        w = down._w
         m = gate.numel() // gate.shape[-1]
-        if (m >= ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_DTYPES and down.plain()
-                and type(down) is EschaLinear and not hooked(down)):
+        fused = type(down) is EschaLinear and not hooked(down)
+        if (fused and 1 <= m < ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_16
+                and x.dtype in ops.ROWS_16 and down.small()):
+            # the activation in down's own launch
+            g = gate.reshape(m, w.IC)
+            y = ops.linear_act(g, up.reshape(m, w.IC), w.code, w.rin, w.rout, w.K, w.IC, w.OC,
+                               down.bias, x.dtype, down._linear_ws(g))
+            return y.reshape(*shape[:-1], w.OC)
+        if (fused and m >= ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_DTYPES
+                and down.plain()):
             # the activation and down's input transform in one pass
-            w = down._w
             xh = ops.act_transform(gate.reshape(m, w.IC), up.reshape(m, w.IC), w.rin)
             dtype = x.dtype if x.dtype in ops.ROWS_DTYPES else torch.float16
             y = ops.linear_xh(xh, w.code, w.rout, w.K, w.IC, w.OC, bias=down.bias, dtype=dtype)
@@ -310,7 +317,7 @@ class EschaMLP(torch.nn.Module):
         g = gate.reshape(-1, gate.shape[-1]).to(torch.float16).contiguous()
         u = up.reshape(-1, up.shape[-1]).to(torch.float16).contiguous()
         h = ops.moe_shared_act(g, u)
-        return self.down_proj(h).reshape(*shape[:-1], self.down_proj._w.OC).to(x.dtype)
+        return down(h).reshape(*shape[:-1], w.OC).to(x.dtype)
 
 
 class EschaKVProjection(torch.nn.Module):

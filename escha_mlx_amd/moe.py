@@ -157,15 +157,15 @@ class EschaMoEExperts(torch.nn.Module):
     def _workspace(self, t: int, x: torch.Tensor, one: bool) -> torch.Tensor:
         # one zero-initialised workspace per token count and form: the one-launch
         # path keeps its counters there and leaves them zero after every call,
-        # and the two forms lay their counters out differently
-        # (float32 rows take the chain, which keeps none, at every shape)
-        key = (t, x.device, "chain" if x.dtype == torch.float32 else one)
-        ws = self._ws.get(key)
-        if ws is None:
-            need = ops.moe_expert_path_workspace(t, self.top_k, self.num_experts, x.shape[1],
-                                                 self._inter)
-            ws = self._ws[key] = torch.zeros(max(need, 4), dtype=torch.uint8, device=x.device)
-        return ws
+        # and the two forms lay their counters out differently.  Rows that are not
+        # f16 and take the chain, which keeps none, get a fresh one per call
+        h = x.shape[1]
+        args = (t, self.top_k, self.num_experts, h, self._inter)
+        if x.dtype == torch.float32 or (x.dtype != torch.float16 and not
+                                        ops.moe_one_launch_takes(t, self.top_k, h, self._inter)):
+            return torch.empty(max(ops.moe_expert_path_workspace(*args), 4), dtype=torch.uint8,
+                               device=x.device)
+        return ops.kept_ws(self._ws, (t, x.device, one), x, ops.moe_expert_path_workspace, *args)
 
     def forward(self, x: torch.Tensor, ids: torch.Tensor, scores: torch.Tensor) -> torch.Tensor:
         """y f16 [T, H], the routed sum rounded to f16 (models/qwen3_5_moe.py:253).

@@ -92,6 +92,7 @@ def decode_tiles(code_u32: torch.Tensor, K: int, IC: int, OC: int,
 
 # element type codes of esc_input_transform_typed (ESC_ROWS_* in escha_hip.h)
 ROWS_DTYPES = {torch.float16: 0, torch.bfloat16: 1, torch.float32: 2}
+ROWS_16 = (torch.float16, torch.bfloat16)
 
 
 def scaled_had(rows: torch.Tensor, rin: torch.Tensor, row_expert: torch.Tensor | None,
@@ -239,6 +240,32 @@ def dense_gemm_rows_direct_out(xh: torch.Tensor, code_u32: torch.Tensor, rout: t
 LINEAR_SMALL_ROWS = 16
 
 
+_STREAM_WS = 64  # per-stream workspaces kept by one module
+
+
+def kept_ws(cache: dict, key: tuple, x: torch.Tensor, need, *args) -> torch.Tensor:
+    """The zero-filled workspace of need(*args) bytes that a module keeps in cache under
+    key.  f16 rows: one per key, so one call at a time.  Rows of other types: one per
+    stream too, the oldest given back beyond a bound (its memory returns to that stream's
+    pool), and under capture one of the graph's own, filled in the graph: their calls
+    overlap on several streams as calls that allocate for themselves do."""
+    if x.dtype == torch.float16:
+        ws = cache.get(key)
+        if ws is not None:
+            return ws
+    elif torch.cuda.is_current_stream_capturing():
+        return torch.zeros(max(need(*args), 4), dtype=torch.uint8, device=x.device)
+    else:
+        cache = cache.setdefault("streams", {})
+        key = (*key, _stream())
+        while len(cache) > _STREAM_WS:
+            cache.pop(next(iter(cache)), None)
+        ws = cache.get(key)
+    if ws is None:
+        ws = cache[key] = torch.zeros(max(need(*args), 4), dtype=torch.uint8, device=x.device)
+    return ws
+
+
 def linear_workspace(m: int, K: int, IC: int, OC: int) -> int:
     return int(_lib.load().esc_linear_workspace(m, K, IC, OC))
 
@@ -248,15 +275,28 @@ def linear(x: torch.Tensor, code_u32: torch.Tensor, rin: torch.Tensor, rout: tor
            rs: float = RS, ws: torch.Tensor | None = None) -> torch.Tensor:
     """The whole coded linear (input transform, GEMV/GEMM, output transform,
     optional f16 bias) -> y f16 [m, OC]; one launch below 16 rows
-    (dense.py:337-362).  From 16 rows x may also be bf16 or f32: transformed
-    from its exact float32 values, y (the f16 result) in x's type.  ws must be
-    zero-filled before its first use (the one-launch path keeps self-resetting
-    counters there)."""
+    (dense.py:337-362).  ws must be zero-filled before its first use (the
+    one-launch path keeps self-resetting counters there)."""
+    if x.dtype != torch.float16:
+        raise ValueError(f"x must be f16 [m, {IC}]")
+    return linear_typed(x, code_u32, rin, rout, K, IC, OC, bias, lut, rs, ws)
+
+
+def _typed(x: torch.Tensor, m: int) -> bool:
+    """Whether the typed linears read rows of x's type: 16-bit, or f32 from 16 rows."""
+    return x.dtype in ROWS_16 or m >= LINEAR_SMALL_ROWS and x.dtype == torch.float32
+
+
+def linear_typed(x: torch.Tensor, code_u32: torch.Tensor, rin: torch.Tensor, rout: torch.Tensor,
+                 K: int, IC: int, OC: int, bias: torch.Tensor | None = None,
+                 lut: bool | None = None, rs: float = RS, ws: torch.Tensor | None = None
+                 ) -> torch.Tensor:
+    """``linear`` for f16, bf16 or (16 rows and more) f32 rows: transformed from
+    their exact float32 values, y (the f16 result) in x's type."""
     _dev(x, code_u32, rin, rout, bias)
     m = x.shape[0]
-    typed = m >= LINEAR_SMALL_ROWS and x.dtype in ROWS_DTYPES
-    if not (typed or x.dtype == torch.float16) or tuple(x.shape) != (m, IC):
-        raise ValueError(f"x must be f16 [m, {IC}]")
+    if (x.dtype not in ROWS_16 and not _typed(x, m)) or tuple(x.shape) != (m, IC):
+        raise ValueError(f"x must be f16, bf16 or f32 (16 rows and more) [m, {IC}]")
     y = torch.empty((m, OC), dtype=x.dtype, device=x.device)
     if m == 0:
         return y
@@ -270,6 +310,25 @@ def linear(x: torch.Tensor, code_u32: torch.Tensor, rin: torch.Tensor, rout: tor
     return y
 
 
+def linear_act(g: torch.Tensor, u: torch.Tensor, code_u32: torch.Tensor, rin: torch.Tensor,
+               rout: torch.Tensor, K: int, IC: int, OC: int, bias: torch.Tensor | None,
+               dtype: torch.dtype, ws: torch.Tensor, rs: float = RS) -> torch.Tensor:
+    """``linear`` of ``moe_shared_act(g, u)`` below 16 rows in one launch: g and u [m, IC]
+    of one 16-bit type (bf16 rounded to f16 first), y [m, OC] of 16-bit `dtype`; ws as
+    ``linear``'s."""
+    _dev(g, u, code_u32, rin, rout, bias)
+    m = g.shape[0]
+    if (g.dtype not in ROWS_16 or u.dtype != g.dtype or dtype not in ROWS_16
+            or tuple(g.shape) != (m, IC) or g.shape != u.shape or m >= LINEAR_SMALL_ROWS):
+        raise ValueError(f"g and u must be [m, {IC}] of one 16-bit type, m < 16")
+    y = torch.empty((m, OC), dtype=dtype, device=g.device)
+    if m:
+        _lib.call("esc_linear_act", _ptr(g), _ptr(u), ROWS_DTYPES[g.dtype], _ptr(rin),
+                  _ptr(_as_u32(code_u32)), _ptr(rout), _ptr(bias), m, K, IC, OC, rs, _ptr(y),
+                  ROWS_DTYPES[dtype], _ptr(ws), ws.numel(), _stream())
+    return y
+
+
 def linear_pair_workspace(m: int, K0: int, K1: int, IC: int, OC0: int, OC1: int) -> int:
     return int(_lib.load().esc_linear_pair_workspace(m, K0, K1, IC, OC0, OC1))
 
@@ -278,14 +337,22 @@ def linear_pair(x: torch.Tensor, p0: tuple, p1: tuple, lut: bool | None = None, 
                 ws: torch.Tensor | None = None):
     """Two coded linears over the same rows in one dispatch (dense.py:365-437):
     p0 / p1 = (code_u32, rin, rout, K, OC, bias or None); returns (y0, y1),
-    each bit-identical to ``linear`` on its own (from 16 rows x may be bf16 or
-    f32, as there).  ws must be zero-filled before its first use."""
+    each bit-identical to ``linear`` on its own.  ws must be zero-filled
+    before its first use."""
+    if x.dtype != torch.float16:
+        raise ValueError("x must be float16")
+    return linear_pair_typed(x, p0, p1, lut, rs, ws)
+
+
+def linear_pair_typed(x: torch.Tensor, p0: tuple, p1: tuple, lut: bool | None = None,
+                      rs: float = RS, ws: torch.Tensor | None = None):
+    """``linear_pair`` for rows of another type, as ``linear_typed``."""
     c0, rin0, rout0, K0, OC0, b0 = p0
     c1, rin1, rout1, K1, OC1, b1 = p1
     _dev(x, c0, rin0, rout0, b0, c1, rin1, rout1, b1)
     m, IC = x.shape
-    if x.dtype != torch.float16 and not (m >= LINEAR_SMALL_ROWS and x.dtype in ROWS_DTYPES):
-        raise ValueError("x must be float16")
+    if not _typed(x, m):
+        raise ValueError("x must be f16, bf16 or (16 rows and more) f32")
     y0 = torch.empty((m, OC0), dtype=x.dtype, device=x.device)
     y1 = torch.empty((m, OC1), dtype=x.dtype, device=x.device)
     if m == 0:
@@ -294,8 +361,8 @@ def linear_pair(x: torch.Tensor, p0: tuple, p1: tuple, lut: bool | None = None, 
         need = linear_pair_workspace(m, K0, K1, IC, OC0, OC1)
         alloc = torch.zeros if m < LINEAR_SMALL_ROWS else torch.empty  # counters below 16 rows
         ws = alloc(max(need, 4), dtype=torch.uint8, device=x.device)
-    _lib.call("esc_linear_pair_typed", _ptr(x), ROWS_DTYPES[x.dtype], m, IC, _ptr(rin0), _ptr(_as_u32(c0)), _ptr(rout0),
-              _ptr(b0), K0, OC0, _ptr(rin1), _ptr(_as_u32(c1)), _ptr(rout1), _ptr(b1), K1, OC1,
+    _lib.call("esc_linear_pair_typed", _ptr(x), ROWS_DTYPES[x.dtype], m, IC, _ptr(rin0),
+              _ptr(_as_u32(c0)), _ptr(rout0), _ptr(b0), K0, OC0, _ptr(rin1), _ptr(_as_u32(c1)), _ptr(rout1), _ptr(b1), K1, OC1,
               _lut_flag(lut), rs, _ptr(y0), _ptr(y1), _ptr(ws), ws.numel(), _stream())
     return y0, y1
 
@@ -351,26 +418,35 @@ def linear_multi(x: torch.Tensor, projs, lut: bool | None = None, rs: float = RS
     tolerance contract of ``linear`` on its own; 2..15 rows: one launch when
     the projections' plans allow, each output bit-identical to ``linear`` on
     its own.  ws must be zero-filled before its first use."""
-    _dev(x, *[t for p in projs for t in (p[0], p[1], p[2], p[5])])
     if x.dtype != torch.float16 or x.dim() != 2:
         raise ValueError("x must be f16 [m, IC]")
+    return linear_multi_typed(x, projs, lut, rs, ws)
+
+
+def linear_multi_typed(x: torch.Tensor, projs, lut: bool | None = None, rs: float = RS,
+                       ws: torch.Tensor | None = None):
+    """``linear_multi`` for rows of another type, as ``linear_typed``."""
+    _dev(x, *[t for p in projs for t in (p[0], p[1], p[2], p[5])])
     m, IC = x.shape
+    if not _typed(x, m):
+        raise ValueError("x must be f16, bf16 or (16 rows and more) f32")
     Ks = {p[3] for p in projs}
     if len(Ks) != 1:
         raise ValueError(f"projections with different K {sorted(Ks)}")
     K = Ks.pop()
     OCs = [int(p[4]) for p in projs]
-    ys = [torch.empty((m, oc), dtype=torch.float16, device=x.device) for oc in OCs]
+    ys = [torch.empty((m, oc), dtype=x.dtype, device=x.device) for oc in OCs]
     if m == 0:
         return ys
     need = linear_multi_workspace(K, IC, OCs, m)
     if ws is None:
         ws = torch.zeros(max(need, 4), dtype=torch.uint8, device=x.device)
     codes = [_as_u32(p[0]) for p in projs]
-    _lib.call("esc_linear_multi", _ptr(x), m, IC, K, len(projs), _ptr_array(codes),
-              _ptr_array([p[1] for p in projs]), _ptr_array([p[2] for p in projs]),
-              _ptr_array([p[5] for p in projs]), (ctypes.c_int * len(OCs))(*OCs), _lut_flag(lut),
-              rs, _ptr_array(ys), _ptr(ws), ws.numel(), _stream())
+    _lib.call("esc_linear_multi_typed", _ptr(x), ROWS_DTYPES[x.dtype], m, IC, K, len(projs),
+              _ptr_array(codes), _ptr_array([p[1] for p in projs]),
+              _ptr_array([p[2] for p in projs]), _ptr_array([p[5] for p in projs]),
+              (ctypes.c_int * len(OCs))(*OCs), _lut_flag(lut), rs, _ptr_array(ys), _ptr(ws),
+              ws.numel(), _stream())
     return ys
 
 

@@ -170,7 +170,7 @@ int esc_linear(const uint16_t* x, const float* rin, const uint32_t* code, const 
 
 /* esc_linear for rows of another element type (ESC_ROWS_*): the rows are
  * transformed from their exact float32 values, y has the rows' element type
- * (the f16 result converted).  bf16 and f32 rows: M >= 16.
+ * (the f16 result converted).  f32 rows: M >= 16.
  * Replaces EschaLinear.__call__ on non-f16 rows (escha_mlx/dense.py:287-292,
  * 337-362). */
 int esc_linear_typed(const void* x, int dtype, const float* rin, const uint32_t* code,
@@ -217,6 +217,15 @@ int esc_linear_xh(const uint16_t* xh, const uint32_t* code, const float* rout,
 int esc_act_transform(const void* g, const void* u, int dtype, const float* rin, int m, int I,
                       float rs, uint16_t* xh, void* stream);
 
+/* esc_linear of the MLP activation of fewer than 16 rows: the rows are h as
+ * esc_act_transform's, computed in the linear's own launch, g and u [M][IC] of 16-bit
+ * element type dtype; y [M][OC] of 16-bit element type y_dtype; ws as esc_linear's.
+ * The down projection of the fused MLP (escha_mlx/models/qwen3_5.py:63-87). */
+int esc_linear_act(const void* g, const void* u, int dtype, const float* rin,
+                   const uint32_t* code, const float* rout, const uint16_t* bias, int M, int K,
+                   int IC, int OC, float rs, void* y, int y_dtype, void* ws, size_t ws_bytes,
+                   void* stream);
+
 /* n (1 to 4) coded linears of the same input rows x f16 [M][IC]:
  * y[i] = esc_linear(x; rin[i], code[i], rout[i], bias[i], K, OC[i]) for the
  * projections of one input (an attention block's q, k and v), all with the
@@ -238,6 +247,13 @@ int esc_linear_multi(const uint16_t* x, int M, int IC, int K, int n, const uint3
                      const float* const* rin, const float* const* rout,
                      const uint16_t* const* bias, const int* OC, int use_lut, float rs,
                      uint16_t* const* y, void* ws, size_t ws_bytes, void* stream);
+
+/* esc_linear_multi for rows of another element type, as esc_linear_typed. */
+int esc_linear_multi_typed(const void* x, int dtype, int M, int IC, int K, int n,
+                           const uint32_t* const* code, const float* const* rin,
+                           const float* const* rout, const uint16_t* const* bias, const int* OC,
+                           int use_lut, float rs, void* const* y, void* ws, size_t ws_bytes,
+                           void* stream);
 
 /* Dense GEMM for a few rows, tolerance contract: y f16 [M][OC] =
  * f16((H128(xh @ decode(code)) * rs) * rout), R rows (2, 4 or 8) per

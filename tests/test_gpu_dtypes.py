@@ -171,3 +171,77 @@ def test_moe_experts_typed_paths(E, H, I, T, k, dtype, monkeypatch):
     x16 = x.half()
     if dtype == torch.bfloat16 or T * k > 64:
         assert torch.equal(blk(x16.to(dtype), ids, sc), blk(x16.to(dtype).half(), ids, sc))
+
+
+def _module(rng, ic, oc, K, bias=True):
+    from escha_mlx_amd.dense import EschaLinear, EschaWeight
+    code, rin, rout, b = _linear_case(rng, ic, oc, K)
+    return EschaLinear(EschaWeight(code, rin, rout, device=DEV), bias=b if bias else None)
+
+
+def _both_types(rng, shape):
+    """bf16 rows that are exact in f16 too."""
+    return torch.from_numpy((rng.integers(-64, 65, shape) / 16).astype(np.float32)).to(DEV).bfloat16()
+
+
+# one row in the split-K kernel (odd column block) and in the persistent kernel
+# (4096 x 16384: 16,384 units), one row group and two, the largest few-row call
+@pytest.mark.parametrize("m,ic,oc,K", [(1, 512, 384, 3), (1, 4096, 16384, 2), (2, 1024, 384, 2),
+                                       (8, 256, 640, 3), (9, 1024, 512, 2), (15, 1024, 512, 3)])
+def test_few_bf16_rows_match_f16_rows(m, ic, oc, K):
+    """bf16 rows below 16 take the f16 rows' kernels: rows exact in both types give the
+    f16 call's result converted, alone, in a pair and of several; from two streams at
+    once and from a replayed graph too."""
+    from escha_mlx_amd.dense import project_many, project_pair
+    rng = np.random.default_rng(500 + m + oc)
+    l0, l1, l2 = (_module(rng, ic, n, K, b) for n, b in ((oc, True), (256, False), (512, True)))
+    x = _both_types(rng, (m, ic))
+    y = l0(x)
+    assert y.dtype == torch.bfloat16 and torch.equal(y, l0(x.half()).bfloat16())
+    for a, b in zip(project_pair(l0, l1, x), project_pair(l0, l1, x.half())):
+        assert torch.equal(a, b.bfloat16())
+    for a, b in zip(project_many([l0, l1, l2], x), project_many([l0, l1, l2], x.half())):
+        assert torch.equal(a, b.bfloat16())
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    outs = [[], []]
+    for _ in range(8):
+        for s, o in zip(streams, outs):
+            with torch.cuda.stream(s):
+                o.append(l0(x))
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, y) for out in outs for o in out)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        yg = l0(x)
+    for _ in range(3):
+        yg.fill_(0)
+        g.replay()
+        assert torch.equal(l0(x), y) and torch.equal(yg, y)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
+@pytest.mark.parametrize("m,ic,inter,oc,K", [(1, 256, 384, 256, 2), (1, 256, 16384, 4096, 3),
+                                             (3, 256, 512, 384, 3), (15, 256, 1024, 256, 2)])
+def test_mlp_few_rows_activation_in_down(m, ic, inter, oc, K, dtype):
+    """EschaMLP below 16 rows computes the activation in down's launch: the bits of the
+    activation and the projection apart, far and infinite gates among them."""
+    from escha_mlx_amd.dense import EschaMLP
+    rng = np.random.default_rng(600 + m + inter)
+    gate, up, down = (_module(rng, a, b, K) for a, b in ((ic, inter), (ic, inter), (inter, oc)))
+    x = _both_types(rng, (m, ic)).to(dtype)
+    apart = down(ops().moe_shared_act(gate(x).half(), up(x).half()))
+    assert torch.equal(EschaMLP(gate, up, down)(x), apart.to(dtype))
+    w = down._w
+    g = torch.randn(m, inter, device=DEV).mul(4).to(dtype)
+    u = torch.randn(m, inter, device=DEV).to(dtype)
+    g[0, :4] = torch.tensor([-1e4, -60000.0, 0.0, 88.0], device=DEV).to(dtype)
+    u[0, :4] = torch.tensor([0.0, 2.0, -3.0, 0.5], device=DEV).to(dtype)
+    for bad in (False, True):
+        if bad:
+            g[0, 5] = float("inf")
+        y = ops().linear_act(g, u, w.code, w.rin, w.rout, K, inter, oc, None, dtype,
+                             down._linear_ws(g))
+        want = ops().linear(ops().moe_shared_act(g.half(), u.half()), w.code, w.rin, w.rout, K,
+                            inter, oc).to(dtype)
+        assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(), want.nan_to_num())
