@@ -136,4 +136,6 @@ def check(rc: int, what: str) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args), name)
+    rc = getattr(_lib or load(), name)(*args)
+    if rc:
+        check(rc, name)

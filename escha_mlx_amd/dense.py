@@ -75,6 +75,15 @@ def dense_block_r(m: int, pin: int | None = None) -> int:
     return max(1, r)
 
 
+def shaped(y: torch.Tensor, shape, dtype: torch.dtype) -> torch.Tensor:
+    """Rows y [m, OC] as [*shape[:-1], OC] of dtype.  A one-row call of a small linear takes
+    longer on the host than on the GPU (2048 x 2048: 10.5 us against 8.4), and a reshape or
+    a cast that changes nothing costs about half a microsecond of it."""
+    if len(shape) != 2:
+        y = y.reshape(*shape[:-1], y.shape[-1])
+    return y if y.dtype == dtype else y.to(dtype)
+
+
 class EschaWeight:
     """One dense linear's coded stream and folded transform vectors (dense.py:158-265)."""
 
@@ -168,17 +177,18 @@ class EschaLinear(torch.nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         w = self._w
         shape = x.shape
+        flat = len(shape) == 2
         # bf16 / f32 rows are transformed from their float32 values
         # (dense.py:287-292); f32 rows below 16 in a launch of its own, then the
         # row-blocked kernels run from xh
-        rows = ops.as_rows(x.reshape(-1, shape[-1]))
+        rows = ops.as_rows(x if flat else x.reshape(-1, shape[-1]))
         m = rows.shape[0]
         if (not self._exact and self._block_r_pin is None and self._fused_had
                 and (self._mat if m >= ops.LINEAR_SMALL_ROWS else rows.dtype in ops.ROWS_16)):
             # the whole linear in esc_linear (one launch below 16 rows)
             y = ops.linear_typed(rows, w.code, w.rin, w.rout, w.K, w.IC, w.OC, bias=self.bias,
                                  lut=self._lut, ws=self._linear_ws(rows))
-            return y.reshape(*shape[:-1], w.OC).to(x.dtype)
+            return shaped(y, shape, x.dtype)
         xh = ops.scaled_had(rows, w.rin, None)
         r = dense_block_r(m, self._block_r_pin)
         if self._mat and r == DENSE_MAT_R and self._fused_had and not self._exact:
@@ -208,7 +218,7 @@ class EschaLinear(torch.nn.Module):
             y = ops.gemv_fast_out(xh, w.code, None, w.rout, w.K, w.IC, w.OC, lut=self._lut)
         if self.bias is not None:
             y = (y.float() + self.bias.float()).to(torch.float16)
-        return y.reshape(*shape[:-1], w.OC).to(x.dtype)
+        return shaped(y, shape, x.dtype)
 
 
 def project_pair(first: EschaLinear, second: EschaLinear, x: torch.Tensor):
@@ -221,7 +231,7 @@ def project_pair(first: EschaLinear, second: EschaLinear, x: torch.Tensor):
     is traded for the saved launch."""
     w0, w1 = first._w, second._w
     shape = x.shape
-    rows = x.reshape(-1, shape[-1]).contiguous()
+    rows = (x if len(shape) == 2 else x.reshape(-1, shape[-1])).contiguous()
     m = rows.shape[0]
     many = m >= ops.LINEAR_SMALL_ROWS
     compatible = (
@@ -242,7 +252,7 @@ def project_pair(first: EschaLinear, second: EschaLinear, x: torch.Tensor):
     y0, y1 = ops.linear_pair_typed(rows, (w0.code, w0.rin, w0.rout, w0.K, w0.OC, first.bias),
                                    (w1.code, w1.rin, w1.rout, w1.K, w1.OC, second.bias),
                                    lut=first._lut, ws=ws)
-    return (y0.reshape(*shape[:-1], w0.OC).to(x.dtype), y1.reshape(*shape[:-1], w1.OC).to(x.dtype))
+    return shaped(y0, shape, x.dtype), shaped(y1, shape, x.dtype)
 
 
 def project_many(linears, x: torch.Tensor):
@@ -258,7 +268,7 @@ def project_many(linears, x: torch.Tensor):
     (escha_mlx/dense.py:365-437)."""
     linears = list(linears)
     shape = x.shape
-    rows = x.reshape(-1, shape[-1]).contiguous()
+    rows = (x if len(shape) == 2 else x.reshape(-1, shape[-1])).contiguous()
     first = linears[0]
     ws_ = [lin._w for lin in linears]
     m = rows.shape[0]
@@ -277,7 +287,7 @@ def project_many(linears, x: torch.Tensor):
                      rows, ops.linear_multi_workspace, ws_[0].K, ws_[0].IC, [w.OC for w in ws_], m)
     ys = ops.linear_multi_typed(rows, [(w.code, w.rin, w.rout, w.K, w.OC, lin.bias)
                                        for w, lin in zip(ws_, linears)], lut=first._lut, ws=ws)
-    return [y.reshape(*shape[:-1], w.OC).to(x.dtype) for y, w in zip(ys, ws_)]
+    return [shaped(y, shape, x.dtype) for y in ys]
 
 
 class EschaMLP(torch.nn.Module):
@@ -298,26 +308,27 @@ class EschaMLP(torch.nn.Module):
         gate, up = project_pair(self.gate_proj, self.up_proj, x)
         down = self.down_proj
         w = down._w
-        m = gate.numel() // gate.shape[-1]
+        flat = len(shape) == 2
+        m = shape[0] if flat else gate.numel() // gate.shape[-1]
         fused = type(down) is EschaLinear and not hooked(down)
         if (fused and 1 <= m < ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_16
                 and x.dtype in ops.ROWS_16 and down.small()):
             # the activation in down's own launch
-            g = gate.reshape(m, w.IC)
-            y = ops.linear_act(g, up.reshape(m, w.IC), w.code, w.rin, w.rout, w.K, w.IC, w.OC,
+            g, u = (gate, up) if flat else (gate.reshape(m, w.IC), up.reshape(m, w.IC))
+            y = ops.linear_act(g, u, w.code, w.rin, w.rout, w.K, w.IC, w.OC,
                                down.bias, x.dtype, down._linear_ws(g))
-            return y.reshape(*shape[:-1], w.OC)
+            return shaped(y, shape, x.dtype)
         if (fused and m >= ops.LINEAR_SMALL_ROWS and gate.dtype in ops.ROWS_DTYPES
                 and down.plain()):
             # the activation and down's input transform in one pass
             xh = ops.act_transform(gate.reshape(m, w.IC), up.reshape(m, w.IC), w.rin)
             dtype = x.dtype if x.dtype in ops.ROWS_DTYPES else torch.float16
             y = ops.linear_xh(xh, w.code, w.rout, w.K, w.IC, w.OC, bias=down.bias, dtype=dtype)
-            return y.reshape(*shape[:-1], w.OC).to(x.dtype)
+            return shaped(y, shape, x.dtype)
         g = gate.reshape(-1, gate.shape[-1]).to(torch.float16).contiguous()
         u = up.reshape(-1, up.shape[-1]).to(torch.float16).contiguous()
         h = ops.moe_shared_act(g, u)
-        return down(h).reshape(*shape[:-1], w.OC).to(x.dtype)
+        return shaped(down(h), shape, x.dtype)
 
 
 class EschaKVProjection(torch.nn.Module):

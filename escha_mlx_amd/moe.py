@@ -172,8 +172,11 @@ class EschaMoEExperts(torch.nn.Module):
         bf16 / f32 rows are transformed from their float32 values
         (models/qwen3_5_moe.py:103-110)."""
         x = ops.as_rows(x)
-        ids = ids.to(torch.int32).contiguous()
-        scores = scores.to(torch.float32).contiguous()
+        if ids.dtype != torch.int32:
+            ids = ids.to(torch.int32)
+        if scores.dtype != torch.float32:
+            scores = scores.to(torch.float32)
+        ids, scores = ids.contiguous(), scores.contiguous()
         if self._exact or not self._fused_had:
             # ESCHA_MLX_FUSED_HAD off: every transform is its own launch around
             # the GEMVs (models/qwen3_5_moe.py:103-122), the staged chain
@@ -231,8 +234,8 @@ class EschaSparseMoeBlock(torch.nn.Module):
         unrounded; the router gate and the shared expert (f16 weights, int8
         w8a16: f16 activations) read the rows rounded to f16."""
         shape = x.shape
-        rows = ops.as_rows(x.reshape(-1, shape[-1]))
-        xf = rows.to(torch.float16).contiguous()
+        rows = ops.as_rows(x if len(shape) == 2 else x.reshape(-1, shape[-1]))
+        xf = rows if rows.dtype == torch.float16 else rows.to(torch.float16)
         ex = self.experts
         if (not ex._exact and ex._fused_had and not ex._one_launch and rows.shape[0]
                 and not dense.hooked(ex, self.sh_gate, self.sh_up, self.sh_down)):
@@ -243,7 +246,9 @@ class EschaSparseMoeBlock(torch.nn.Module):
                                 (self.sh_down.w8, self.sh_down.scale),
                                 (gu.code, gu.rin, gu.rout, gu.K), (dn.code, dn.rin, dn.rout, dn.K),
                                 ex._workspace(rows.shape[0], rows, False), lut=ex._lut)
-            return out.reshape(shape).to(x.dtype)
+            if len(shape) != 2:
+                out = out.reshape(shape)
+            return out if out.dtype == x.dtype else out.to(x.dtype)
         logits = ops.gemv_f16w(xf, self.gate_w).to(torch.float32)
         ids, scores = route(logits, self.top_k)
         y = self.experts(rows, ids, scores)

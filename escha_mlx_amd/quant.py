@@ -39,10 +39,12 @@ class EschaQ8Linear(torch.nn.Module):
         self.out_features, self.in_features = self.w8.shape
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        lead = x.shape[:-1]
-        xf = x.reshape(-1, self.in_features).to(torch.float16).contiguous()
+        flat = x.dim() == 2 and x.shape[1] == self.in_features
+        xf = (x if flat else x.reshape(-1, self.in_features)).to(torch.float16).contiguous()
         y = ops.w8a16(xf, self.w8, self.scale)
-        return y.reshape(*lead, self.out_features).to(x.dtype)
+        if not flat:
+            y = y.reshape(*x.shape[:-1], self.out_features)
+        return y if x.dtype == torch.float16 else y.to(x.dtype)
 
 
 class EschaQ8Head(EschaQ8Linear):
