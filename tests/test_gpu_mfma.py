@@ -202,7 +202,7 @@ def test_linear_split_steps(K, ic, oc, m, dtype):
     bias = (rng.standard_normal(oc) * 0.05).astype(np.float16)
     x = torch.from_numpy(rng.standard_normal((m, ic)).astype(np.float32)).to(dtype).to(DEV)
     rin_d, rout_d, bias_d = (torch.from_numpy(a).to(DEV) for a in (rin, rout, bias))
-    y = ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d)
+    y = ops().linear_typed(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d)
     assert y.dtype == dtype
     xh = R.input_transform(x.float().cpu().numpy(), rin)
     exact = R.h128(xh.astype(np.float64) @ R.reconstruct(u32, ic, oc, K).astype(np.float64)) \
@@ -210,12 +210,12 @@ def test_linear_split_steps(K, ic, oc, m, dtype):
     got = y.float().cpu().numpy().astype(np.float64)
     err = (np.abs(got - exact).max(axis=1) / np.abs(exact).max(axis=1)).max()
     assert err < 2e-3 + (2.0 ** -9 if dtype == torch.bfloat16 else 0.0), err
-    assert torch.equal(ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d), y)
+    assert torch.equal(ops().linear_typed(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d), y)
     al = lambda v: (v + 255) // 256 * 256
     small = al(2 * m * ic) + al(4 * m * oc)
     assert ops().linear_workspace(m, K, ic, oc) > small
     ws = torch.empty(small, dtype=torch.uint8, device=DEV)
-    one = ops().linear(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d, ws=ws)
+    one = ops().linear_typed(x, code, rin_d, rout_d, K, ic, oc, bias=bias_d, ws=ws)
     want = ops().gemm_mfma_out(ops().scaled_had(x, rin_d, None), code, rout_d, K, ic, oc, bias=bias_d)
     assert torch.equal(one, want.to(dtype))
 
@@ -235,9 +235,9 @@ def test_pair_many_rows_bit_identical(K, ic, ocs, m, dtype):
         rin = torch.from_numpy(rng.choice([-1.0, 1.0], ic).astype(np.float32)).to(DEV)
         bias = torch.from_numpy((rng.standard_normal(oc) * 0.05).astype(np.float16)).to(DEV)
         ps.append((code, rin, torch.from_numpy(_rout(rng, oc)).to(DEV), K, oc, bias))
-    got = ops().linear_pair(x, ps[0], ps[1])
+    got = ops().linear_pair_typed(x, ps[0], ps[1])
     for y, (code, rin, rout, _, oc, bias) in zip(got, ps):
-        assert torch.equal(y, ops().linear(x, code, rin, rout, K, ic, oc, bias=bias))
+        assert torch.equal(y, ops().linear_typed(x, code, rin, rout, K, ic, oc, bias=bias))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
