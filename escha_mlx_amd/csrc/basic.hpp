@@ -86,10 +86,45 @@ __device__ __forceinline__ void h128_wave(float& v0, float& v1) {
              lane & 32);
 }
 
-// Transform kernels: one wave per (row, 128-block); a 256-thread workgroup
-// covers kTransformRows rows of one 128-block (kTransformRows / 4 per wave,
-// their loads issued together).  grid (dim/128, ceil(m / kTransformRows)).
-constexpr int kTransformRows = 16;
+// The same transform with 8 lanes per 128-block, a wave working on 8 blocks at
+// once: v[8b + j] is element 64b + 8 oct_chunk() + j, so element bits 0..2 and 6 are
+// additions between registers and bits 3..5 one DPP move and one addition each
+// (lane ^ 1, ^ 2 and ^ 7 = quad permutes and the half-row mirror; oct_chunk() is the
+// lane numbering in which these flip one bit each).  The stages run in h128_wave's
+// order on the same operands (a - b of the upper lane as fma(v, -1, other), exact):
+// bit-identical to it.  29 VALU instructions per block with its conversions against
+// 60, and 16- and 32-byte accesses per lane.
+__device__ __forceinline__ int oct_chunk() {
+  const int l = threadIdx.x & 7;
+  return l < 4 ? l : l ^ 3;
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+  const int x = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(x, x, CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ void h128_oct(float (&v)[16]) {
+  auto pair = [&](int a, int b) {
+    const float x = v[a], y = v[b];
+    v[a] = x + y;
+    v[b] = x - y;
+  };
+#pragma unroll
+  for (int s = 1; s < 8; s *= 2)
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      if (!(j & s)) pair(j, j | s);
+  const int ch = oct_chunk();
+  const float s3 = ch & 1 ? -1.f : 1.f, s4 = ch & 2 ? -1.f : 1.f, s5 = ch & 4 ? -1.f : 1.f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) v[j] = __builtin_fmaf(v[j], s3, dpp_move<0xB1>(v[j]));   // ^ 1
+#pragma unroll
+  for (int j = 0; j < 16; ++j) v[j] = __builtin_fmaf(v[j], s4, dpp_move<0x4E>(v[j]));   // ^ 2
+#pragma unroll
+  for (int j = 0; j < 16; ++j) v[j] = __builtin_fmaf(v[j], s5, dpp_move<0x141>(v[j]));  // ^ 7
+#pragma unroll
+  for (int j = 0; j < 8; ++j) pair(j, j + 8);
+}
 
 // Element types of the rows an input transform reads (esc_input_transform_typed).
 enum { kRowsF16 = 0, kRowsBF16 = 1, kRowsF32 = 2 };
@@ -117,6 +152,68 @@ __device__ __forceinline__ float2 row_pair(const void* rows, size_t i) {
   }
 }
 
+// 16 bytes at any element alignment (a caller's rows may start at any element).
+struct __attribute__((packed, aligned(2))) Bytes16 {
+  uint32_t w[4];
+};
+// Elements i .. i + 7 and i + 64 .. i + 71 of a row as float32 (exact for every type).
+template <int DT>
+__device__ __forceinline__ void load_oct(const void* rows, size_t i, float (&v)[16]) {
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    if constexpr (DT == kRowsF32) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const Bytes16 q = *reinterpret_cast<const Bytes16*>(static_cast<const float*>(rows) + i +
+                                                            64 * b + 4 * h);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[8 * b + 4 * h + j] = __builtin_bit_cast(float, q.w[j]);
+      }
+    } else {
+      const Bytes16 q =
+          *reinterpret_cast<const Bytes16*>(static_cast<const uint16_t*>(rows) + i + 64 * b);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t w = q.w[j];
+        v[8 * b + 2 * j] = DT == kRowsBF16 ? __builtin_bit_cast(float, w << 16)
+                                           : (float)__builtin_bit_cast(half_t, (uint16_t)w);
+        v[8 * b + 2 * j + 1] = DT == kRowsBF16
+                                   ? __builtin_bit_cast(float, w & 0xFFFF0000u)
+                                   : (float)__builtin_bit_cast(half_t, (uint16_t)(w >> 16));
+      }
+    }
+  }
+}
+// f16(v * rs) to elements i .. i + 7 and i + 64 .. i + 71 of out.
+__device__ __forceinline__ void store_oct(uint16_t* out, size_t i, const float (&v)[16], float rs) {
+#pragma unroll
+  for (int b = 0; b < 2; ++b) {
+    Bytes16 q;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+      q.w[j] = (uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[8 * b + 2 * j] * rs)) |
+               ((uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[8 * b + 2 * j + 1] * rs)) << 16);
+    *reinterpret_cast<Bytes16*>(out + i + 64 * b) = q;
+  }
+}
+// The place of this lane's group of 8 in a grid over (ROWS rows, 128-block), the blocks
+// fastest (a wave reads 2 KB runs of a row): first row and element column.  Groups past
+// the end repeat the last one's reads (row0 = m: nothing is stored).
+struct OctPlace {
+  int row0, col;
+};
+template <int ROWS>
+__device__ __forceinline__ OctPlace oct_place(int m, int nblk) {
+  const unsigned item = (blockIdx.x * blockDim.x + threadIdx.x) >> 3;
+  const unsigned rp = item / (unsigned)nblk, blk = item - rp * (unsigned)nblk;
+  return {min(ROWS * (int)rp, m), 128 * (int)blk + 8 * oct_chunk()};
+}
+
+// Output transform: one wave per (row, 128-block); a 256-thread workgroup
+// covers kTransformRows rows of one 128-block (kTransformRows / 4 per wave,
+// their loads issued together).  grid (dim/128, ceil(m / kTransformRows)).
+constexpr int kTransformRows = 16;
+
 // xh = f16(H128(f32(rows) * rin) * RS); rin is [E][IC] gathered by row_expert,
 // or [IC] when row_expert is null (escha_mlx/msl.py:875-916, 1029-1047).
 // DT: the rows' element type; f16 rows are the fused kernel's input, bf16 and
@@ -124,7 +221,9 @@ __device__ __forceinline__ float2 row_pair(const void* rows, size_t i) {
 // models/qwen3_5_moe.py:108-110), converted exactly to float32 here with no
 // f16 rounding before the transform.
 // TWO: the rows are read once for two projections (rin / out and rin1 / out1).
-template <int DT, bool TWO = false>
+// HBM-bound from some hundred rows on, latency-bound below.  2048 x 5120 f16 rows for
+// two projections 23 -> 16.6 us by 8 lanes per block against one wave.  grid: oct_place.
+template <int DT, int ROWS, bool TWO = false>
 __global__ __launch_bounds__(256) void k_input_transform(const void* __restrict__ rows,
                                                          const float* __restrict__ rin,
                                                          const int* __restrict__ row_expert,
@@ -132,39 +231,32 @@ __global__ __launch_bounds__(256) void k_input_transform(const void* __restrict_
                                                          uint16_t* __restrict__ out,
                                                          const float* __restrict__ rin1 = nullptr,
                                                          uint16_t* __restrict__ out1 = nullptr) {
-  constexpr int RPW = kTransformRows / 4;
-  const int blk = blockIdx.x, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c = blk * 128 + 2 * lane;
-  const int row0 = blockIdx.y * kTransformRows + RPW * wave;
-  float2 xv[RPW];
-  float v[RPW][2];
+  const OctPlace at = oct_place<ROWS>(m, IC / 128);
+  float xv[ROWS][16], r[16];
 #pragma unroll
-  for (int j = 0; j < RPW; ++j) {
-    const int row = min(row0 + j, m - 1);
-    xv[j] = row_pair<DT>(rows, (size_t)row * IC + c);
-    const float* r = rin + (row_expert ? (size_t)row_expert[row] * IC : 0) + c;
-    v[j][0] = xv[j].x * r[0];
-    v[j][1] = xv[j].y * r[1];
+  for (int j = 0; j < ROWS; ++j)
+    load_oct<DT>(rows, (size_t)min(at.row0 + j, m - 1) * IC + at.col, xv[j]);
+  if (!row_expert) load_oct<kRowsF32>(rin, at.col, r);
+#pragma unroll
+  for (int j = 0; j < ROWS; ++j) {
+    const int row = at.row0 + j;
+    if (row_expert) load_oct<kRowsF32>(rin, (size_t)row_expert[min(row, m - 1)] * IC + at.col, r);
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = xv[j][i] * r[i];
+    h128_oct(v);
+    if (row < m) store_oct(out, (size_t)row * IC + at.col, v, rs);
   }
-  auto finish = [&](uint16_t* o) {
-#pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-      h128_wave(v[j][0], v[j][1]);
-      if (row0 + j < m)
-        *reinterpret_cast<uint32_t*>(o + (size_t)(row0 + j) * IC + c) =
-            (uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[j][0] * rs)) |
-            ((uint32_t)__builtin_bit_cast(uint16_t, to_f16(v[j][1] * rs)) << 16);
-    }
-  };
-  finish(out);
   if constexpr (TWO) {
-    const float r0 = rin1[c], r1 = rin1[c + 1];
+    load_oct<kRowsF32>(rin1, at.col, r);
 #pragma unroll
-    for (int j = 0; j < RPW; ++j) {
-      v[j][0] = xv[j].x * r0;
-      v[j][1] = xv[j].y * r1;
+    for (int j = 0; j < ROWS; ++j) {
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = xv[j][i] * r[i];
+      h128_oct(v);
+      if (at.row0 + j < m) store_oct(out1, (size_t)(at.row0 + j) * IC + at.col, v, rs);
     }
-    finish(out1);
   }
 }
 

@@ -272,6 +272,19 @@ int device_cus() {
   return cus[dev];
 }
 
+// The launch of a transform by 8 lanes per 128-block: f(rows per lane group as a
+// constant, grid, block).  Two rows per group (the scales read once) in workgroups of
+// 256 once those fill eight waves per CU; below that one row, in single waves, for more
+// of them in flight.
+template <typename F>
+void oct_launch(int m, int dim, F f) {
+  const long two = (long)(dim / 128) * ((m + 1) / 2);
+  if (two >= 64L * device_cus())
+    f(std::integral_constant<int, 2>{}, dim3((unsigned)((two + 31) / 32)), dim3(256));
+  else
+    f(std::integral_constant<int, 1>{}, dim3((unsigned)(((long)(dim / 128) * m + 7) / 8)), dim3(64));
+}
+
 // Row blocks of 16 per k_gemm_mma2 workgroup (NRB in {2,4,6,8}) and splits S of
 // the K steps (4 kt each).  A step of one workgroup takes about 0.66 + 0.055 NRB
 // us of its CU (K = 3; decode, then MFMAs), a lone workgroup on a CU 1.24 times
@@ -662,17 +675,12 @@ int esc_input_transform_typed(const void* rows, int dtype, const float* rin,
               "row element type must be ESC_ROWS_F16, ESC_ROWS_BF16 or ESC_ROWS_F32, got %d",
               dtype);
   if (m == 0) return ESC_OK;
-  const int ry = (m + esc::kTransformRows - 1) / esc::kTransformRows;
-  const dim3 grid(IC / 128, ry), blk(256);
-  if (dtype == ESC_ROWS_F16)
-    hipLaunchKernelGGL(esc::k_input_transform<esc::kRowsF16>, grid, blk, 0, S(stream), rows, rin,
-                       row_expert, m, IC, rs, out);
-  else if (dtype == ESC_ROWS_BF16)
-    hipLaunchKernelGGL(esc::k_input_transform<esc::kRowsBF16>, grid, blk, 0, S(stream), rows,
-                       rin, row_expert, m, IC, rs, out);
-  else
-    hipLaunchKernelGGL(esc::k_input_transform<esc::kRowsF32>, grid, blk, 0, S(stream), rows, rin,
-                       row_expert, m, IC, rs, out);
+  by_rows_type(dtype, [&](auto dt) {
+    oct_launch(m, IC, [&](auto r, dim3 grid, dim3 blk) {
+      hipLaunchKernelGGL((esc::k_input_transform<decltype(dt)::value, decltype(r)::value>), grid,
+                         blk, 0, S(stream), rows, rin, row_expert, m, IC, rs, out);
+    });
+  });
   return launched("k_input_transform");
 }
 
@@ -820,10 +828,11 @@ int esc_act_transform(const void* g, const void* u, int dtype, const float* rin,
               "row element type must be ESC_ROWS_F16, ESC_ROWS_BF16 or ESC_ROWS_F32, got %d",
               dtype);
   if (m == 0) return ESC_OK;
-  const dim3 grid(I / 128, (m + esc::kTransformRows - 1) / esc::kTransformRows);
   by_rows_type(dtype, [&](auto dt) {
-    hipLaunchKernelGGL(esc::k_act_transform<decltype(dt)::value>, grid, dim3(256), 0, S(stream), g,
-                       u, rin, m, I, rs, xh);
+    oct_launch(m, I, [&](auto r, dim3 grid, dim3 blk) {
+      hipLaunchKernelGGL((esc::k_act_transform<decltype(dt)::value, decltype(r)::value>), grid, blk,
+                         0, S(stream), g, u, rin, m, I, rs, xh);
+    });
   });
   return launched("k_act_transform");
 }
@@ -902,10 +911,11 @@ int esc_linear_pair_typed(const void* x, int dtype, int M, int IC, const float* 
     char* w1 = w + off1;
     uint16_t* xh0 = reinterpret_cast<uint16_t*>(w + p0.off_xh);
     uint16_t* xh1 = reinterpret_cast<uint16_t*>(w1 + p1.off_xh);
-    const dim3 tg(IC / 128, (M + esc::kTransformRows - 1) / esc::kTransformRows);
     by_rows_type(dtype, [&](auto dt) {
-      hipLaunchKernelGGL((esc::k_input_transform<decltype(dt)::value, true>), tg, dim3(256), 0, s,
-                         x, rin0, nullptr, M, IC, rs, xh0, rin1, xh1);
+      oct_launch(M, IC, [&](auto r, dim3 grid, dim3 blk) {
+        hipLaunchKernelGGL((esc::k_input_transform<decltype(dt)::value, decltype(r)::value, true>),
+                           grid, blk, 0, s, x, rin0, nullptr, M, IC, rs, xh0, rin1, xh1);
+      });
     });
     if (int rc = launched("k_input_transform")) return rc;
     const esc::MmaArgs a0{xh0, code0, M, TK, OC0 / 16, reinterpret_cast<float*>(w + p0.off_mid),
@@ -1605,18 +1615,19 @@ int moe_mma(int K, int nrb, const esc::MoeMmaArgs& a, hipStream_t s) {
 int moe_prep(const void* x, int dtype, const int32_t* ids, int T, int top_k, const float* rin,
              int H, float rs, uint16_t* xh, const MoePlan& p, int E, int* rows, int* gexp,
              int* nact, hipStream_t s) {
-  // four slots per wave once that leaves eight waves per SIMD
-  const bool four = (long)T * top_k * (H / 128) / 4 >= 32L * device_cus();
-  const long waves = (long)(H / 128) * T * (four ? (top_k + 3) / 4 : top_k);
+  // 8 lanes per block once that leaves eight waves per CU
+  const long rows8 = (long)(H / 128) * T * ((top_k + esc::kOctSlots - 1) / esc::kOctSlots);
+  const bool oct = rows8 >= 64L * device_cus();
+  const long waves = oct ? (rows8 + 7) / 8 : (long)(H / 128) * p.M;
   const dim3 grid((unsigned)(1 + (waves + 15) / 16)), blk(1024);
   by_rows_type(dtype, [&](auto dt) {
     constexpr int DT = decltype(dt)::value;
-    if (four)
-      hipLaunchKernelGGL((esc::k_moe_prep<4, DT>), grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh,
-                         p.M, E, p.R, p.n_groups, rows, gexp, nact);
+    if (oct)
+      hipLaunchKernelGGL((esc::k_moe_prep<true, DT>), grid, blk, 0, s, x, ids, top_k, rin, H, rs,
+                         xh, p.M, E, p.R, p.n_groups, rows, gexp, nact);
     else
-      hipLaunchKernelGGL((esc::k_moe_prep<1, DT>), grid, blk, 0, s, x, ids, top_k, rin, H, rs, xh,
-                         p.M, E, p.R, p.n_groups, rows, gexp, nact);
+      hipLaunchKernelGGL((esc::k_moe_prep<false, DT>), grid, blk, 0, s, x, ids, top_k, rin, H, rs,
+                         xh, p.M, E, p.R, p.n_groups, rows, gexp, nact);
   });
   return launched("k_moe_prep");
 }

@@ -9,30 +9,49 @@
 namespace esc {
 
 // xh[row] = f16(H128(f32(x[tok]) * rin[ids[row]]) * RS) (DT: x's element type,
-// converted exactly to float32), 128-block blk of the
-// rows row = tok * top_k + s of up to NS slots s from s0 of one token, by one
-// wave: the token's inputs are read once, every slot's scales are requested
-// before any is used (slots past the last re-read it and store nothing).
-template <int NS, int DT>
+// converted exactly to float32), 128-block blk of routed row row = tok * top_k + s,
+// by one wave.
+template <int DT>
 __device__ __forceinline__ void moe_input_wave(const void* __restrict__ x,
                                                const int* __restrict__ ids, int top_k,
                                                const float* __restrict__ rin, int H, float rs,
-                                               uint16_t* __restrict__ xh, int blk, int tok,
-                                               int s0) {
-  const int lane = threadIdx.x & 63;
-  const int c = blk * 128 + 2 * lane, row0 = tok * top_k + s0, n = top_k - s0;
-  const float2 xv = row_pair<DT>(x, (size_t)tok * H + c);
-  float2 r[NS];
+                                               uint16_t* __restrict__ xh, int blk, int row) {
+  const int c = blk * 128 + 2 * (threadIdx.x & 63);
+  const float2 xv = row_pair<DT>(x, (size_t)(row / top_k) * H + c);
+  const float2 r = ld_global_f2(rin + (size_t)ids[row] * H + c);
+  float v0 = xv.x * r.x, v1 = xv.y * r.y;
+  h128_wave(v0, v1);
+  *reinterpret_cast<uint32_t*>(xh + (size_t)row * H + c) =
+      pack2(to_f16(v0 * rs), to_f16(v1 * rs));
+}
+
+// The same for item's (token, kOctSlots slots, 128-block), the blocks fastest, by 8
+// lanes (h128_oct): the token's inputs are read once, every slot's scales are
+// requested before any is used (slots past the last, and items past n, re-read the
+// last and store nothing).
+constexpr int kOctSlots = 4;
+template <int DT>
+__device__ __forceinline__ void moe_input_oct(const void* __restrict__ x,
+                                              const int* __restrict__ ids, int top_k,
+                                              const float* __restrict__ rin, int H, float rs,
+                                              uint16_t* __restrict__ xh, unsigned item,
+                                              unsigned n) {
+  const unsigned nhb = H / 128, ns = (top_k + kOctSlots - 1) / kOctSlots;
+  const unsigned it = min(item, n - 1), p = it / nhb, tok = p / ns;
+  const int s0 = (int)(p - tok * ns) * kOctSlots, left = item < n ? top_k - s0 : 0;
+  const size_t row0 = (size_t)tok * top_k + s0;
+  const int c = 128 * (int)(it - p * nhb) + 8 * oct_chunk();
+  float xv[16], r[kOctSlots][16];
+  load_oct<DT>(x, (size_t)tok * H + c, xv);
 #pragma unroll
-  for (int j = 0; j < NS; ++j)
-    r[j] = ld_global_f2(rin + (size_t)ids[row0 + min(j, n - 1)] * H + c);
+  for (int j = 0; j < kOctSlots; ++j)
+    load_oct<kRowsF32>(rin, (size_t)ids[row0 + min(j, top_k - s0 - 1)] * H + c, r[j]);
 #pragma unroll
-  for (int j = 0; j < NS; ++j) {
-    float v0 = xv.x * r[j].x, v1 = xv.y * r[j].y;
-    h128_wave(v0, v1);
-    if (j < n)
-      *reinterpret_cast<uint32_t*>(xh + (size_t)(row0 + j) * H + c) =
-          pack2(to_f16(v0 * rs), to_f16(v1 * rs));
+  for (int j = 0; j < kOctSlots; ++j) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) r[j][i] *= xv[i];
+    h128_oct(r[j]);
+    if (j < left) store_oct(xh, (row0 + j) * H + c, r[j], rs);
   }
 }
 
@@ -42,17 +61,17 @@ __global__ __launch_bounds__(64) void k_moe_input(const void* __restrict__ x,
                                                   const int* __restrict__ ids, int top_k,
                                                   const float* __restrict__ rin, int H, float rs,
                                                   uint16_t* __restrict__ xh) {
-  const int row = blockIdx.y, tok = row / top_k;
-  moe_input_wave<1, DT>(x, ids, top_k, rin, H, rs, xh, blockIdx.x, tok, row - tok * top_k);
+  moe_input_wave<DT>(x, ids, top_k, rin, H, rs, xh, blockIdx.x, blockIdx.y);
 }
 
 // The chain's two independent first steps in one launch: block 0 groups the
-// routed rows by expert (build_groups_block); every other block runs 16 of
-// the input transforms of (128-block, token, NS slots), one per wave.  NS = 4
-// (a token's inputs and ids read once per four slots, 4-byte accesses) where
-// the rows fill the GPU all the same; NS = 1 below that.  grid
-// 1 + ceil(H/128 * T * ceil(top_k/NS) / 16), block 1024.
-template <int NS, int DT>
+// routed rows by expert (build_groups_block); every other block runs input
+// transforms, one (128-block, row) per wave, or (OCT) 8 per wave and two slots of a
+// token each.  The grouping's registers and LDS leave one workgroup of 16 waves per
+// CU, so a wave's few loads are what is in flight: by 8 lanes per block 2048 tokens'
+// rows of top-8, hidden 2048 take 51 -> 36 us.  grid 1 + the transforms' blocks,
+// block 1024.
+template <bool OCT, int DT>
 __global__ __launch_bounds__(1024) void k_moe_prep(const void* __restrict__ x,
                                                    const int* __restrict__ ids, int top_k,
                                                    const float* __restrict__ rin, int H, float rs,
@@ -64,11 +83,16 @@ __global__ __launch_bounds__(1024) void k_moe_prep(const void* __restrict__ x,
     build_groups_block(ids, m, E, R, n_groups, rows_idx, group_expert, n_active);
     return;
   }
-  const int nhb = H / 128, ns = (top_k + NS - 1) / NS;
-  const int w = __builtin_amdgcn_readfirstlane((blockIdx.x - 1) * 16 + (threadIdx.x >> 6));
-  const int p = w / nhb, tok = p / ns;  // (token, slots), blk fastest
-  if (tok < m / top_k)
-    moe_input_wave<NS, DT>(x, ids, top_k, rin, H, rs, xh, w % nhb, tok, (p - tok * ns) * NS);
+  const int nhb = H / 128;
+  if constexpr (OCT) {
+    const unsigned n = (unsigned)nhb * (m / top_k) * ((top_k + kOctSlots - 1) / kOctSlots);
+    moe_input_oct<DT>(x, ids, top_k, rin, H, rs, xh,
+                      ((blockIdx.x - 1) * 1024u + threadIdx.x) >> 3, n);
+  } else {
+    const int w = __builtin_amdgcn_readfirstlane((blockIdx.x - 1) * 16 + (threadIdx.x >> 6));
+    const int row = w / nhb;
+    if (row < m) moe_input_wave<DT>(x, ids, top_k, rin, H, rs, xh, w - row * nhb, row);
+  }
 }
 
 // The grouped split-K GEMM of k_gemv_fast_rows with the table decode, as a

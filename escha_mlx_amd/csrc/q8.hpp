@@ -527,26 +527,23 @@ __global__ __launch_bounds__(256) void k_shared_act(const uint16_t* __restrict__
 // The activation and the down projection's input transform in one pass (the MLP
 // of many rows): xh = f16(H128(f32(h) * rin) * rs), h = f16((g / (1 + exp(-g))) * u)
 // as k_shared_act, g and u [m][I] read as f16 (bf16 rows rounded to f16 first, as
-// the module's cast does; f32 rows hold f16 values).  One wave per 128-block of
-// kTransformRows / 4 rows, as k_input_transform: HBM-bound, and h is never
-// written.  grid (I/128, ceil(m / kTransformRows)), block 256.
-template <int DT>
+// the module's cast does; f32 rows hold f16 values).  HBM-bound, and h is never
+// written: 2048 x 17408 62 -> 55 us by 8 lanes per block (h128_oct) against one wave.
+// grid: oct_place.
+template <int DT, int ROWS>
 __global__ __launch_bounds__(256) void k_act_transform(const void* __restrict__ g,
                                                        const void* __restrict__ u,
                                                        const float* __restrict__ rin, int m, int I,
                                                        float rs, uint16_t* __restrict__ xh) {
-  constexpr int RPW = kTransformRows / 4;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int c = blockIdx.x * 128 + 2 * lane;
-  const int row0 = blockIdx.y * kTransformRows + RPW * wave;
-  const float r0 = rin[c], r1 = rin[c + 1];
-  float2 gv[RPW], uv[RPW];
+  const OctPlace at = oct_place<ROWS>(m, I / 128);
+  float gv[ROWS][16], uv[ROWS][16], r[16];
 #pragma unroll
-  for (int j = 0; j < RPW; ++j) {
-    const size_t i = (size_t)min(row0 + j, m - 1) * I + c;
-    gv[j] = row_pair<DT>(g, i);
-    uv[j] = row_pair<DT>(u, i);
+  for (int j = 0; j < ROWS; ++j) {
+    const size_t i = (size_t)min(at.row0 + j, m - 1) * I + at.col;
+    load_oct<DT>(g, i, gv[j]);
+    load_oct<DT>(u, i, uv[j]);
   }
+  load_oct<kRowsF32>(rin, at.col, r);
   auto act = [](float gf, float uf) {
     if constexpr (DT != kRowsF16) {
       gf = (float)(half_t)gf;
@@ -555,12 +552,12 @@ __global__ __launch_bounds__(256) void k_act_transform(const void* __restrict__ 
     return (float)to_f16((gf / (1.0f + expf(-gf))) * uf);
   };
 #pragma unroll
-  for (int j = 0; j < RPW; ++j) {
-    float v0 = act(gv[j].x, uv[j].x) * r0, v1 = act(gv[j].y, uv[j].y) * r1;
-    h128_wave(v0, v1);
-    if (row0 + j < m)
-      *reinterpret_cast<uint32_t*>(xh + (size_t)(row0 + j) * I + c) =
-          pack2(to_f16(v0 * rs), to_f16(v1 * rs));
+  for (int j = 0; j < ROWS; ++j) {
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = act(gv[j][i], uv[j][i]) * r[i];
+    h128_oct(v);
+    if (at.row0 + j < m) store_oct(xh, (size_t)(at.row0 + j) * I + at.col, v, rs);
   }
 }
 

@@ -245,3 +245,23 @@ def test_mlp_few_rows_activation_in_down(m, ic, inter, oc, K, dtype):
         want = ops().linear(ops().moe_shared_act(g.half(), u.half()), w.code, w.rin, w.rout, K,
                             inter, oc).to(dtype)
         assert torch.equal(y.isnan(), want.isnan()) and torch.equal(y.nan_to_num(), want.nan_to_num())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["f16", "bf16", "f32"])
+@pytest.mark.parametrize("m,IC", [(1, 128), (3, 1152), (70, 384)])
+def test_input_transform_any_start(dtype, m, IC):
+    """Rows and scales that start at any element (16-byte loads of 8 lanes per
+    128-block): the oracle's bits, per-row scales too."""
+    rng = np.random.default_rng(m + IC)
+    x = torch.from_numpy(rng.standard_normal((m, IC)).astype(np.float32)).to(DEV).to(dtype)
+    v = x.float().cpu().numpy()
+    rin = rng.uniform(-1.5, 1.5, (3, IC)).astype(np.float32)
+    re = rng.integers(0, 3, m).astype(np.int32)
+    xs = torch.empty(m * IC + 5, dtype=dtype, device=DEV)[5:].view(m, IC).copy_(x)
+    rs = torch.empty(3 * IC + 3, dtype=torch.float32, device=DEV)[3:].view(3, IC)
+    rs.copy_(torch.from_numpy(rin))
+    got = ops().scaled_had(xs, rs[1], None)
+    assert np.array_equal(bits16(got), R.input_transform(v, rin[1]).view(np.uint16))
+    got = ops().scaled_had(xs, rs, torch.from_numpy(re).to(DEV))
+    assert np.array_equal(bits16(got), R.input_transform(v, rin[re]).view(np.uint16))

@@ -86,3 +86,21 @@ def test_route_topk_edges(T, E, k):
         ids, _ = ops().route_topk(torch.from_numpy(nan).to(DEV), k)
         want, _ = R.route_topk(np.where(np.isnan(nan), -np.inf, nan), k)
         assert np.array_equal(ids.cpu().numpy(), want)
+
+
+# 16,440 transforms of 8 lanes: past the size where a wave takes 8 of them; three
+# 128-blocks per row, an odd top_k (the last slot of each token alone)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32],
+                         ids=["f16", "bf16", "f32"])
+def test_many_tokens_match_fewer(dtype):
+    """A token's result does not depend on the tokens beside it: one call of 2740
+    tokens has the bits of calls of 548, whose input transforms run one block a wave."""
+    E, T, k, H, I, K_gu, K_dn = 4, 2740, 3, 384, 128, 2, 3
+    c = _moe_case(E, H, I, K_gu, K_dn, T, k, 77)
+    ids, sc = ops().route_topk(torch.from_numpy(c["logits"]).to(DEV), k)
+    x = torch.from_numpy(c["x"]).to(DEV).to(dtype)
+    args = _args(c, K_gu, K_dn)
+    y = ops().moe_expert_path(x, ids, sc, *args)
+    parts = [ops().moe_expert_path(*(t[i:i + 548].contiguous() for t in (x, ids, sc)), *args)
+             for i in range(0, T, 548)]
+    assert torch.equal(y, torch.cat(parts))
