@@ -1465,17 +1465,22 @@ int moe_input(const void* x, int dtype, const int32_t* ids, int top_k, const flo
 // Row blocks of 16 per group of the grouped matrix-core GEMM (k_moe_mma), 0:
 // the split-K chain.  Measured on MI355X (256 experts, hidden 2048, intermediate
 // 512, top-8; whole call, the split-K chain in brackets): 6 rows per expert 175 us
-// (150), 9 rows 175 (164), 12 rows 180 (187), 16 rows 183 (218), 64 rows 306 (1200
+// (150), 9 rows 175 (164), 12 rows 173 (187), 16 rows 171 (218), 64 rows 284 (1200
 // in groups of 8); 64 experts, 8 rows 78 (80 by hash), 12 rows 79 (99), 4 rows 78
 // (66).  So from 8 rows per expert, or 11 where the experts' weights fill the chip
-// (the split-K chain then decodes with the table), at the row-block size with the
-// least work: a group costs 0.43 + 0.071 NRB (208, 263, 292 and 337 us with one
-// group of 2, 4, 6 and 8 row blocks per expert), and an expert with Poisson(M / E)
-// rows takes sum over j of P(rows > 16 NRB j) groups.
+// (the split-K chain then decodes with the table).  The row-block size is that of the
+// least cost: a group multiplies only the row blocks that hold rows, the same ones at
+// every size, so a size is paid for in waves per SIMD (its accumulators) and in groups
+// (each decodes its expert anew): 2, 4, 6 and 8 row blocks measure 171, 174, 193 and
+// 197 us at 16 rows per expert, 248, 227, 223 and 232 at 32, 318, 251, 243 and 257 at
+// 47, 387, 324, 284 and 304 at 64, 524, 429, 392 and 354 at 94, which groups of cost
+// 0.45, 0.55, 0.54 and 0.60 order alike; an expert with Poisson(M / E) rows takes sum
+// over j of P(rows > 16 NRB j) groups.
 int moe_mma_nrb(int M, int E, int H, int I) {
   if (E > 4096 || M / E < (moe_rows_table(E, H, I) ? 11 : 8)) return 0;
   // 32-bit byte offsets into the transformed rows
   if ((size_t)M * std::max(H, I) * 2 > 0xFFFFFFF0u) return 0;
+  static constexpr double group_cost[] = {0.45, 0.55, 0.54, 0.60};
   const double lam = (double)M / E, dev = std::sqrt(2.0 * lam);
   int best = 8;
   double best_cost = 1e30;
@@ -1488,7 +1493,7 @@ int moe_mma_nrb(int M, int E, int H, int I) {
       p = 0.5 * std::erfc((j * br + 0.5 - lam) / dev);
       groups += p;
     }
-    const double cost = groups * (0.43 + 0.071 * nrb);
+    const double cost = groups * group_cost[nrb / 2 - 1];
     if (cost < best_cost * 0.999) {
       best_cost = cost;
       best = nrb;

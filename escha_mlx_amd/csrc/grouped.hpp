@@ -17,10 +17,14 @@
 //
 // What bounds it: the decode (about 4.6 VALU per weight) of one pass over the
 // experts' code, so the row-block size is chosen for the fewest, smallest groups
-// (moe_mma_nrb), against the split-K chain's one pass per 8 rows.  256 experts,
-// hidden 2048, intermediate 512, top-8, 2048 tokens (64 rows per expert): the
-// whole call 357 us, the split-K chain 1200.
+// (moe_mma_nrb), against the split-K chain's one pass per 8 rows; the main loop and
+// the epilogue run over the row blocks that hold rows, rounded to an even number in
+// the loop (one instance of it per size).  256 experts, hidden 2048, intermediate
+// 512, top-8, 2048 tokens (64 rows per expert): the whole call 274 us (289 over all
+// row blocks of every group), the split-K chain 1200.
 #pragma once
+
+#include <type_traits>
 
 #include "mfma.hpp"
 #include "moe.hpp"
@@ -78,8 +82,25 @@ __global__ __launch_bounds__(256, 2) void k_moe_mma(MoeMmaArgs a) {
     xoff[j] = 2u * ((uint32_t)(row < M ? row : 0) * IC) + mma2_x_chunk(tid, j);
   }
   const __amdgpu_buffer_rsrc_t xrs = buf_rsrc(a.xh, (size_t)M * IC * 2);
+  // row blocks that hold rows (a group's rows come first, then padding)
+  int nact = 1;
+#pragma unroll
+  for (int r = 1; r < NRB; ++r) nact += rows[16 * r] < M;
   f32x4_t acc[D::NA][NRB];
-  mma2_loop<NRB>(CodedCols<K>{cbase, kstride}, xrs, xoff, 0, TK / 4, s_x, acc);
+  const CodedCols<K> cols{cbase, kstride};
+  auto loop = [&](auto n) {
+    mma2_loop<NRB, decltype(n)::value>(cols, xrs, xoff, 0, TK / 4, s_x, acc);
+  };
+  if constexpr (NRB > 6) {
+    if (nact <= NRB - 6) loop(std::integral_constant<int, NRB - 6>{});
+  }
+  if constexpr (NRB > 4) {
+    if (nact > NRB - 6 && nact <= NRB - 4) loop(std::integral_constant<int, NRB - 4>{});
+  }
+  if constexpr (NRB > 2) {
+    if (nact > NRB - 4 && nact <= NRB - 2) loop(std::integral_constant<int, NRB - 2>{});
+  }
+  if (nact > NRB - 2) loop(std::integral_constant<int, NRB>{});
 
   float4* so = kOwn ? s_o : reinterpret_cast<float4*>(&s_x[0][0]);
   const float rs = a.rs;
@@ -100,6 +121,7 @@ __global__ __launch_bounds__(256, 2) void k_moe_mma(MoeMmaArgs a) {
     float4* s_b = s_a + 256;
 #pragma unroll
     for (int r = 0; r < NRB; ++r) {
+      if (r >= nact) break;
       const int row = rows[16 * r + c];
       float v[16], o[16];
       mma2_h64<K, NRB>(acc, r, v);
@@ -186,6 +208,7 @@ __global__ __launch_bounds__(256, 2) void k_moe_mma(MoeMmaArgs a) {
       ro[j] = as_global(a.rout + (size_t)e * OC)[col + 64 * (j >> 3) + (j & 7)];
 #pragma unroll
     for (int r = 0; r < NRB; ++r) {
+      if (r >= nact) break;
       const int row = rows[16 * r + c];
       mma2_out<K, NRB>(acc, r, so + (r & 1) * kMma2Xch, rs, ro, nullptr, col, row < M && live,
                        a.out, kRowsF16, (size_t)row * OC + col);

@@ -92,12 +92,13 @@ struct CodedCols {
 };
 
 // The main loop over steps [s0, s1) (s1 > s0): acc[a][r] += the wave's 64
-// columns x row block r.  xoff: byte offsets of the thread's x chunks.
-template <int NRB, typename Cols>
+// columns x row block r, of the first NACT row blocks (even; the others: zero).
+// xoff: byte offsets of the thread's x chunks.
+template <int NRB, int NACT = NRB, typename Cols>
 __device__ __forceinline__ void mma2_loop(const Cols& cols, __amdgpu_buffer_rsrc_t xrs,
                                           const uint32_t* xoff, int s0, int s1,
                                           uint4 (*s_x)[16 * NRB * 8], f32x4_t (*acc)[NRB]) {
-  constexpr int NA = 4, XCH = NRB / 2;
+  constexpr int NA = 4, XCH = NACT / 2;
   const int tid = threadIdx.x, lane = tid & 63;
   const int gk = lane >> 4, c = lane & 15;
   auto load_x = [&](uint4* xr, int s) {
@@ -137,7 +138,7 @@ __device__ __forceinline__ void mma2_loop(const Cols& cols, __amdgpu_buffer_rsrc
 #pragma unroll
     for (int P = 0; P < 2; ++P)
 #pragma unroll
-      for (int r = 0; r < NRB; ++r) {
+      for (int r = 0; r < NACT; ++r) {
         const uint4 bv = s_x[buf][(16 * r + c) * 8 + ((2 * gk + P) ^ (c & 7))];
         const u32x4_t b = __builtin_bit_cast(u32x4_t, bv);
 #pragma unroll
