@@ -259,8 +259,9 @@ def kept_ws(cache: dict, key: tuple, x: torch.Tensor, need, *args) -> torch.Tens
     else:
         cache = cache.setdefault("streams", {})
         key = (*key, _stream())
-        while len(cache) > _STREAM_WS:
-            cache.pop(next(iter(cache)), None)
+        if len(cache) > _STREAM_WS:  # a copy of the keys: other threads may add theirs
+            for old in list(cache)[:-_STREAM_WS]:
+                cache.pop(old, None)
         ws = cache.get(key)
     if ws is None:
         ws = cache[key] = torch.zeros(max(need(*args), 4), dtype=torch.uint8, device=x.device)
